@@ -104,7 +104,12 @@ __global__ void __launch_bounds__(256) k_clear_map(int *__restrict__ map, int n,
 // group's window of nfr frames claim their map slot [frame][cid][fid] with
 // atomicMin -> lowest index wins.  Geometry: n_cid x n_fid packets per frame
 // of pkt_words words each (reference: 256 x 8 x 264; 8 x 1024: 16 x 16 x 2056).
-__global__ void __launch_bounds__(256)
+// The counters are one address each for the whole grid, so their atomics run
+// one after another: one per counter and 1024-thread workgroup (78 for a group
+// of 39 B-frames) in place of one per wave (1248), which held the kernel at
+// 17.5 us per group, now 6.3.
+constexpr int MAP_WG = 1024;
+__global__ void __launch_bounds__(MAP_WG)
 k_packet_map(const uint32_t *__restrict__ pk, int n, uint32_t bzero32, int nfr, int n_cid, int n_fid,
              int pkt_words, int *__restrict__ map, int *__restrict__ cnt) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -124,12 +129,19 @@ k_packet_map(const uint32_t *__restrict__ pk, int n, uint32_t bzero32, int nfr, 
             atomicMin(map + ((rel * n_cid + (int)cid) * n_fid + (int)fid), i);
         }
     }
-    // one atomic per wave per counter
+    __shared__ int red[3][MAP_WG / 64];
     const unsigned long long bi = __ballot(inval), br = __ballot(range), ba = __ballot(acc);
     if ((threadIdx.x & 63) == 0) {
-        if (bi) atomicAdd(cnt + CNT_INVALID, __popcll(bi));
-        if (br) atomicAdd(cnt + CNT_RANGE, __popcll(br));
-        if (ba) atomicAdd(cnt + CNT_ACCEPTED, __popcll(ba));
+        red[0][threadIdx.x >> 6] = __popcll(bi);
+        red[1][threadIdx.x >> 6] = __popcll(br);
+        red[2][threadIdx.x >> 6] = __popcll(ba);
+    }
+    __syncthreads();
+    if (threadIdx.x < 3) {
+        int n = 0;
+#pragma unroll
+        for (int i = 0; i < MAP_WG / 64; ++i) n += red[threadIdx.x][i];
+        if (n) atomicAdd(cnt + threadIdx.x, n);   // CNT_INVALID, CNT_RANGE, CNT_ACCEPTED
     }
 }
 
@@ -173,17 +185,15 @@ k_reorder(const uint32_t *__restrict__ pk, const int *__restrict__ map, int8_t *
         pidx[w] = map[(frame * 256 + 2 * h + lo) * 8 + fid];
     }
     __syncthreads();
-    if (t < 2) {   // fid bitmap byte of cid = 2h + t, and the unique count
-        uint32_t byte = 0;
-        int found = 0;
-        for (int fid = 0; fid < 8; ++fid) {
-            if (pidx[2 * fid + t] != MAP_NONE) {
-                byte |= 1u << fid;
-                ++found;
-            }
+    if (t < 64) {   // fid bitmap bytes of cids 2h, 2h + 1 (slot w = 2 fid + lo), and the unique count
+        const unsigned long long b = __ballot(t < 16 && pidx[t & 15] != MAP_NONE);
+        if (t < 2) {
+            uint32_t byte = 0;
+#pragma unroll
+            for (int fid = 0; fid < 8; ++fid) byte |= (uint32_t)((b >> (2 * fid + t)) & 1) << fid;
+            bitmap[frame * 256 + 2 * h + t] = (uint8_t)byte;
         }
-        bitmap[frame * 256 + 2 * h + t] = (uint8_t)byte;
-        if (found) atomicAdd(cnt + CNT_UNIQUE, found);
+        if (t == 0 && b) atomicAdd(cnt + CNT_UNIQUE, __popcll(b));
     }
     if ((((uintptr_t)pk) & 15) == 0) {        // 16-byte payload units, a packet per wave and load
         uint4 v[4];
@@ -996,12 +1006,17 @@ k_stats(const double *__restrict__ part, int bp0, double2 *__restrict__ ms, doub
 }
 
 // Threshold policy over a chunk.  PER_BLOCK and FIXED are per block-pol and
-// run in parallel.  REFERENCE is sequential in block-pol order: the first
+// run in parallel.  REFERENCE is sequential in block-pol order: every
 // polarisation-0 block-pol seen while its slot's threshold is 0 latches its
 // sigma and mean, which then serve both polarisations
-// (vdif_inout_gpu_thread.cu:954-1005).  One thread walks the chunk for it,
-// over the statistics, policy fields and latch slots staged in LDS, so that
-// no step of the walk waits on global memory; the slots go back at the end.
+// (vdif_inout_gpu_thread.cu:954-1005).  So, in a slot that enters with
+// threshold 0, the first polarisation-0 block-pol f with sigma != 0 ends the
+// latching: block-pols from f on use its values, and an earlier one uses those
+// of the last polarisation-0 block-pol up to it (sigma 0), or the slot's own if
+// there is none.  f and the slot's last polarisation-0 block-pol are minima and
+// maxima over the chunk, so no thread walks it (one thread's walk over LDS took
+// 28 us for 256 block-pols, this THRTIME); the search back before f runs only
+// for empty leading blocks.
 constexpr int THRESH_MAX_CHUNK = SDBE_MAX_CHUNK;
 __global__ void __launch_bounds__(256) k_thresh(const double2 *__restrict__ ms, int nbpl,
                                                 const BpDesc *__restrict__ bpd, float *__restrict__ latch,
@@ -1009,37 +1024,48 @@ __global__ void __launch_bounds__(256) k_thresh(const double2 *__restrict__ ms, 
     __shared__ float2 sms[THRESH_MAX_CHUNK];      // (sigma, mean) as float
     __shared__ int sinfo[THRESH_MAX_CHUNK];       // pol | slot << 8, or -1: not REFERENCE
     __shared__ float2 slat[SDBE_LATCH_SLOTS];
-    __shared__ int any_ref;
+    __shared__ int sfirst[SDBE_LATCH_SLOTS], slast[SDBE_LATCH_SLOTS];
     const int t = threadIdx.x;
-    if (t == 0) any_ref = 0;
-    if (t < SDBE_LATCH_SLOTS) slat[t] = make_float2(latch[2 * t], latch[2 * t + 1]);
+    if (t < SDBE_LATCH_SLOTS) {
+        slat[t] = make_float2(latch[2 * t], latch[2 * t + 1]);
+        sfirst[t] = THRESH_MAX_CHUNK;
+        slast[t] = -1;
+    }
     __syncthreads();
     for (int b = t; b < nbpl; b += blockDim.x) {
         const BpDesc &d = bpd[b];
         const float2 v = make_float2((float)ms[b].y, (float)ms[b].x);
         sms[b] = v;
         if (d.policy == SDBE_THRESH_REFERENCE) {
-            sinfo[b] = (int)d.pol | ((int)d.slot << 8);
-            any_ref = 1;
+            const int slot = d.slot;
+            sinfo[b] = (int)d.pol | (slot << 8);
+            if (d.pol == 0) {
+                atomicMax(&slast[slot], b);
+                if (!(v.x == 0.0f)) atomicMin(&sfirst[slot], b);
+            }
         } else {
             sinfo[b] = -1;
             thr[b] = d.policy == SDBE_THRESH_PER_BLOCK ? v : make_float2(d.fixed_th, d.fixed_off);
         }
     }
     __syncthreads();
-    if (t != 0 || !any_ref) return;
-    for (int b = 0; b < nbpl; ++b) {
+    for (int b = t; b < nbpl; b += blockDim.x) {
         const int info = sinfo[b];
         if (info < 0) continue;
-        const int pol = info & 0xFF, slot = info >> 8;
+        const int slot = info >> 8, f = sfirst[slot];
         float2 l = slat[slot];
-        if (l.x == 0.0f && pol == 0) {
-            l = sms[b];
-            slat[slot] = l;
-            latch[2 * slot] = l.x;
-            latch[2 * slot + 1] = l.y;
+        if (l.x == 0.0f) {
+            int c = f;
+            if (b < f)
+                for (c = b; c >= 0 && sinfo[c] != slot << 8;) --c;
+            if (c >= 0) l = sms[c];
         }
         thr[b] = l;
+    }
+    if (t < SDBE_LATCH_SLOTS && slat[t].x == 0.0f && slast[t] >= 0) {
+        const float2 l = sms[sfirst[t] < THRESH_MAX_CHUNK ? sfirst[t] : slast[t]];
+        latch[2 * t] = l.x;
+        latch[2 * t + 1] = l.y;
     }
 }
 
@@ -1859,7 +1885,7 @@ sdbe_stream_state_t state_plus(const sdbe_stream_state_t &st, int64_t n_frames) 
 int unpack_map(sdbe_handle_t *h, const void *d_pkts, int32_t n_pkts, uint64_t b_zero, hipStream_t s) {
     LAUNCH(h, KID_CLEAR, 1, s, k_clear_map, dim3((h->map_n + 255) / 256), dim3(256), h->map, h->map_n, h->cnt);
     if (n_pkts > 0)
-        LAUNCH(h, KID_MAP, 1, s, k_packet_map, dim3((n_pkts + 255) / 256), dim3(256), (const uint32_t *)d_pkts,
+        LAUNCH(h, KID_MAP, 1, s, k_packet_map, dim3((n_pkts + MAP_WG - 1) / MAP_WG), dim3(MAP_WG), (const uint32_t *)d_pkts,
                n_pkts, (uint32_t)(b_zero & 0xFFFFFFFFull), h->nfr, h->n_cid, h->n_fid, h->pkt_words, h->map,
                h->cnt);
     HIP_TRY(h, hipGetLastError());
