@@ -2,10 +2,10 @@
 // corr_Xt_search / corr_Xt (software/verification/cross_corr.py:23-116).
 //
 // Kernels (32768-sample windows, 16384-point complex FFTs in LDS):
-//   k_xc_r2c    one workgroup per window: packed R2C, bins 0..16383 (numpy fft scale)
-//   k_xc_pow0   auto-power of the x0 windows, weighted for its lag-0 value
-//   k_xc_cross  per (bin block, offset): mean cross-power S_0x1 and the lag-0
-//               weighted auto-power of that offset's x1 windows
+//   k_xc_r2c    one workgroup per window of either series: packed R2C, bins
+//               0..16383 (numpy fft scale), and the window's auto-power,
+//               weighted for its lag-0 value
+//   k_xc_cross  per (bin block, tile of offsets): mean cross-power S_0x1
 //   k_xc_c2r    one workgroup per offset: packed C2R of S_0x1 (numpy irfft
 //               scale, bin 16384 zero) divided by sqrt(s_0x0[0] s_1x1[0]),
 //               with the peak |s| and the standard deviation of s
@@ -28,17 +28,44 @@ namespace {
 
 constexpr int LW = SDBE_XCORR_WINDOW;     // 32768
 constexpr int NHW = LW / 2;               // 16384
-constexpr int KB = NHW / 256;             // bin blocks of k_xc_cross / k_xc_pow0
+constexpr int KB = NHW / 256;             // bin blocks of k_xc_cross
+// Offsets per wide k_xc_cross tile.  From 64 offsets on the wide tiles give every
+// SIMD a wave (256 waves a tile, 1024 SIMDs) and what is left over goes to
+// 4-wide tiles; below that all tiles are 4 wide.  257 offsets of 256 windows, a
+// whole call: 355 us with 4-wide tiles, 287 with 8, 279 with 12, 268 with 16;
+// 63 of 128: 85 with 4, 90 with 16; 65 of 128: 92 and 83.
+constexpr int XC_OT = 16, XC_TILE_MIN = 64;
 static_assert(NHW == NCH, "the correlator reuses the 16384-point FFT");
 
+// Sum over the 1024 threads of a workgroup, in every thread (red: 16 doubles).
+__device__ __forceinline__ double block_sum_1024(double a, double *red) {
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) a += __shfl_xor(a, off);
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = a;
+    __syncthreads();
+    double s = 0.0;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) s += red[i];
+    return s;
+}
+
+// Workgroups 0 .. avg - 1 take the x0 windows, the others the x1 windows, so one
+// launch spreads both over the CUs.  pw[w] = sum over bins of (k ? 2 : 1) |X[w][k]|^2,
+// the window's share of the lag-0 autocorrelation: a mean over any windows is a
+// mean of these, so no later pass reads the spectra for it.
 __global__ void __launch_bounds__(1024)
-k_xc_r2c(const float *__restrict__ x, int w0, float2 *__restrict__ X, const float2 *__restrict__ fft_img,
-         const float2 *__restrict__ tw32k) {
+k_xc_r2c(const float *__restrict__ x0, int first0, const float *__restrict__ x1, int first1, int avg,
+         float2 *__restrict__ X0, float2 *__restrict__ X1, double *__restrict__ pw0, double *__restrict__ pw1,
+         const float2 *__restrict__ fft_img, const float2 *__restrict__ tw32k) {
     __shared__ float lds[LDS_FFT_N];
     __shared__ FftTw ftw;
+    __shared__ double red[16];
     fft_tw_load(&ftw, fft_img);
-    const int w = blockIdx.x, t = threadIdx.x;
-    const float2 *xb = reinterpret_cast<const float2 *>(x + (size_t)(w0 + w) * LW);
+    const int t = threadIdx.x;
+    const bool second = (int)blockIdx.x >= avg;
+    const int w = second ? (int)blockIdx.x - avg : (int)blockIdx.x;
+    const float2 *xb = reinterpret_cast<const float2 *>(second ? x1 + (size_t)(first1 + w) * LW
+                                                               : x0 + (size_t)(first0 + w) * LW);
     float2 v[16];
 #pragma unroll
     for (int q = 0; q < 16; ++q) v[q] = xb[t + 1024 * q];
@@ -47,7 +74,8 @@ k_xc_r2c(const float *__restrict__ x, int w0, float2 *__restrict__ X, const floa
 #pragma unroll
     for (int q = 0; q < 16; ++q) lds_put(lds, lds_re(t + 1024 * q), v[q]);
     __syncthreads();
-    float2 *out = X + (size_t)w * NHW;
+    float2 *out = (second ? X1 : X0) + (size_t)w * NHW;
+    double p = 0.0;
 #pragma unroll
     for (int q = 0; q < 16; ++q) {
         const int k = t + 1024 * q;
@@ -55,55 +83,83 @@ k_xc_r2c(const float *__restrict__ x, int w0, float2 *__restrict__ X, const floa
         const float2 zm = cconj(lds_get(lds, lds_re(km)));   // conj Z[N - k]
         const float2 E = cscale(cadd(v[q], zm), 0.5f);
         const float2 D = cscale(csub(v[q], zm), 0.5f);
-        out[k] = cadd(E, mul_si<-1>(cmul(cconj(tw32k[k]), D)));
+        const float2 X = cadd(E, mul_si<-1>(cmul(cconj(tw32k[k]), D)));
+        out[k] = X;
+        p += (k == 0 ? 1.0 : 2.0) * ((double)X.x * X.x + (double)X.y * X.y);
     }
+    const double s = block_sum_1024(p, red);
+    if (t == 0) (second ? pw1 : pw0)[w] = s;
 }
 
-__device__ __forceinline__ double block_sum_256(double a, double *red) {
+// Offsets o0 .. o0 + OT - 1 of bin k: S[o][k] = mean_w X0[w][k] conj(X1[o + w][k]),
+// FP64 sums.  One thread keeps OT sums and the OT windows of x1 that the current
+// w meets, in a ring that takes one new window per step (unrolled, so its
+// indices are constants): one load of each series and two conversions per OT
+// offsets, where a thread per (bin, offset) loaded and converted both for every
+// offset.  That is 4 OT FP64 FMAs per step, which bound it: 110 us for 257
+// offsets of 256 windows at one wave instruction per CU and cycle, measured 170
+// (before: 1050, the loads and conversions).
+// Bin blocks are the fastest grid dimension, 64 of them, so the tiles of a bin
+// block run on one XCD and read the same windows through its L2 at about the
+// same time.
+template <int OT>
+__device__ __forceinline__ void cross_tile(const float2 *__restrict__ X0, const float2 *__restrict__ X1, int avg,
+                                           int n_off, int o0, int k, float2 *__restrict__ S) {
+    const int last = n_off + avg - 2;          // last x1 window; a tile past n_off loads it again
+    double sr[OT], si[OT], bx[OT], by[OT];
 #pragma unroll
-    for (int off = 32; off > 0; off >>= 1) a += __shfl_xor(a, off);
-    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = a;
-    __syncthreads();
-    return red[0] + red[1] + red[2] + red[3];
+    for (int j = 0; j < OT; ++j) {
+        const float2 b = X1[(size_t)min(o0 + j, last) * NHW + k];
+        sr[j] = si[j] = 0.0;
+        bx[j] = b.x;       // slot OT - 1 is replaced by the first step
+        by[j] = b.y;
+    }
+    // step i of a block of OT: window o0 + w + j of x1 is in slot (i + j) % OT
+    auto step = [&](int i, float2 a, float2 b) {
+        const double ax = a.x, ay = a.y;
+        bx[(i + OT - 1) % OT] = b.x;
+        by[(i + OT - 1) % OT] = b.y;
+#pragma unroll
+        for (int j = 0; j < OT; ++j) {
+            const double cx = bx[(i + j) % OT], cy = by[(i + j) % OT];
+            sr[j] = fma(ax, cx, fma(ay, cy, sr[j]));     // a conj(b)
+            si[j] = fma(ay, cx, fma(-ax, cy, si[j]));
+        }
+    };
+    int w = 0;
+    for (; w + OT <= avg; w += OT) {
+        float2 a[OT], b[OT];
+#pragma unroll
+        for (int i = 0; i < OT; ++i) {
+            a[i] = X0[(size_t)(w + i) * NHW + k];
+            b[i] = X1[(size_t)min(o0 + w + i + OT - 1, last) * NHW + k];
+        }
+#pragma unroll
+        for (int i = 0; i < OT; ++i) step(i, a[i], b[i]);
+    }
+#pragma unroll
+    for (int i = 0; i < OT; ++i)
+        if (w + i < avg)
+            step(i, X0[(size_t)(w + i) * NHW + k], X1[(size_t)min(o0 + w + i + OT - 1, last) * NHW + k]);
+#pragma unroll
+    for (int j = 0; j < OT; ++j)
+        if (o0 + j < n_off) S[(size_t)(o0 + j) * NHW + k] = make_float2((float)(sr[j] / avg), (float)(si[j] / avg));
 }
 
-// part0[kb] = sum over the block's bins of (k ? 2 : 1) mean_w |X0[w][k]|^2
+// n_wide tiles of OT offsets, then tiles of 4 for the rest
+template <int OT>
 __global__ void __launch_bounds__(256)
-k_xc_pow0(const float2 *__restrict__ X0, int avg, double *__restrict__ part0) {
-    __shared__ double red[4];
-    const int k = blockIdx.x * 256 + threadIdx.x;
-    double p = 0.0;
-    for (int w = 0; w < avg; ++w) {
-        const float2 a = X0[(size_t)w * NHW + k];
-        p += (double)a.x * a.x + (double)a.y * a.y;
-    }
-    p *= (k == 0 ? 1.0 : 2.0) / avg;
-    const double s = block_sum_256(p, red);
-    if (threadIdx.x == 0) part0[blockIdx.x] = s;
-}
-
-// offset o: S[o][k] = mean_w X0[w][k] conj(X1[o + w][k]); part1[o][kb] as part0
-// for the windows X1[o .. o + avg)
-__global__ void __launch_bounds__(256)
-k_xc_cross(const float2 *__restrict__ X0, const float2 *__restrict__ X1, int avg, float2 *__restrict__ S,
-           double *__restrict__ part1) {
-    __shared__ double red[4];
-    const int k = blockIdx.x * 256 + threadIdx.x, o = blockIdx.y;
-    double sr = 0.0, si = 0.0, p = 0.0;
-    for (int w = 0; w < avg; ++w) {
-        const float2 a = X0[(size_t)w * NHW + k], b = X1[(size_t)(o + w) * NHW + k];
-        sr += (double)a.x * b.x + (double)a.y * b.y;     // a conj(b)
-        si += (double)a.y * b.x - (double)a.x * b.y;
-        p += (double)b.x * b.x + (double)b.y * b.y;
-    }
-    S[(size_t)o * NHW + k] = make_float2((float)(sr / avg), (float)(si / avg));
-    p *= (k == 0 ? 1.0 : 2.0) / avg;
-    const double s = block_sum_256(p, red);
-    if (threadIdx.x == 0) part1[(size_t)o * KB + blockIdx.x] = s;
+k_xc_cross(const float2 *__restrict__ X0, const float2 *__restrict__ X1, int avg, int n_off, int n_wide,
+           float2 *__restrict__ S) {
+    const int k = blockIdx.x * 256 + threadIdx.x, y = blockIdx.y;
+    if (y < n_wide)
+        cross_tile<OT>(X0, X1, avg, n_off, y * OT, k, S);
+    else
+        cross_tile<4>(X0, X1, avg, n_off, n_wide * OT + 4 * (y - n_wide), k, S);
 }
 
 __global__ void __launch_bounds__(1024)
-k_xc_c2r(const float2 *__restrict__ S, const double *__restrict__ part0, const double *__restrict__ part1,
+k_xc_c2r(const float2 *__restrict__ S, const double *__restrict__ pw0, const double *__restrict__ pw1, int avg,
          float *__restrict__ s_out, float *__restrict__ peak, float *__restrict__ sdev,
          const float2 *__restrict__ fft_img, const float2 *__restrict__ tw32k) {
     __shared__ float lds[LDS_FFT_N];
@@ -111,11 +167,15 @@ k_xc_c2r(const float2 *__restrict__ S, const double *__restrict__ part0, const d
     __shared__ double red[3][16];
     fft_tw_load(&ftw, fft_img);
     const int o = blockIdx.x, t = threadIdx.x;
+    // mean lag-0 powers of the offset's windows
     double n0 = 0.0, n1 = 0.0;
-    for (int i = 0; i < KB; ++i) {
-        n0 += part0[i];
-        n1 += part1[(size_t)o * KB + i];
+    for (int i = t; i < avg; i += 1024) {
+        n0 += pw0[i];
+        n1 += pw1[o + i];
     }
+    n0 = block_sum_1024(n0, red[0]) / avg;
+    n1 = block_sum_1024(n1, red[1]) / avg;
+    __syncthreads();    // red is used again below
     // irfft scale 1 / 32768 and the normalisation by the lag-0 autocorrelations
     const float sc = (float)(1.0 / ((double)LW * sqrt((n0 / LW) * (n1 / LW))));
     const float2 *Xo = S + (size_t)o * NHW;
@@ -179,8 +239,8 @@ struct sdbe_xcorr {
     float2 *X0 = nullptr;         // [max_win][16384]
     float2 *X1 = nullptr;         // [max_win][16384]
     float2 *S = nullptr;          // [max_off][16384]
-    double *part0 = nullptr;      // [KB]
-    double *part1 = nullptr;      // [max_off][KB]
+    double *pw0 = nullptr;        // [max_win] lag-0 power of each window
+    double *pw1 = nullptr;        // [max_win]
 };
 
 namespace {
@@ -206,8 +266,8 @@ void sdbe_xcorr_destroy(sdbe_xcorr_t *x) {
     (void)hipFree(x->X0);
     (void)hipFree(x->X1);
     (void)hipFree(x->S);
-    (void)hipFree(x->part0);
-    (void)hipFree(x->part1);
+    (void)hipFree(x->pw0);
+    (void)hipFree(x->pw1);
     delete x;
 }
 
@@ -245,8 +305,8 @@ int sdbe_xcorr_create(int device, int32_t max_windows, int32_t max_offsets, sdbe
     XALLOC(x->X0, (size_t)max_windows * NHW * sizeof(float2));
     XALLOC(x->X1, (size_t)max_windows * NHW * sizeof(float2));
     XALLOC(x->S, (size_t)max_offsets * NHW * sizeof(float2));
-    XALLOC(x->part0, KB * sizeof(double));
-    XALLOC(x->part1, (size_t)max_offsets * KB * sizeof(double));
+    XALLOC(x->pw0, (size_t)max_windows * sizeof(double));
+    XALLOC(x->pw1, (size_t)max_windows * sizeof(double));
 #undef XALLOC
     if (hipMemcpy(x->fft_img, img.data(), FFT_TW_N * sizeof(float2), hipMemcpyHostToDevice) != hipSuccess ||
         hipMemcpy(x->tw32k, tw.data(), NHW * sizeof(float2), hipMemcpyHostToDevice) != hipSuccess) {
@@ -273,15 +333,14 @@ int sdbe_xcorr_search(sdbe_xcorr_t *x, const float *d_x0, int32_t n0_windows, co
     XC_TRY(x, hipSetDevice(x->device));
     hipStream_t s = (hipStream_t)stream;
     // spectra of the windows the search uses: x0[c, c + avg), x1[lo, lo + n_offsets + avg - 1)
-    hipLaunchKernelGGL(k_xc_r2c, dim3(avg), dim3(1024), 0, s, d_x0, (int)c, x->X0, (const float2 *)x->fft_img,
-                       (const float2 *)x->tw32k);
-    hipLaunchKernelGGL(k_xc_r2c, dim3(n_offsets + avg - 1), dim3(1024), 0, s, d_x1, (int)lo, x->X1,
-                       (const float2 *)x->fft_img, (const float2 *)x->tw32k);
-    hipLaunchKernelGGL(k_xc_pow0, dim3(KB), dim3(256), 0, s, (const float2 *)x->X0, (int)avg, x->part0);
-    hipLaunchKernelGGL(k_xc_cross, dim3(KB, n_offsets), dim3(256), 0, s, (const float2 *)x->X0,
-                       (const float2 *)x->X1, (int)avg, x->S, x->part1);
+    hipLaunchKernelGGL(k_xc_r2c, dim3(avg + n_offsets + avg - 1), dim3(1024), 0, s, d_x0, (int)c, d_x1, (int)lo,
+                       (int)avg, x->X0, x->X1, x->pw0, x->pw1, (const float2 *)x->fft_img, (const float2 *)x->tw32k);
+    const int n_wide = n_offsets >= XC_TILE_MIN ? n_offsets / XC_OT : 0;
+    const int n_tiles = n_wide + (n_offsets - n_wide * XC_OT + 3) / 4;
+    hipLaunchKernelGGL(k_xc_cross<XC_OT>, dim3(KB, n_tiles), dim3(256), 0, s, (const float2 *)x->X0,
+                       (const float2 *)x->X1, (int)avg, (int)n_offsets, n_wide, x->S);
     hipLaunchKernelGGL(k_xc_c2r, dim3(n_offsets), dim3(1024), 0, s, (const float2 *)x->S,
-                       (const double *)x->part0, (const double *)x->part1, d_s, d_peak, d_std,
+                       (const double *)x->pw0, (const double *)x->pw1, (int)avg, d_s, d_peak, d_std,
                        (const float2 *)x->fft_img, (const float2 *)x->tw32k);
     XC_TRY(x, hipGetLastError());
     return SDBE_OK;
