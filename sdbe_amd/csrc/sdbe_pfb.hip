@@ -14,6 +14,13 @@
 //   k_pfb_fold_r2c  one workgroup per spectrum: 4-tap fold, packed R2C
 //                   (16384-point complex FFT in LDS + split post-processing)
 //   k_pfb_c2r       one workgroup per spectrum: packed C2R to the pseudo-timestream
+// The solve, for any prototype without zeros together on the unit circle:
+//   k_pfb_spectral  once per plan, one thread per branch: the constant
+//                   minimum-phase factor of P P^T and the tables built on it
+//   k_pfb_span, k_pfb_join, k_pfb_solve
+//                   two recursive filters, block-parallel over the rows
+//   k_pfb_corner    calls of up to 256 rows: their tables, then k_pfb_solve alone
+// and for the others the factor-row kernels:
 //   k_pfb_factor    once per plan, one thread per branch: banded Cholesky of
 //                   P P^T (bandwidth 3, Toeplitz per branch), FP64; the factor's
 //                   state is checkpointed every 16 rows
@@ -536,6 +543,552 @@ k_pfb_bfin(const float *__restrict__ yh, const double *__restrict__ uck, int nbl
     }
 }
 
+// --------------------------------------------- constant-coefficient solve
+// P P^T is Toeplitz per branch, so it has a constant minimum-phase factor b:
+// b(q) = b0 + b1 q + b2 q^2 + b3 q^3 with the taps' autocorrelation and no zero
+// inside the unit circle (the taps' polynomial with its zeros inside reflected),
+// and with B the lower-triangular Toeplitz matrix of b
+//   P P^T = B B^T + E H H^T E^T,   H[i][m] = b_{i+m+1}  (E: the first three rows).
+// B B^T is two recursive filters with three constant coefficients beta = b_k / b0
+// (no factor rows to recompute or checkpoint), and the corner is a rank-3
+// correction: with z0 the filters' solution, g = W z0[0..2] is taken off the
+// first three right-hand sides, W = H (I + H^T G H)^-1 H^T, G the first 3 x 3
+// block of (B B^T)^-1.  In scaled units v = b0 B^-1 y, zeta = b0^2 z:
+//   v_i = y_i - beta1 v_{i-1} - beta2 v_{i-2} - beta3 v_{i-3},
+//   zeta_i = v_i - beta1 zeta_{i+1} - beta2 zeta_{i+2} - beta3 zeta_{i+3}.
+// Rounding grows with the rows like the factor-row recurrences' does (both below
+// 1e-8 of the result for 4096 rows of the Hamming and Hann-sinc prototypes, far
+// under the FP32 rounding of yh), except where two zeros fall together on the
+// unit circle: taps 1, 2, 1 lose 5e-5 in 1000 rows here and 1e-8 by factor rows.
+// k_pfb_spectral counts such branches, and a plan that has any takes those.
+//
+// Thread (branch, span of 32 rows) keeps its rows' v in registers; a workgroup
+// holds 64 branches x 8 spans and scans the spans' boundary states through LDS.
+// Up to 256 rows that is the whole problem.  Above, k_pfb_span takes every
+// 256-row block's outgoing states in both directions (from zero incoming ones) in
+// one read of yh, k_pfb_join composes them per branch into the blocks' true
+// incoming states with the corner, and k_pfb_solve finishes the blocks: two
+// reads of yh and one write of x, all in 256-byte runs.  4096 spectra: span 130 us
+// (4.1 TB/s), join 22, solve 225 (4.8 TB/s, the rate of a large copy); the
+// factor-row kernels, which read yh four times beside 0.8 GB of checkpoints and
+// recompute every factor row four times, take 890.  (Tiles of 8 branches over
+// all 4096 rows read yh once, but in 32-byte runs: 700 us.)
+constexpr int SR = 32, SWV = 8, SBLK = SR * SWV;     // rows per thread, waves and rows per workgroup
+// table rows, [row][LB] doubles
+constexpr int TB_BETA = 0;                // beta1..3
+constexpr int TB_WZ = 3;                  // taps / b0^2
+constexpr int TB_CS = 7;                  // C^32: the state after a span of no input
+constexpr int TB_CB = 16;                 // C^256
+constexpr int TB_RS = 25;                 // a span's head zeta per unit incoming state
+constexpr int TB_HS = 34;                 // its impulse response h27..h31
+constexpr int TB_RB = 39;                 // the same of a block: head zeta
+constexpr int TB_HB = 48;                 // ... h251..h255
+constexpr int TB_N = 53;
+// ... and of a call
+constexpr int TC_W = 0;                   // corner matrix W (scaled)
+constexpr int TC_RS = 9;                  // TB_RS of the partial last span
+constexpr int TC_G = 18;                  // more than one block: g
+constexpr int TC_N = 21;
+
+// 3 x 3 matrices, m[3 r + c]
+__device__ __forceinline__ void mat_mul(double (&o)[9], const double (&a)[9], const double (&b)[9]) {
+#pragma unroll
+    for (int r = 0; r < 3; ++r)
+#pragma unroll
+        for (int c = 0; c < 3; ++c) o[3 * r + c] = a[3 * r] * b[c] + a[3 * r + 1] * b[3 + c] + a[3 * r + 2] * b[6 + c];
+}
+
+// sum_{k < n} C^k X (C^k)^T (TR) or sum_{k < n} C^k X C^k, by doubling over the
+// bits of n.
+template <bool TR>
+__device__ __forceinline__ void power_sum(int n, const double (&C)[9], const double (&X)[9], double (&S)[9]) {
+    double P[9], t[9], u[9];
+    auto add = [&](const double (&m)[9], const double (&x)[9]) {   // S = x + m S m(^T)
+        mat_mul(t, m, S);
+        if (TR) {
+#pragma unroll
+            for (int r = 0; r < 3; ++r)
+#pragma unroll
+                for (int c = 0; c < 3; ++c)
+                    u[3 * r + c] = t[3 * r] * m[3 * c] + t[3 * r + 1] * m[3 * c + 1] + t[3 * r + 2] * m[3 * c + 2];
+        } else {
+            mat_mul(u, t, m);
+        }
+#pragma unroll
+        for (int i = 0; i < 9; ++i) S[i] = x[i] + u[i];
+    };
+#pragma unroll
+    for (int i = 0; i < 9; ++i) {
+        P[i] = C[i];
+        S[i] = n > 0 ? X[i] : 0.0;
+    }
+    for (int bit = n > 0 ? 30 - __builtin_clz(n) : -1; bit >= 0; --bit) {     // below n's leading bit
+        add(P, S);
+        mat_mul(t, P, P);
+#pragma unroll
+        for (int i = 0; i < 9; ++i) P[i] = t[i];
+        if ((n >> bit) & 1) {
+            add(C, X);
+            mat_mul(t, C, P);
+#pragma unroll
+            for (int i = 0; i < 9; ++i) P[i] = t[i];
+        }
+    }
+}
+
+// Head zeta (rows 0..2, nothing incoming from below) of n rows whose v is the
+// response to the incoming state e_c, in column c: v_k = (C^(k+1))[0][c], and
+// zeta_r = sum_k v_k h_{k-r} with (h_k, h_{k-1}, h_{k-2}) = C^k e_0.
+__device__ __forceinline__ void head_response(int n, double be1, double be2, double be3, double (&rm)[9]) {
+    const double C[9] = {-be1, -be2, -be3, 1.0, 0.0, 0.0, 0.0, 1.0, 0.0};
+    const double X[9] = {-be1, -be2, -be3, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
+    power_sum<false>(n, C, X, rm);
+}
+
+// Per plan, one thread per branch: the minimum-phase factor and the tables.
+// The cubic's real zero by Cardano's formula and Newton steps, deflated from the
+// end that keeps the remaining coefficients accurate, then the quadratic.
+// *clustered counts the branches with two zeros together on the unit circle.
+__global__ void __launch_bounds__(SOLVE_WG)
+k_pfb_spectral(const float *__restrict__ win, double *__restrict__ tab, int *__restrict__ clustered) {
+    const int n = blockIdx.x * SOLVE_WG + threadIdx.x;
+    const double w[4] = {win[n], win[LB + n], win[2 * LB + n], win[3 * LB + n]};
+    const double sc = fmax(fmax(fabs(w[0]), fabs(w[1])), fmax(fabs(w[2]), fabs(w[3])));
+    // c0 x^3 + c1 x^2 + c2 x + c3, |c0| >= |c3| (either order has the autocorrelation),
+    // zeros wanted in |x| <= 1
+    const bool rev = fabs(w[3]) > fabs(w[0]);
+    double c[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) c[i] = (rev ? w[3 - i] : w[i]) / sc;
+    double b[4];
+    bool close = false;
+    if (fabs(c[0]) <= 1e-15) {      // both ends vanish: two taps
+        const bool f = fabs(c[1]) >= fabs(c[2]);
+        b[0] = f ? c[1] : c[2];
+        b[1] = f ? c[2] : c[1];
+        b[2] = b[3] = 0.0;
+    } else {
+        const double A = c[1] / c[0], B = c[2] / c[0], C = c[3] / c[0];
+        const double Q = (A * A - 3.0 * B) / 9.0, R = (2.0 * A * A * A - 9.0 * A * B + 27.0 * C) / 54.0;
+        double r;
+        if (R * R < Q * Q * Q) {    // three real zeros: the largest
+            const double th = acos(fmax(-1.0, fmin(1.0, R / sqrt(Q * Q * Q))));
+            const double m = -2.0 * sqrt(Q), tau = 6.283185307179586476925286766559;
+            r = m * cos(th / 3.0) - A / 3.0;
+            for (int k = 1; k < 3; ++k) {
+                const double x = m * cos((th + k * tau) / 3.0) - A / 3.0;
+                if (fabs(x) > fabs(r)) r = x;
+            }
+        } else {
+            const double s = -copysign(cbrt(fabs(R) + sqrt(fmax(R * R - Q * Q * Q, 0.0))), R);
+            r = s + (s != 0.0 ? Q / s : 0.0) - A / 3.0;
+        }
+        for (int k = 0; k < 4; ++k) {
+            const double f = ((r + A) * r + B) * r + C, d = (3.0 * r + 2.0 * A) * r + B;
+            if (d == 0.0) break;
+            const double x = r - f / d;
+            if (!(fabs(((x + A) * x + B) * x + C) < fabs(f))) break;
+            r = x;
+        }
+        // x^2 + d1 x + d0: coefficients above the largest of the terms |C|, |B r|,
+        // |A r^2|, |r^3| from the top, those below it from the bottom
+        double d1 = A + r, d0 = B + d1 * r;
+        if (r != 0.0) {
+            const double t0 = fabs(C), t1 = fabs(B * r), t2 = fabs(A * r * r), t3 = fabs(r * r * r);
+            if (fmax(t2, t3) > fmax(t0, t1) || t1 > t0) d0 = -C / r;
+            if (fmax(t2, t3) > fmax(t0, t1)) d1 = (d0 - B) / r;
+        }
+        double pol[4] = {c[0], 0.0, 0.0, 0.0};
+        auto times = [&](double x) {        // times (x' - x), or reflected: (1 - x x')
+            const double u = fabs(x) > 1.0 ? -x : 1.0, v = fabs(x) > 1.0 ? 1.0 : -x;
+#pragma unroll
+            for (int i = 3; i >= 1; --i) pol[i] = pol[i] * u + pol[i - 1] * v;
+            pol[0] *= u;
+        };
+        auto inside = [](double x) { return fabs(x) > 1.0 ? 1.0 / x : x; };
+        times(r);
+        const double disc = d1 * d1 - 4.0 * d0, ri = inside(r);
+        constexpr double NEAR = 0.998, GAP = 0.02;
+        if (disc >= 0.0) {
+            const double s = -0.5 * (d1 + copysign(sqrt(disc), d1)), x2 = s != 0.0 ? d0 / s : 0.0;
+            times(s);
+            times(x2);
+            const double si = inside(s), xi = inside(x2);
+            close = (fmin(fabs(ri), fabs(si)) > NEAR && fabs(ri - si) < GAP) ||
+                    (fmin(fabs(ri), fabs(xi)) > NEAR && fabs(ri - xi) < GAP) ||
+                    (fmin(fabs(si), fabs(xi)) > NEAR && fabs(si - xi) < GAP);
+        } else {
+            const bool out = d0 > 1.0;
+            const double e0 = out ? d0 : 1.0, e2 = out ? 1.0 : d0;
+            const double p0 = pol[0], p1 = pol[1];
+            pol[0] = p0 * e0;
+            pol[1] = p0 * d1 + p1 * e0;
+            pol[2] = p0 * e2 + p1 * d1;
+            pol[3] = p1 * e2;
+            const double re = -0.5 * d1 / e0, im = 0.5 * sqrt(-disc) / e0, mod = sqrt(fmin(d0, 1.0 / d0));
+            close = mod > NEAR && (2.0 * im < GAP || (fabs(ri) > NEAR && hypot(ri - re, im) < GAP));
+        }
+#pragma unroll
+        for (int i = 0; i < 4; ++i) b[i] = pol[i];
+    }
+    if (close) atomicAdd(clustered, 1);
+    const double be1 = b[1] / b[0], be2 = b[2] / b[0], be3 = b[3] / b[0], b0 = b[0] * sc;
+    double *o = tab + n;
+    o[(size_t)(TB_BETA + 0) * LB] = be1;
+    o[(size_t)(TB_BETA + 1) * LB] = be2;
+    o[(size_t)(TB_BETA + 2) * LB] = be3;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) o[(size_t)(TB_WZ + i) * LB] = w[i] / b0 / b0;
+    double m[9] = {-be1, -be2, -be3, 1.0, 0.0, 0.0, 0.0, 1.0, 0.0};
+    for (int k = 1; k <= 8; ++k) {          // C^2, C^4, .. C^256
+        double q[9];
+        mat_mul(q, m, m);
+#pragma unroll
+        for (int i = 0; i < 9; ++i) m[i] = q[i];
+        if (k == 5 || k == 8)
+#pragma unroll
+            for (int i = 0; i < 9; ++i) o[(size_t)((k == 5 ? TB_CS : TB_CB) + i) * LB] = m[i];
+    }
+    for (int v = 0; v < 2; ++v) {
+        const int rows = v ? SBLK : SR;
+        double rm[9];
+        head_response(rows, be1, be2, be3, rm);
+#pragma unroll
+        for (int i = 0; i < 9; ++i) o[(size_t)((v ? TB_RB : TB_RS) + i) * LB] = rm[i];
+        double h1 = 0.0, h2 = 0.0, h3 = 0.0;
+        for (int k = 0; k < rows; ++k) {
+            const double h = (k == 0 ? 1.0 : 0.0) - be1 * h1 - be2 * h2 - be3 * h3;
+            if (k >= rows - 5) o[(size_t)((v ? TB_HB : TB_HS) + k - (rows - 5)) * LB] = h;
+            h3 = h2;
+            h2 = h1;
+            h1 = h;
+        }
+    }
+}
+
+// The corner matrix W of N rows.  G = sum_{i < N} s_i s_i^T with s_i = C^i e_0.
+__device__ __forceinline__ void corner(int N, double be1, double be2, double be3, double (&W)[9]) {
+    const double C[9] = {-be1, -be2, -be3, 1.0, 0.0, 0.0, 0.0, 1.0, 0.0};
+    const double X[9] = {1.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
+    double G[9], t[9];
+    power_sum<true>(N, C, X, G);
+    // H (scaled by 1 / b0), rows past N zero
+    const double H[9] = {be1, be2, be3, N > 1 ? be2 : 0.0, N > 1 ? be3 : 0.0, 0.0, N > 2 ? be3 : 0.0, 0.0, 0.0};
+    double S[9], K[9];
+    mat_mul(t, G, H);
+#pragma unroll
+    for (int r = 0; r < 3; ++r)
+#pragma unroll
+        for (int c = 0; c < 3; ++c)
+            S[3 * r + c] = (r == c ? 1.0 : 0.0) + H[r] * t[c] + H[3 + r] * t[3 + c] + H[6 + r] * t[6 + c];
+    // S = L L^T (symmetric, eigenvalues >= 1); K = L^-1 H^T, W = K^T K
+    const double l00 = 1.0 / sqrt(S[0]), l10 = S[3] * l00, l20 = S[6] * l00;
+    const double l11 = 1.0 / sqrt(S[4] - l10 * l10), l21 = (S[7] - l20 * l10) * l11;
+    const double l22 = 1.0 / sqrt(S[8] - l20 * l20 - l21 * l21);
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {      // column c of H^T is row c of H
+        K[c] = H[3 * c] * l00;
+        K[3 + c] = (H[3 * c + 1] - l10 * K[c]) * l11;
+        K[6 + c] = (H[3 * c + 2] - l20 * K[c] - l21 * K[3 + c]) * l22;
+    }
+#pragma unroll
+    for (int r = 0; r < 3; ++r)
+#pragma unroll
+        for (int c = 0; c < 3; ++c) W[3 * r + c] = K[r] * K[c] + K[3 + r] * K[3 + c] + K[6 + r] * K[6 + c];
+}
+
+// Per call of at most one block, one thread per branch: its tables.
+__global__ void __launch_bounds__(SOLVE_WG)
+k_pfb_corner(const double *__restrict__ tab, int N, double *__restrict__ tc) {
+    const int n = blockIdx.x * SOLVE_WG + threadIdx.x;
+    const double be1 = tab[n], be2 = tab[LB + n], be3 = tab[2 * LB + n];
+    double W[9], rm[9];
+    corner(N, be1, be2, be3, W);
+    head_response(N & (SR - 1), be1, be2, be3, rm);
+#pragma unroll
+    for (int i = 0; i < 9; ++i) {
+        tc[(size_t)(TC_W + i) * LB + n] = W[i];
+        tc[(size_t)(TC_RS + i) * LB + n] = rm[i];
+    }
+}
+
+struct V3 {
+    double a, b, c;
+};
+__device__ __forceinline__ V3 v3_load(const double *__restrict__ p, int n) {
+    return V3{p[n], p[LB + n], p[2 * LB + n]};
+}
+__device__ __forceinline__ void v3_store(double *__restrict__ p, int n, V3 v) {
+    p[n] = v.a;
+    p[LB + n] = v.b;
+    p[2 * LB + n] = v.c;
+}
+// x + M y, M's element i at m[i * ST]
+template <int ST>
+__device__ __forceinline__ V3 mv_add(V3 x, const double *m, V3 y) {
+    return V3{fma(m[0], y.a, fma(m[ST], y.b, fma(m[2 * ST], y.c, x.a))),
+              fma(m[3 * ST], y.a, fma(m[4 * ST], y.b, fma(m[5 * ST], y.c, x.b))),
+              fma(m[6 * ST], y.a, fma(m[7 * ST], y.b, fma(m[8 * ST], y.c, x.c)))};
+}
+
+// The filter's next value from its last three.
+#define PFB_FILTER(in, s) fma(-be1, (s).a, fma(-be2, (s).b, fma(-be3, (s).c, (in))))
+
+// Outgoing states of block blockIdx.y from zero incoming ones: P = its last three
+// v, Q = its first three zeta.  Q is a sum over the rows, sum_k v_k h_{k-r}, so
+// the rows are read once, in order, and none is kept.
+__global__ void __launch_bounds__(SOLVE_WG)
+k_pfb_span(const float *__restrict__ yh, int N, const double *__restrict__ tab, double *__restrict__ P,
+           double *__restrict__ Q) {
+    const int n = blockIdx.x * SOLVE_WG + threadIdx.x, blk = blockIdx.y, r0 = blk * SBLK, r1 = min(r0 + SBLK, N);
+    const double be1 = tab[n], be2 = tab[LB + n], be3 = tab[2 * LB + n];
+    V3 st{0.0, 0.0, 0.0}, q = st, h{0.0, 0.0, 0.0};
+    double in = 1.0;                       // h's input: an impulse at the block's first row
+    constexpr int CH = 32;
+    for (int c0 = r0; c0 < r1; c0 += CH) {
+        float y[CH];
+#pragma unroll
+        for (int k = 0; k < CH; ++k) y[k] = yh[(size_t)min(c0 + k, N - 1) * LB + n];
+        const bool full = c0 + CH <= r1;
+#pragma unroll
+        for (int k = 0; k < CH; ++k) {
+            if (full || c0 + k < r1) {
+                const double v = PFB_FILTER((double)y[k], st), hk = PFB_FILTER(in, h);
+                in = 0.0;
+                q = V3{fma(v, hk, q.a), fma(v, h.a, q.b), fma(v, h.b, q.c)};
+                st = V3{v, st.a, st.b};
+                h = V3{hk, h.a, h.b};
+            }
+        }
+    }
+    v3_store(P + (size_t)3 * blk * LB, n, st);
+    v3_store(Q + (size_t)3 * blk * LB, n, q);
+}
+
+// Per branch: the blocks' true incoming states A (from above) and B (from below),
+// the corner's g, and the partial last span's head response.  The walks over the
+// blocks are short dependent chains on few waves (512), so up to JOIN_LDS blocks
+// the states wait in LDS, all loaded at the start (IN_LDS); longer calls keep
+// them in A and Q, which is overwritten.
+constexpr int JOIN_LDS = 16;
+template <bool IN_LDS>
+__global__ void __launch_bounds__(SOLVE_WG)
+k_pfb_join(const double *__restrict__ tab, int N, int nb, const double *__restrict__ P, double *Q, double *A,
+           double *__restrict__ B, double *__restrict__ tc) {
+    __shared__ V3 sh[IN_LDS ? 2 * JOIN_LDS * SOLVE_WG : 1];
+    const int t = threadIdx.x, n = blockIdx.x * SOLVE_WG + t;
+    constexpr size_t B3 = (size_t)3 * LB;
+    // slot 0: P, then A; slot 1: Q
+    auto get = [&](int slot, int k) {
+        return IN_LDS ? sh[(2 * k + slot) * SOLVE_WG + t] : v3_load((slot ? Q : A) + B3 * k, n);
+    };
+    auto put = [&](int slot, int k, V3 v) {
+        if (IN_LDS)
+            sh[(2 * k + slot) * SOLVE_WG + t] = v;
+        else
+            v3_store((slot ? Q : A) + B3 * k, n, v);
+    };
+    if (IN_LDS) {
+        constexpr int U = 8;
+        for (int k0 = 0; k0 < nb; k0 += U) {
+            V3 p[U], q[U];
+#pragma unroll
+            for (int i = 0; i < U; ++i) {
+                p[i] = v3_load(P + B3 * min(k0 + i, nb - 1), n);
+                q[i] = v3_load(Q + B3 * min(k0 + i, nb - 1), n);
+            }
+#pragma unroll
+            for (int i = 0; i < U; ++i)
+                if (k0 + i < nb) {
+                    put(0, k0 + i, p[i]);
+                    put(1, k0 + i, q[i]);
+                }
+        }
+    }
+    const double be1 = tab[n], be2 = tab[LB + n], be3 = tab[2 * LB + n];
+    double cb[9], rb[9], rl[9], W[9];
+#pragma unroll
+    for (int i = 0; i < 9; ++i) {
+        cb[i] = tab[(size_t)(TB_CB + i) * LB + n];
+        rb[i] = tab[(size_t)(TB_RB + i) * LB + n];
+    }
+    head_response(N & (SR - 1), be1, be2, be3, rl);
+#pragma unroll
+    for (int i = 0; i < 9; ++i) tc[(size_t)(TC_RS + i) * LB + n] = rl[i];
+    head_response((N - 1) % SBLK + 1, be1, be2, be3, rl);     // the last block's
+    corner(N, be1, be2, be3, W);
+    const V3 zero{0.0, 0.0, 0.0};
+    V3 a = zero;
+    for (int k = 0; k < nb; ++k) {
+        const V3 p = IN_LDS ? get(0, k) : v3_load(P + B3 * k, n), q = get(1, k);
+        put(0, k, a);
+        put(1, k, k == nb - 1 ? mv_add<1>(q, rl, a) : mv_add<1>(q, rb, a));
+        a = mv_add<1>(p, cb, a);
+    }
+    V3 z = zero;                                               // zeta at the head of block k
+    for (int k = nb - 1; k >= 0; --k) z = mv_add<1>(get(1, k), cb, z);
+    const V3 g = mv_add<1>(zero, W, z);
+    v3_store(tc + (size_t)TC_G * LB, n, g);
+    const double *h = tab + (size_t)TB_HB * LB + n;
+    const double h0 = h[0], h1 = h[LB], h2 = h[2 * LB], h3 = h[3 * LB], h4 = h[4 * LB];
+    // state after the first block from -g on its first three rows
+    V3 d{-(g.a * h4 + g.b * h3 + g.c * h2), -(g.a * h3 + g.b * h2 + g.c * h1), -(g.a * h2 + g.b * h1 + g.c * h0)};
+    v3_store(A, n, zero);
+    for (int k = 1; k < nb; ++k) {
+        const V3 p = get(0, k), q = get(1, k);
+        v3_store(A + B3 * k, n, V3{p.a + d.a, p.b + d.b, p.c + d.c});
+        put(1, k, k == nb - 1 ? mv_add<1>(q, rl, d) : mv_add<1>(q, rb, d));
+        d = mv_add<1>(zero, cb, d);
+    }
+    V3 b = zero;
+    for (int k = nb - 1; k >= 0; --k) {
+        v3_store(B + B3 * k, n, b);
+        b = mv_add<1>(get(1, k), cb, b);
+    }
+}
+
+// One block of 256 rows x 64 branches (a row of a wave: 256 contiguous bytes).
+// ONE: the block is the whole problem, and the corner is solved here; else its
+// incoming states and g come from k_pfb_join.  Rows past N read as zero and are
+// not written (range-checked buffers).
+template <bool ONE>
+__global__ void __launch_bounds__(64 * SWV, 4)
+k_pfb_solve(const float *__restrict__ yh, int N, const double *__restrict__ tab, const double *__restrict__ tc,
+            const double *__restrict__ A, const double *__restrict__ B, float *__restrict__ x) {
+    // rows of the workgroup's table in LDS
+    constexpr int L_CS = 0, L_RS = 9, L_HS = 18, L_TC = 23, L_N = L_TC + TC_N;
+    static_assert(TB_HS == TB_RS + 9, "a span's responses are contiguous");
+    __shared__ double T[L_N * 64];
+    __shared__ V3 tot[SWV][64], sg[64], sd[64];
+    const int t = threadIdx.x, br = t & 63, wave = t >> 6, n0 = (int)blockIdx.x * 64, n = n0 + br;
+    const int blk = ONE ? 0 : (int)blockIdx.y, r0 = SBLK * blk + SR * wave;
+    const int nv = N - r0;                       // this span's rows: nv, at most 32 (none if <= 0)
+    const __amdgpu_buffer_rsrc_t ry =
+        __builtin_amdgcn_make_buffer_rsrc((void *)(yh + (size_t)SBLK * blk * LB), 0,
+                                          min(N - SBLK * blk, SBLK) * LB * (int)sizeof(float), 0x00020000);
+    double v[SR];
+    const double be1 = tab[n], be2 = tab[LB + n], be3 = tab[2 * LB + n];
+    V3 gin{0.0, 0.0, 0.0}, c0{0.0, 0.0, 0.0}, b0 = c0;
+    if (!ONE) {
+        if (blk == 0 && wave == 0) gin = v3_load(tc + (size_t)TC_G * LB, n);
+        c0 = v3_load(A + (size_t)3 * blk * LB, n);
+        b0 = v3_load(B + (size_t)3 * blk * LB, n);
+    }
+    {
+        float y[SR];
+        const int vo = 4 * (SR * wave * LB + n);
+#pragma unroll
+        for (int k = 0; k < SR; ++k) y[k] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(ry, vo + 4 * LB * k, 0, 0));
+        for (int e = t; e < L_N * 64; e += 64 * SWV) {
+            const int r = e >> 6, c = n0 + (e & 63);
+            T[e] = r < L_RS   ? tab[(size_t)(TB_CS + r) * LB + c]
+                   : r < L_TC ? tab[(size_t)(TB_RS + r - L_RS) * LB + c]
+                              : tc[(size_t)(r - L_TC) * LB + c];
+        }
+#pragma unroll
+        for (int k = 0; k < SR; ++k) v[k] = (double)y[k];
+    }
+    if (!ONE) {
+        v[0] -= gin.a;
+        v[1] -= gin.b;
+        v[2] -= gin.c;
+    }
+    const V3 zero{0.0, 0.0, 0.0};
+    const double *cs = T + L_CS * 64 + br;
+    // the span from zero states, both ways
+    V3 p = zero, q = zero;
+#pragma unroll
+    for (int k = 0; k < SR; ++k) {
+        v[k] = PFB_FILTER(v[k], p);
+        p = V3{v[k], p.a, p.b};
+    }
+    const bool part = nv < SR;                   // the span ends early
+    if (part) {
+#pragma unroll
+        for (int k = 0; k < SR; ++k)
+            if (k >= nv) v[k] = 0.0;
+    }
+#pragma unroll
+    for (int k = SR - 1; k >= 0; --k) q = V3{PFB_FILTER(v[k], q), q.a, q.b};
+    // incoming state: a_j = C^(32 j) c0 + sum_{i < j} C^(32 (j - 1 - i)) p_i
+    tot[wave][br] = p;
+    __syncthreads();
+    V3 a = c0;
+    for (int i = 0; i < wave; ++i) a = mv_add<64>(tot[i][br], cs, a);
+    __syncthreads();
+    // from below: C^(32 (7 - j)) b0 + sum_{i > j} C^(32 (i - 1 - j)) q_i
+    auto suffix = [&](V3 in) {
+        tot[wave][br] = in;
+        __syncthreads();
+        V3 c = b0;
+        for (int i = SWV - 1; i > wave; --i) c = mv_add<64>(tot[i][br], cs, c);
+        return c;
+    };
+    // head response of this span (the partial last one has its own; none past it)
+    const double *rm = T + (part ? L_TC + TC_RS : L_RS) * 64 + br;
+    if (nv > 0) q = mv_add<64>(q, rm, a);
+    V3 b = suffix(q);
+    if (ONE) {
+        if (wave == 0) {
+            const double *h = T + L_HS * 64 + br;
+            const V3 zh = mv_add<64>(q, cs, b);               // zeta[0..2] without the corner
+            const V3 g = mv_add<64>(zero, T + (L_TC + TC_W) * 64 + br, zh);
+            sg[br] = g;
+            // state after the first span from -g on its first three rows
+            sd[br] = V3{-(g.a * h[4 * 64] + g.b * h[3 * 64] + g.c * h[2 * 64]),
+                        -(g.a * h[3 * 64] + g.b * h[2 * 64] + g.c * h[64]),
+                        -(g.a * h[2 * 64] + g.b * h[64] + g.c * h[0])};
+        }
+        __syncthreads();
+        if (wave > 0) {        // C^(32 (j - 1)) of it
+            V3 d = sd[br];
+            for (int i = 1; i < wave; ++i) d = mv_add<64>(zero, cs, d);
+            a = V3{a.a + d.a, a.b + d.b, a.c + d.c};
+            if (nv > 0) q = mv_add<64>(q, rm, d);
+        } else {
+            gin = sg[br];
+        }
+        b = suffix(q);
+    }
+    if (nv <= 0) return;
+    // the rows from their true states
+    {
+        V3 d = a;
+#pragma unroll
+        for (int k = 0; k < SR; ++k) {
+            const double dk = PFB_FILTER(!ONE ? 0.0 : k == 0 ? -gin.a : k == 1 ? -gin.b : k == 2 ? -gin.c : 0.0, d);
+            v[k] += dk;
+            d = V3{dk, d.a, d.b};
+        }
+    }
+    if (part) {
+#pragma unroll
+        for (int k = 0; k < SR; ++k)
+            if (k >= nv) v[k] = 0.0;
+    }
+    const double w0 = tab[(size_t)TB_WZ * LB + n], w1 = tab[(size_t)(TB_WZ + 1) * LB + n],
+                 w2 = tab[(size_t)(TB_WZ + 2) * LB + n], w3 = tab[(size_t)(TB_WZ + 3) * LB + n];
+    // x[i + 3] = w0 z[i+3] + w1 z[i+2] + w2 z[i+1] + w3 z[i]; the first span also x[0..2].
+    // The buffer starts at the block's row i + 3 = SBLK blk + 3.
+    const __amdgpu_buffer_rsrc_t rx =
+        __builtin_amdgcn_make_buffer_rsrc((void *)(x + (size_t)(SBLK * blk + 3) * LB), 0,
+                                          min(N - SBLK * blk, SBLK) * LB * (int)sizeof(float), 0x00020000);
+    const int vs = lds_opaque(4 * (SR * wave * LB + n));   // not the loads' offsets kept live until here
+#pragma unroll
+    for (int k = SR - 1; k >= 0; --k) {
+        const double z = PFB_FILTER(v[k], b);
+        __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint((float)(w0 * b.c + w1 * b.b + w2 * b.a + w3 * z)), rx,
+                                              vs + 4 * LB * k, 0, 0);
+        b = V3{z, b.a, b.b};
+    }
+    if (r0 == 0) {
+        x[(size_t)2 * LB + n] = (float)(w0 * b.c + w1 * b.b + w2 * b.a);
+        x[(size_t)LB + n] = (float)(w0 * b.b + w1 * b.a);
+        x[n] = (float)(w0 * b.a);
+    }
+}
+#undef PFB_FILTER
+
 }  // namespace
 
 struct sdbe_pfb {
@@ -553,6 +1106,11 @@ struct sdbe_pfb {
     double *mf = nullptr;         // [spans][9][32768] forward transfers of full spans
     double *mb = nullptr;         // [spans][9][32768] backward transfers of full spans
     double *state = nullptr;      // [spans][3][32768] incoming state of every span
+    double *tab = nullptr;        // [TB_N][32768] constant-coefficient solve: tables
+    double *tc = nullptr;         // [TC_N][32768] ... of the current call
+    double *bst = nullptr;        // [4][nb][3][32768] ... its blocks' states, out and in, both ways
+    int nb = 0;                   // blocks of max_spec rows
+    int constant = 0;             // no branch has zeros together on the unit circle
 };
 
 namespace {
@@ -578,6 +1136,9 @@ void sdbe_pfb_destroy(sdbe_pfb_t *p) {
     (void)hipFree(p->win);
     (void)hipFree(p->a);
     (void)hipFree(p->yh);
+    (void)hipFree(p->tab);
+    (void)hipFree(p->tc);
+    (void)hipFree(p->bst);
     (void)hipFree(p->uck);
     (void)hipFree(p->ckpt);
     (void)hipFree(p->pst);
@@ -600,25 +1161,14 @@ int sdbe_pfb_create(int device, int32_t n_taps, const float *h_window, int32_t m
     if (!p) return SDBE_ERR_NOMEM;
     p->device = device;
     p->max_spec = max_spectra;
-    // one transfer per span; checkpoints up to the chunk after the last full span
-    const size_t nspan = (size_t)(max_spectra + SPAN - 1) / SPAN;
-    const size_t nck = nspan * (SPAN / SEG) + 1;
-    int rc = SDBE_OK;
+    int rc = SDBE_OK, clustered = 0, *d_clustered = nullptr;
     std::vector<float2> img(FFT_TW_N), tw(NH);
-    std::vector<double> band((size_t)NT * LB);
     const double two_pi = 6.283185307179586476925286766559;
     fft_tw_fill(img.data());
     for (int k = 0; k < NH; ++k) {
         const double ang = two_pi * (double)k / (double)LB;
         tw[k] = make_float2((float)cos(ang), (float)sin(ang));
     }
-    for (int n = 0; n < LB; ++n)
-        for (int d = 0; d < NT; ++d) {
-            double acc = 0.0;
-            for (int k = 0; k + d < NT; ++k)
-                acc += (double)h_window[(size_t)(k + d) * LB + n] * (double)h_window[(size_t)k * LB + n];
-            band[(size_t)d * LB + n] = acc;
-        }
 #define PALLOC(ptr, bytes)                                              \
     do {                                                                \
         if (hipMalloc((void **)&(ptr), (bytes)) != hipSuccess) {        \
@@ -629,30 +1179,60 @@ int sdbe_pfb_create(int device, int32_t n_taps, const float *h_window, int32_t m
     PALLOC(p->fft_img, FFT_TW_N * sizeof(float2));
     PALLOC(p->tw32k, NH * sizeof(float2));
     PALLOC(p->win, (size_t)NT * LB * sizeof(float));
-    PALLOC(p->a, (size_t)NT * LB * sizeof(double));
     PALLOC(p->yh, (size_t)max_spectra * LB * sizeof(float));
-    PALLOC(p->uck, nck * 3 * LB * sizeof(double));
-    PALLOC(p->ckpt, nck * CKW * LB * sizeof(double));
-    PALLOC(p->pst, nspan * 3 * LB * sizeof(double));
-    PALLOC(p->mf, nspan * 9 * LB * sizeof(double));
-    PALLOC(p->mb, nspan * 9 * LB * sizeof(double));
-    PALLOC(p->state, nspan * 3 * LB * sizeof(double));
-#undef PALLOC
+    PALLOC(p->tab, (size_t)TB_N * LB * sizeof(double));
+    PALLOC(p->tc, (size_t)TC_N * LB * sizeof(double));
+    d_clustered = reinterpret_cast<int *>(p->tc);    // until the first call writes its tables
     if (hipMemcpy(p->fft_img, img.data(), FFT_TW_N * sizeof(float2), hipMemcpyHostToDevice) != hipSuccess ||
         hipMemcpy(p->tw32k, tw.data(), NH * sizeof(float2), hipMemcpyHostToDevice) != hipSuccess ||
         hipMemcpy(p->win, h_window, (size_t)NT * LB * sizeof(float), hipMemcpyHostToDevice) != hipSuccess ||
-        hipMemcpy(p->a, band.data(), (size_t)NT * LB * sizeof(double), hipMemcpyHostToDevice) != hipSuccess) {
+        hipMemcpy(d_clustered, &clustered, sizeof(int), hipMemcpyHostToDevice) != hipSuccess) {
         rc = SDBE_ERR_HIP;
         goto fail;
     }
-    // the factor's checkpoints and the full spans' transfers depend on the window only
-    hipLaunchKernelGGL(k_pfb_factor, dim3(LB / SOLVE_WG), dim3(SOLVE_WG), 0, 0, (int)nck, (const double *)p->a,
-                       p->ckpt);
-    hipLaunchKernelGGL(k_pfb_fspan<true>, dim3(LB / SOLVE_WG, nspan), dim3(SOLVE_WG), 0, 0, (const float *)nullptr,
-                       (int)(nspan * SPAN), (const double *)p->a, (const double *)p->ckpt, p->mf);
-    hipLaunchKernelGGL(k_pfb_bspan<true>, dim3(LB / SOLVE_WG, nspan), dim3(SOLVE_WG), 0, 0, (const float *)nullptr,
-                       (const double *)nullptr, (int)(nspan * SPAN), (const double *)p->a, (const double *)p->ckpt,
-                       p->mb);
+    hipLaunchKernelGGL(k_pfb_spectral, dim3(LB / SOLVE_WG), dim3(SOLVE_WG), 0, 0, (const float *)p->win, p->tab,
+                       d_clustered);
+    if (hipMemcpy(&clustered, d_clustered, sizeof(int), hipMemcpyDeviceToHost) != hipSuccess) {
+        rc = SDBE_ERR_HIP;
+        goto fail;
+    }
+    p->constant = clustered == 0;
+    if (p->constant) {
+        p->nb = (max_spectra + SBLK - 1) / SBLK;
+        PALLOC(p->bst, (size_t)4 * 3 * p->nb * LB * sizeof(double));
+    } else {                                         // the factor-row kernels
+        // one transfer per span; checkpoints up to the chunk after the last full span
+        const size_t nspan = (size_t)(max_spectra + SPAN - 1) / SPAN;
+        const size_t nck = nspan * (SPAN / SEG) + 1;
+        std::vector<double> band((size_t)NT * LB);
+        for (int n = 0; n < LB; ++n)
+            for (int d = 0; d < NT; ++d) {
+                double acc = 0.0;
+                for (int k = 0; k + d < NT; ++k)
+                    acc += (double)h_window[(size_t)(k + d) * LB + n] * (double)h_window[(size_t)k * LB + n];
+                band[(size_t)d * LB + n] = acc;
+            }
+        PALLOC(p->a, (size_t)NT * LB * sizeof(double));
+        PALLOC(p->uck, nck * 3 * LB * sizeof(double));
+        PALLOC(p->ckpt, nck * CKW * LB * sizeof(double));
+        PALLOC(p->pst, nspan * 3 * LB * sizeof(double));
+        PALLOC(p->mf, nspan * 9 * LB * sizeof(double));
+        PALLOC(p->mb, nspan * 9 * LB * sizeof(double));
+        PALLOC(p->state, nspan * 3 * LB * sizeof(double));
+        if (hipMemcpy(p->a, band.data(), (size_t)NT * LB * sizeof(double), hipMemcpyHostToDevice) != hipSuccess) {
+            rc = SDBE_ERR_HIP;
+            goto fail;
+        }
+        // the factor's checkpoints and the full spans' transfers depend on the window only
+        hipLaunchKernelGGL(k_pfb_factor, dim3(LB / SOLVE_WG), dim3(SOLVE_WG), 0, 0, (int)nck, (const double *)p->a,
+                           p->ckpt);
+        hipLaunchKernelGGL(k_pfb_fspan<true>, dim3(LB / SOLVE_WG, nspan), dim3(SOLVE_WG), 0, 0, (const float *)nullptr,
+                           (int)(nspan * SPAN), (const double *)p->a, (const double *)p->ckpt, p->mf);
+        hipLaunchKernelGGL(k_pfb_bspan<true>, dim3(LB / SOLVE_WG, nspan), dim3(SOLVE_WG), 0, 0, (const float *)nullptr,
+                           (const double *)nullptr, (int)(nspan * SPAN), (const double *)p->a, (const double *)p->ckpt,
+                           p->mb);
+    }
+#undef PALLOC
     if (hipDeviceSynchronize() != hipSuccess) {
         rc = SDBE_ERR_HIP;
         goto fail;
@@ -682,6 +1262,29 @@ int sdbe_pfb_inverse(sdbe_pfb_t *p, const void *d_spec, int32_t n_spectra, float
     hipStream_t s = (hipStream_t)stream;
     hipLaunchKernelGGL(k_pfb_c2r, dim3(n_spectra), dim3(1024), 0, s, (const float2 *)d_spec, p->yh,
                        (const float2 *)p->fft_img, (const float2 *)p->tw32k);
+    if (p->constant) {
+        const int N = n_spectra, nb = (N + SBLK - 1) / SBLK;
+        const dim3 br(LB / SOLVE_WG), wg(SOLVE_WG);
+        const double *tab = p->tab;
+        const float *yh = p->yh;
+        if (nb == 1) {
+            hipLaunchKernelGGL(k_pfb_corner, br, wg, 0, s, tab, N, p->tc);
+            hipLaunchKernelGGL(k_pfb_solve<true>, dim3(LB / 64), dim3(64 * SWV), 0, s, yh, N, tab, (const double *)p->tc,
+                               (const double *)nullptr, (const double *)nullptr, d_x);
+        } else {
+            double *P = p->bst, *Q = P + (size_t)3 * p->nb * LB, *A = Q + (size_t)3 * p->nb * LB,
+                   *B = A + (size_t)3 * p->nb * LB;
+            hipLaunchKernelGGL(k_pfb_span, dim3(LB / SOLVE_WG, nb), wg, 0, s, yh, N, tab, P, Q);
+            if (nb <= JOIN_LDS)
+                hipLaunchKernelGGL(k_pfb_join<true>, br, wg, 0, s, tab, N, nb, (const double *)P, Q, A, B, p->tc);
+            else
+                hipLaunchKernelGGL(k_pfb_join<false>, br, wg, 0, s, tab, N, nb, (const double *)P, Q, A, B, p->tc);
+            hipLaunchKernelGGL(k_pfb_solve<false>, dim3(LB / 64, nb), dim3(64 * SWV), 0, s, yh, N, tab,
+                               (const double *)p->tc, (const double *)A, (const double *)B, d_x);
+        }
+        PFB_TRY(p, hipGetLastError());
+        return SDBE_OK;
+    }
     const int nspan = (n_spectra + SPAN - 1) / SPAN;
     const dim3 grid(LB / SOLVE_WG, nspan);
     const double *ck = p->ckpt, *a = p->a;
