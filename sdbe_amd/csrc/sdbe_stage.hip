@@ -1127,8 +1127,7 @@ __device__ __forceinline__ void c2_load(const float *__restrict__ Bc, int row, f
 
 template <bool F32, int P>
 __global__ void __launch_bounds__(1024)
-k_stage_c2(const float *__restrict__ Bc, const float2 *__restrict__ thr, const BpDesc *__restrict__ bpd,
-           uint8_t *__restrict__ stage, const int *__restrict__ slot_col, Tables tb, int n_rows) {
+k_stage_c2(float *Bc, const float2 *__restrict__ thr, uint8_t *__restrict__ stage, const int *__restrict__ slot_col, Tables tb, int n_rows) {
     // the work array, then a junk row (words LDS_FFT_N + lane, + 64) that takes
     // the slots without a column, so the scatter has no branches
     __shared__ float lds[LDS_FFT_N + 128];
@@ -1211,11 +1210,14 @@ k_stage_c2(const float *__restrict__ Bc, const float2 *__restrict__ thr, const B
         // element of v[0]: fft16k_tord(t) on the VALU path, t on the matrix-core path
         const int te = P == 0 ? fft16k_tord(t) : t;
         if (F32) {
-            GAS uint64_t *dst = gptr(reinterpret_cast<uint64_t *>(bpd[bpl].out)) + tx + KHI * te;
+            // the row of z, contiguous, over its own (consumed) input row: stored
+            // straight to the output, the 8-byte samples of 64 rows would interleave
+            // at a 512-byte stride (k_samples writes the output)
+            GAS uint64_t *dst = gptr(reinterpret_cast<uint64_t *>(Bc + (size_t)row * 2 * BC_ROW)) + te;
 #pragma unroll
             for (int q = 0; q < 16; ++q) {
                 const float2 y = cscale(v[q], scale);
-                dst[(size_t)KHI * 1024 * q] = (uint64_t)__float_as_uint(y.x) | ((uint64_t)__float_as_uint(y.y) << 32);
+                dst[1024 * q] = (uint64_t)__float_as_uint(y.x) | ((uint64_t)__float_as_uint(y.y) << 32);
             }
         } else {
             const float2 to = thr[bpl];
@@ -1248,6 +1250,31 @@ k_stage_c2(const float *__restrict__ Bc, const float2 *__restrict__ thr, const B
         }
         if (next >= n_rows) break;
         row = next;
+    }
+}
+
+// Float output of a chunk: row tx of a block-pol (stage C2's z[tx + 64 ty], ty =
+// 0..16383, as (samples 2p, 2p + 1) pairs) goes to every 64th pair of its samples.
+// HBM-bound transpose through LDS, 64 rows x 64 columns per workgroup: 512-byte
+// runs in, one 32 KB run out.  33 block-pols: 85 us
+// beside a C2 of 153, where C2 storing them itself took 530.
+__global__ void __launch_bounds__(256) k_samples(const float *__restrict__ Bc, const BpDesc *__restrict__ bpd) {
+    __shared__ float2 tile[64][65];
+    const int t = threadIdx.x, l = t & 63, r0 = t >> 6, ty0 = 64 * blockIdx.x, bpl = blockIdx.y;
+    const float *src = Bc + (size_t)bpl * KHI * 2 * BC_ROW;
+    float2 v[16];
+#pragma unroll
+    for (int i = 0; i < 16; ++i)
+        v[i] = reinterpret_cast<const float2 *>(src + (size_t)(r0 + 4 * i) * 2 * BC_ROW)[ty0 + l];
+#pragma unroll
+    for (int i = 0; i < 16; ++i) tile[r0 + 4 * i][l] = v[i];
+    __syncthreads();
+    GAS uint64_t *dst = gptr(reinterpret_cast<uint64_t *>(bpd[bpl].out)) + (size_t)KHI * ty0 + l;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+        const float2 y = tile[l][r0 + 4 * i];
+        __builtin_nontemporal_store((uint64_t)__float_as_uint(y.x) | ((uint64_t)__float_as_uint(y.y) << 32),
+                                    dst + KHI * (r0 + 4 * i));
     }
 }
 
@@ -1424,13 +1451,13 @@ __global__ void __launch_bounds__(64) k_spectra_desc(SpecDescArgs a, int n_bp, B
 enum KernelId {
     KID_FILL, KID_MAP, KID_REORDER, KID_A, KID_B, KID_C1, KID_STATS, KID_THRESH, KID_C2,
     KID_PACK, KID_HEADERS, KID_TRIM_C2R, KID_TRIM_SEG, KID_TRIM_PACK, KID_A_PK, KID_BITMAP,
-    KID_REORDER8, KID_A_PK8, KID_BITMAP8, KID_TRIM_C2R_PK, KID_CLEAR, KID_N
+    KID_REORDER8, KID_A_PK8, KID_BITMAP8, KID_TRIM_C2R_PK, KID_CLEAR, KID_SAMPLES, KID_N
 };
 static const char *const kKernelNames[KID_N] = {
     "k_fill_i32", "k_packet_map", "k_reorder", "k_stage_a", "k_stage_b",
     "k_stage_c1", "k_stats", "k_thresh", "k_stage_c2", "k_pack", "k_headers", "k_trim_c2r", "k_trim_seg",
     "k_trim_pack", "k_stage_a_pk", "k_group_bitmap", "k_reorder_8x1024", "k_stage_a_pk8",
-    "k_group_bitmap_8x1024", "k_trim_c2r_pk", "k_clear_map"};
+    "k_group_bitmap_8x1024", "k_trim_c2r_pk", "k_clear_map", "k_samples"};
 
 struct ProfRec {
     int kid;
@@ -1689,20 +1716,20 @@ int build_slot_table(sdbe_handle_t *h) {
 
 // Run stages A..C2 over block-pols [0, n_bp) in chunks.
 template <typename K>
-void launch_c2_kernel(sdbe_handle_t *h, int nb, hipStream_t s, const BpDesc *bpd, K kern) {
+void launch_c2_kernel(sdbe_handle_t *h, int nb, hipStream_t s, K kern) {
     const int rows = KHI * nb, pairs = rows / 2;
     const int grid = pairs < h->n_cu ? pairs : h->n_cu;
-    LAUNCH(h, KID_C2, nb, s, kern, dim3(grid), dim3(1024), (const float *)h->Bc, (const float2 *)h->thr, bpd,
-           h->stage, (const int *)h->slot_col, h->tb, rows);
+    LAUNCH(h, KID_C2, nb, s, kern, dim3(grid), dim3(1024), (float *)h->Bc, (const float2 *)h->thr, h->stage,
+           (const int *)h->slot_col, h->tb, rows);
 }
 
 template <bool F32>
-void launch_c2(sdbe_handle_t *h, int nb, hipStream_t s, const BpDesc *bpd) {
+void launch_c2(sdbe_handle_t *h, int nb, hipStream_t s) {
     switch (h->cfg.fft_precision) {
-    case FFT_BF16X3: launch_c2_kernel(h, nb, s, bpd, k_stage_c2<F32, FFT_BF16X3>); break;
-    case FFT_BF16: launch_c2_kernel(h, nb, s, bpd, k_stage_c2<F32, FFT_BF16>); break;
-    case FFT_FP16: launch_c2_kernel(h, nb, s, bpd, k_stage_c2<F32, FFT_FP16>); break;
-    default: launch_c2_kernel(h, nb, s, bpd, k_stage_c2<F32, 0>);
+    case FFT_BF16X3: launch_c2_kernel(h, nb, s, k_stage_c2<F32, FFT_BF16X3>); break;
+    case FFT_BF16: launch_c2_kernel(h, nb, s, k_stage_c2<F32, FFT_BF16>); break;
+    case FFT_FP16: launch_c2_kernel(h, nb, s, k_stage_c2<F32, FFT_FP16>); break;
+    default: launch_c2_kernel(h, nb, s, k_stage_c2<F32, 0>);
     }
 }
 
@@ -1806,9 +1833,10 @@ int run_resampler(sdbe_handle_t *h, const BpDesc *d_bpd, int n_bp, const OutDesc
             LAUNCH(h, KID_THRESH, nb, s, k_thresh, dim3(1), dim3(256), (const double2 *)h->ms, nb, bpd, h->latch,
                    h->thr);
         if (f32) {
-            launch_c2<true>(h, nb, s, bpd);
+            launch_c2<true>(h, nb, s);
+            LAUNCH(h, KID_SAMPLES, nb, s, k_samples, dim3(NCH / 64, nb), dim3(256), (const float *)h->Bc, bpd);
         } else {
-            launch_c2<false>(h, nb, s, bpd);
+            launch_c2<false>(h, nb, s);
             // with the block-pols' headers (FRAMES mode)
             LAUNCH(h, KID_PACK, nb, s, k_pack, dim3(16 * nb), dim3(256), (const uint8_t *)h->stage, bpd, nb, od);
         }
