@@ -145,7 +145,8 @@ typedef struct sdbe_config {
     int32_t use_graph;          /* sdbe_process_blocks: capture the launch
                                    sequence once per batch shape as a HIP graph
                                    and replay it                               */
-    int32_t c1_tiles_per_wg;    /* tuning: stage-C1 tiles per workgroup (1..64, 0 = 8) */
+    int32_t c1_tiles_per_wg;    /* tuning: stage-C1 tiles per workgroup (1..64,
+                                   0 = by the size of the launch, at most 8)   */
     int32_t max_batch_blockpols;/* capacity of sdbe_process_blocks (0 = 1024)   */
     int32_t fft_precision;      /* SDBE_FFT_*: arithmetic of the 16384-point FFT
                                    passes of stages B and C2                   */

@@ -67,7 +67,7 @@ constexpr int G2_PKT_WORDS = 8 + G2_SNAPS * NCH / G2_CIDS / 4;   // 2056
 // (c = a + 39 (16 u + j)), 14 tiles per class, 39 classes.
 constexpr int C1_CLASS_TILES = 14;
 constexpr int C1_TILES = NBLK * C1_CLASS_TILES;   // 546
-constexpr int C1_TILES_PER_WG = 8;                 // default tiles per stage C1 workgroup
+constexpr int C1_TILES_PER_WG = 8;                 // default tiles per stage C1 workgroup of a large launch
 constexpr int C1_INTERLEAVE = 16;                  // default stage C1 workgroups per group of adjacent tiles
 constexpr int BC_ROW = C1_TILES * 32;            // 17472 slots per row of the first-pass output
 constexpr int OUT_FRAME_PAYLOAD = 8192;
@@ -1092,7 +1092,7 @@ struct OutDesc {
 // The workgroups are persistent (one per CU: the FFT's LDS fills a CU) and take
 // the rows of pairs blockIdx.x, blockIdx.x + gridDim.x, ... in turn (pair i =
 // rows 2i, 2i + 1, so that a byte's two nibbles are stored once, by the odd
-// row's pass).  A row arrives in stage C1's
+// row's pass; SINGLE: the rows one by one, each with a byte per ty of its own).  A row arrives in stage C1's
 // tile-major slot order (planar: real plane then imaginary plane) and is
 // scattered into LDS in column order (slot_col: column of each slot, -1 for
 // none); the LDS word of each of a thread's slots is computed once.  The next
@@ -1125,7 +1125,7 @@ __device__ __forceinline__ void c2_load(const float *__restrict__ Bc, int row, f
     pi[C2_NSLOT] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rs, tl, 4 * BC_ROW + 4096 * C2_NSLOT, 0));
 }
 
-template <bool F32, int P>
+template <bool F32, int P, bool SINGLE>
 __global__ void __launch_bounds__(1024)
 k_stage_c2(float *Bc, const float2 *__restrict__ thr, uint8_t *__restrict__ stage, const int *__restrict__ slot_col, Tables tb, int n_rows) {
     // the work array, then a junk row (words LDS_FFT_N + lane, + 64) that takes
@@ -1154,7 +1154,7 @@ k_stage_c2(float *Bc, const float2 *__restrict__ thr, uint8_t *__restrict__ stag
     // rows go in pairs (2 i, 2 i + 1) of one block-pol, pair blockIdx.x, + gridDim.x, ...:
     // the even row's codes wait in hold (byte q & 3 of hold[q >> 2] for element
     // te + 1024 q) and the odd row stores both as one byte
-    int row = 2 * (int)blockIdx.x;
+    int row = SINGLE ? (int)blockIdx.x : 2 * (int)blockIdx.x;
     uint32_t hold[4] = {0u, 0u, 0u, 0u};
     if constexpr (P == 0) c2_load(Bc, row, pr, pi);
     for (;;) {
@@ -1167,7 +1167,7 @@ k_stage_c2(float *Bc, const float2 *__restrict__ thr, uint8_t *__restrict__ stag
             lds_put(lds, (i & 1) ? (int)(pos2[i >> 1] >> 16) : (int)(pos2[i >> 1] & 0xffffu),
                     make_float2(pr[i], pi[i]));
         __syncthreads();
-        const int next = (row & 1) ? row - 1 + 2 * (int)gridDim.x : row + 1;
+        const int next = SINGLE ? row + (int)gridDim.x : (row & 1) ? row - 1 + 2 * (int)gridDim.x : row + 1;
         float2 v[16];
         if constexpr (P == 0) {
             const int tr = row_tid();
@@ -1231,7 +1231,13 @@ k_stage_c2(float *Bc, const float2 *__restrict__ thr, uint8_t *__restrict__ stag
                 code[q] = ((fabsf(a) >= to.x) ? 3u : 2u) ^ (a < 0.f ? 3u : 0u) ^
                           ((fabsf(b) >= to.x) ? 12u : 8u) ^ (b < 0.f ? 12u : 0u);
             }
-            if ((tx & 1) == 0) {   // workgroup-uniform
+            if constexpr (SINGLE) {
+                const __amdgpu_buffer_rsrc_t rd = __builtin_amdgcn_make_buffer_rsrc(
+                    (void *)(stage + (size_t)row * NCH), 0, NCH, BUF_RSRC_WORD3);
+#pragma unroll
+                for (int q = 0; q < 16; ++q)
+                    __builtin_amdgcn_raw_buffer_store_b8((uint8_t)code[q], rd, te, 1024 * q, 0);
+            } else if ((tx & 1) == 0) {   // workgroup-uniform
 #pragma unroll
                 for (int j = 0; j < 4; ++j)
                     hold[j] = code[4 * j] | (code[4 * j + 1] << 8) | (code[4 * j + 2] << 16) | (code[4 * j + 3] << 24);
@@ -1312,16 +1318,21 @@ __device__ __forceinline__ uint32_t pack_word(const uint32_t (&M)[32], int w) {
            (((M[i0 + 2] >> (8 * j)) & 0xFFu) << 16) | (((M[i0 + 3] >> (8 * j)) & 0xFFu) << 24);
 }
 
+// SINGLE: stage C2 stored its rows one by one, M_i = S[2i] | S[2i+1] << 4 is formed here.
+template <bool SINGLE>
 __global__ void __launch_bounds__(256)
 k_pack(const uint8_t *__restrict__ stage, const BpDesc *__restrict__ bpd, int nb, OutDesc od) {
     const int bpl = blockIdx.x >> 4, c = ((blockIdx.x & 15) << 8) + threadIdx.x;   // 4096 column quads
     // the block-pol's 64 frame headers (FRAMES mode), by its first workgroup
     if (od.hdr_bytes && od.bp_headers && (blockIdx.x & 15) == 0 && threadIdx.x < OUT_FRAMES_BLOCK)
         stamp_header(bpd[bpl], (int)threadIdx.x, od.frame_bytes);
-    const GAS uint32_t *src = gptr(reinterpret_cast<const uint32_t *>(stage + (size_t)bpl * (KHI / 2) * NCH)) + c;
+    const GAS uint32_t *src =
+        gptr(reinterpret_cast<const uint32_t *>(stage + (size_t)bpl * (SINGLE ? KHI : KHI / 2) * NCH)) + c;
     uint32_t M[32];
 #pragma unroll
-    for (int i = 0; i < 32; ++i) M[i] = src[(size_t)i * (NCH / 4)];
+    for (int i = 0; i < 32; ++i)
+        M[i] = SINGLE ? src[(size_t)(2 * i) * (NCH / 4)] | (src[(size_t)(2 * i + 1) * (NCH / 4)] << 4)
+                      : src[(size_t)i * (NCH / 4)];
     GAS uint8_t *ob = gptr(bpd[bpl].out) + od.hdr_bytes;
     const int64_t qb0 = 128 * (int64_t)c;                 // stream byte of the run, relative to the block
     if (od.shift_bytes == 0 && od.lim_bytes == INT64_MAX && (((uintptr_t)ob) & 15) == 0) {
@@ -1503,7 +1514,7 @@ struct sdbe_handle {
     BpDesc *g_h = nullptr, *g_d = nullptr;
     hipEvent_t g_done = nullptr;
     int g_used = 0;
-    int c1_tpw = 8;
+    int c1_tpw = 0;                  // 0: by the size of the launch (c1_tiles)
     int c1_ilv = 16;
     int n_cu = 256;                  // compute units of the device
     int prof_kid = -1;               // profile only this kernel kind (-1: all)
@@ -1715,22 +1726,51 @@ int build_slot_table(sdbe_handle_t *h) {
 }
 
 // Run stages A..C2 over block-pols [0, n_bp) in chunks.
-template <typename K>
-void launch_c2_kernel(sdbe_handle_t *h, int nb, hipStream_t s, K kern) {
-    const int rows = KHI * nb, pairs = rows / 2;
-    const int grid = pairs < h->n_cu ? pairs : h->n_cu;
-    LAUNCH(h, KID_C2, nb, s, kern, dim3(grid), dim3(1024), (float *)h->Bc, (const float2 *)h->thr, h->stage,
-           (const int *)h->slot_col, h->tb, rows);
+template <bool F32, int P>
+void launch_c2_kernel(sdbe_handle_t *h, int nb, hipStream_t s, bool single) {
+    const int rows = KHI * nb, units = single ? rows : rows / 2;
+    const int grid = units < h->n_cu ? units : h->n_cu;
+    if (F32 || single)
+        LAUNCH(h, KID_C2, nb, s, (k_stage_c2<F32, P, true>), dim3(grid), dim3(1024), (float *)h->Bc,
+               (const float2 *)h->thr, h->stage, (const int *)h->slot_col, h->tb, rows);
+    else
+        LAUNCH(h, KID_C2, nb, s, (k_stage_c2<F32, P, F32>), dim3(grid), dim3(1024), (float *)h->Bc,
+               (const float2 *)h->thr, h->stage, (const int *)h->slot_col, h->tb, rows);
 }
 
 template <bool F32>
-void launch_c2(sdbe_handle_t *h, int nb, hipStream_t s) {
+void launch_c2(sdbe_handle_t *h, int nb, hipStream_t s, bool single) {
     switch (h->cfg.fft_precision) {
-    case FFT_BF16X3: launch_c2_kernel(h, nb, s, k_stage_c2<F32, FFT_BF16X3>); break;
-    case FFT_BF16: launch_c2_kernel(h, nb, s, k_stage_c2<F32, FFT_BF16>); break;
-    case FFT_FP16: launch_c2_kernel(h, nb, s, k_stage_c2<F32, FFT_FP16>); break;
-    default: launch_c2_kernel(h, nb, s, k_stage_c2<F32, 0>);
+    case FFT_BF16X3: launch_c2_kernel<F32, FFT_BF16X3>(h, nb, s, single); break;
+    case FFT_BF16: launch_c2_kernel<F32, FFT_BF16>(h, nb, s, single); break;
+    case FFT_FP16: launch_c2_kernel<F32, FFT_FP16>(h, nb, s, single); break;
+    default: launch_c2_kernel<F32, 0>(h, nb, s, single);
     }
+}
+
+// Block-pols up to which stage C2 may store its code rows one by one (the stage
+// buffer of a handle holds that many at 64 rows each, or its chunk at 32).
+constexpr int C2_SINGLE_MAX = 24;
+
+// Rows in pairs halve C2's stores and k_pack's reads (0.3 us per block-pol), but
+// a workgroup then runs two rows in turn: with few block-pols that can cost a
+// row time (12 us) in the last round, or half the CUs when the pairs are fewer
+// than the CUs.  One by one where it saves a round: 1 block-pol 24 -> 13 us, 12
+// block-pols 54 -> 41; from some 24 on the bytes cost as much as the round.
+bool c2_single(const sdbe_handle_t *h, int nb) {
+    const int rows = KHI * nb, cu = h->n_cu;
+    return nb <= C2_SINGLE_MAX && (rows + cu - 1) / cu < 2 * ((rows / 2 + cu - 1) / cu);
+}
+
+// Stage-C1 tiles per workgroup where the configuration does not say: 8 (fewer
+// lose the prefetch of the next tile), but on small calls enough workgroups to
+// fill the chip three times over (5 per CU), which the latency of a tile's phases
+// needs more than the prefetch.  1, 4, 12, 24 block-pols with 8 tiles: 27, 31, 53,
+// 87 us; as chosen here 12, 22, 47, 83.
+int c1_tiles(const sdbe_handle_t *h, int nb) {
+    if (h->c1_tpw) return h->c1_tpw;
+    const int fill = 15 * h->n_cu, t = (C1_TILES * nb + fill / 2) / fill;
+    return t < 1 ? 1 : t > C1_TILES_PER_WG ? C1_TILES_PER_WG : t;
 }
 
 // The band-trimmed resampler over n_bp blocks of D snapshots, in chunks: the
@@ -1822,23 +1862,27 @@ int run_resampler(sdbe_handle_t *h, const BpDesc *d_bpd, int n_bp, const OutDesc
                        xm, rows);
             }
         }
-        // whole groups of c1_ilv workgroups, c1_tpw tiles each
-        const int per_grp = h->c1_tpw * h->c1_ilv;
+        // whole groups of c1_ilv workgroups, tpw tiles each
+        const int tpw = c1_tiles(h, nb), per_grp = tpw * h->c1_ilv;
         const int c1_wgs = (C1_TILES * nb + per_grp - 1) / per_grp * h->c1_ilv;
         LAUNCH(h, KID_C1, nb, s, k_stage_c1, dim3(c1_wgs), dim3(256), (const float2 *)h->Zf, (float *)h->Bc, h->part, h->tb,
-               nb, h->c1_tpw, h->c1_ilv);
+               nb, tpw, h->c1_ilv);
         LAUNCH(h, KID_STATS, nb, s, k_stats, dim3(nb), dim3(256), (const double *)h->part, bp0, h->ms, d_stats, bpd,
                h->thr);
         if (ref_walk)   // some block-pol of the call has the REFERENCE policy
             LAUNCH(h, KID_THRESH, nb, s, k_thresh, dim3(1), dim3(256), (const double2 *)h->ms, nb, bpd, h->latch,
                    h->thr);
         if (f32) {
-            launch_c2<true>(h, nb, s);
+            launch_c2<true>(h, nb, s, true);
             LAUNCH(h, KID_SAMPLES, nb, s, k_samples, dim3(NCH / 64, nb), dim3(256), (const float *)h->Bc, bpd);
         } else {
-            launch_c2<false>(h, nb, s);
+            const bool single = c2_single(h, nb);
+            launch_c2<false>(h, nb, s, single);
             // with the block-pols' headers (FRAMES mode)
-            LAUNCH(h, KID_PACK, nb, s, k_pack, dim3(16 * nb), dim3(256), (const uint8_t *)h->stage, bpd, nb, od);
+            if (single)
+                LAUNCH(h, KID_PACK, nb, s, k_pack<true>, dim3(16 * nb), dim3(256), (const uint8_t *)h->stage, bpd, nb, od);
+            else
+                LAUNCH(h, KID_PACK, nb, s, k_pack<false>, dim3(16 * nb), dim3(256), (const uint8_t *)h->stage, bpd, nb, od);
         }
         HIP_TRY(h, hipGetLastError());
     }
@@ -2066,7 +2110,7 @@ int sdbe_create(const sdbe_config_t *cfg_in, int device, sdbe_handle_t **out) {
     h->device = device;
     h->cfg = cfg;
     h->chunk = cfg.chunk_blockpols;
-    h->c1_tpw = cfg.c1_tiles_per_wg ? cfg.c1_tiles_per_wg : C1_TILES_PER_WG;
+    h->c1_tpw = cfg.c1_tiles_per_wg;
     h->c1_ilv = cfg.c1_interleave ? cfg.c1_interleave : C1_INTERLEAVE;
     h->trim = tg;
     if (tg.D) {
@@ -2128,7 +2172,7 @@ int sdbe_create(const sdbe_config_t *cfg_in, int device, sdbe_handle_t **out) {
     ALLOC(h->slot_col, C2_SLOT_TAB * sizeof(int));
     ALLOC(h->part, C * C1_TILES * 2 * sizeof(double));
     ALLOC(h->thr, C * sizeof(float2));
-    ALLOC(h->stage, C * (KHI / 2) * NCH);
+    ALLOC(h->stage, (C > 2 * C2_SINGLE_MAX ? C : C < C2_SINGLE_MAX ? 2 * C : 2 * C2_SINGLE_MAX) * (KHI / 2) * NCH);
     ALLOC(h->ms, C * sizeof(double2));
 #undef ALLOC
     if (hipHostMalloc((void **)&h->h_cnt, CNT_N * sizeof(int) + 2 * sizeof(float), hipHostMallocDefault) !=
@@ -2615,7 +2659,7 @@ constexpr size_t NA_V = 0;
 constexpr size_t NA_ZF = NA_V + na_al((size_t)NA_CHUNK * NBLK * NCH * sizeof(float2));
 constexpr size_t NA_BC = NA_ZF + na_al((size_t)NA_CHUNK * MP * sizeof(float2));
 constexpr size_t NA_STAGE = NA_BC + na_al((size_t)NA_CHUNK * KHI * BC_ROW * sizeof(float2));
-constexpr size_t NA_PART = NA_STAGE + na_al((size_t)NA_CHUNK * (KHI / 2) * NCH);
+constexpr size_t NA_PART = NA_STAGE + na_al((size_t)NA_CHUNK * KHI * NCH);
 constexpr size_t NA_THR = NA_PART + na_al((size_t)NA_CHUNK * C1_TILES * 2 * sizeof(double));
 constexpr size_t NA_MS = NA_THR + na_al((size_t)NA_CHUNK * sizeof(float2));
 constexpr size_t NA_SLOT = NA_MS + na_al((size_t)NA_CHUNK * sizeof(double2));
@@ -2696,7 +2740,7 @@ extern "C" int sdbe_process_spectra_noalloc(const sdbe_config_t *cfg, sdbe_strea
     h.device = dev;
     h.cfg = *cfg;
     h.chunk = NA_CHUNK;
-    h.c1_tpw = cfg->c1_tiles_per_wg ? cfg->c1_tiles_per_wg : C1_TILES_PER_WG;
+    h.c1_tpw = cfg->c1_tiles_per_wg;
     h.c1_ilv = cfg->c1_interleave ? cfg->c1_interleave : C1_INTERLEAVE;
     h.n_cu = nd->n_cu;
     h.tb = tables_bind((const float2 *)(base + NA_TAB));
