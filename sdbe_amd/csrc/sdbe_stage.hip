@@ -2,8 +2,8 @@
 // of include/sdbe_stage.h.
 //
 // Pipeline per group (39 B-frames, both polarisations, 256 block-pols):
-//   k_clear_map + k_packet_map  packet index map [frame][cid][fid], first packet
-//                               wins; invalid / out-of-window packets counted
+//   k_begin + k_packet_map      descriptors in; packet index map [frame][cid][fid],
+//                               first packet wins; invalid / out-of-window packets counted
 //   k_reorder                   LDS transpose of 16 packets per (frame, cid pair)
 //                               into the reference int8 [snapshot][channel][im,re]
 //                               rows, missing packets -> 0 + 0j, fid bitmap
@@ -90,13 +90,6 @@ __device__ __forceinline__ GAS T *gptr(T *p) {
 __global__ void __launch_bounds__(256) k_fill_i32(int *p, int n, int val) {
     int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i < n) p[i] = val;
-}
-
-// A group's packet map to MAP_NONE and its counters to zero, in one launch.
-__global__ void __launch_bounds__(256) k_clear_map(int *__restrict__ map, int n, int *__restrict__ cnt) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) map[i] = MAP_NONE;
-    if (i < CNT_N) cnt[i] = 0;
 }
 
 // One thread per packet: header words 0, 4, 5 give invalid, B-count, cid, fid
@@ -295,6 +288,30 @@ struct BpDesc {
 };
 static_assert(sizeof(BpDesc) == 64, "BpDesc layout");
 
+
+// Start of a call, in one launch: the descriptors out of the call's pinned host
+// table (src, read over the bus by the kernel: a copy beside a fill kernel put
+// 10 us and two gaps in front of every call), the counters to zero, and a
+// group's packet map to MAP_NONE.
+__global__ void __launch_bounds__(256) k_begin(const BpDesc *src, BpDesc *__restrict__ bpd, int n_bp,
+                                               int *__restrict__ map, int n_map, int *__restrict__ cnt) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < n_bp * (int)(sizeof(BpDesc) / 16))
+        reinterpret_cast<uint4 *>(bpd)[i] = reinterpret_cast<const uint4 *>(src)[i];
+    if (i < n_map) map[i] = MAP_NONE;
+    if (i < CNT_N) cnt[i] = 0;
+}
+
+// The counters and latch slot 0, written to their pinned host mirror by the last
+// kernel of a call that does not change them (dst null: not here).
+struct Mirror {
+    const int *src;
+    int *dst;
+};
+constexpr int MIRROR_N = CNT_N + 2;
+__device__ __forceinline__ void mirror_out(const Mirror &m) {
+    if (m.dst && blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x < MIRROR_N) m.dst[threadIdx.x] = m.src[threadIdx.x];
+}
 
 // Word 3 of a raw buffer resource (untyped dword access, gfx9 family): loads
 // through it are range-checked against the resource's size and read 0 past it.
@@ -966,12 +983,21 @@ k_stage_c1(const float2 *__restrict__ Zf, float *__restrict__ Bc, double *__rest
 //   sigma = sqrt((sum x^2 - L mean^2) / (L - 1))
 // PER_BLOCK and FIXED thresholds depend on the block-pol alone and are written
 // here; the REFERENCE walk (k_thresh) runs only for chunks that need it.
+// (mean, sigma) from the block-pol's sums W and Re Y[0].
+__device__ __forceinline__ double2 block_moments(double w, double y0) {
+    const double L = 2097152.0, FA = 65536.0;
+    const double sumsq = w / (FA * FA * L);
+    const double mean = y0 / (FA * L);
+    double var = (sumsq - L * mean * mean) / (L - 1.0);
+    if (var < 0.0) var = 0.0;
+    return make_double2(mean, sqrt(var));
+}
+
 __global__ void __launch_bounds__(256)
 k_stats(const double *__restrict__ part, int bp0, double2 *__restrict__ ms, double *__restrict__ stats_out,
         const BpDesc *__restrict__ bpd, float2 *__restrict__ thr) {
     __shared__ double red[2][256];
     const int t = threadIdx.x, b = blockIdx.x;
-    const double L = 2097152.0, FA = 65536.0;
     double a = 0.0, d = 0.0;
     for (int i = t; i < C1_TILES; i += 256) {
         a += part[((size_t)b * C1_TILES + i) * 2];
@@ -988,12 +1014,9 @@ k_stats(const double *__restrict__ part, int bp0, double2 *__restrict__ ms, doub
         __syncthreads();
     }
     if (t == 0) {
-        const double sumsq = red[0][0] / (FA * FA * L);
-        const double mean = red[1][0] / (FA * L);
-        double var = (sumsq - L * mean * mean) / (L - 1.0);
-        if (var < 0.0) var = 0.0;
-        const double sig = sqrt(var);
-        ms[b] = make_double2(mean, sig);
+        const double2 m = block_moments(red[0][0], red[1][0]);
+        const double mean = m.x, sig = m.y;
+        ms[b] = m;
         const BpDesc &d = bpd[b];
         if (d.policy != SDBE_THRESH_REFERENCE)
             thr[b] = d.policy == SDBE_THRESH_PER_BLOCK ? make_float2((float)sig, (float)mean)
@@ -1018,17 +1041,17 @@ k_stats(const double *__restrict__ part, int bp0, double2 *__restrict__ ms, doub
 // 28 us for 256 block-pols, this THRTIME); the search back before f runs only
 // for empty leading blocks.
 constexpr int THRESH_MAX_CHUNK = SDBE_MAX_CHUNK;
-__global__ void __launch_bounds__(256) k_thresh(const double2 *__restrict__ ms, int nbpl,
-                                                const BpDesc *__restrict__ bpd, float *__restrict__ latch,
-                                                float2 *__restrict__ thr) {
-    __shared__ float2 sms[THRESH_MAX_CHUNK];      // (sigma, mean) as float
-    __shared__ int sinfo[THRESH_MAX_CHUNK];       // pol | slot << 8, or -1: not REFERENCE
+template <int MAXB>
+__device__ __forceinline__ void thresholds(const double2 *ms, int nbpl, const BpDesc *__restrict__ bpd,
+                                           float *__restrict__ latch, float2 *__restrict__ thr) {
+    __shared__ float2 sms[MAXB];      // (sigma, mean) as float
+    __shared__ int sinfo[MAXB];       // pol | slot << 8, or -1: not REFERENCE
     __shared__ float2 slat[SDBE_LATCH_SLOTS];
     __shared__ int sfirst[SDBE_LATCH_SLOTS], slast[SDBE_LATCH_SLOTS];
     const int t = threadIdx.x;
     if (t < SDBE_LATCH_SLOTS) {
         slat[t] = make_float2(latch[2 * t], latch[2 * t + 1]);
-        sfirst[t] = THRESH_MAX_CHUNK;
+        sfirst[t] = MAXB;
         slast[t] = -1;
     }
     __syncthreads();
@@ -1063,10 +1086,60 @@ __global__ void __launch_bounds__(256) k_thresh(const double2 *__restrict__ ms, 
         thr[b] = l;
     }
     if (t < SDBE_LATCH_SLOTS && slat[t].x == 0.0f && slast[t] >= 0) {
-        const float2 l = sms[sfirst[t] < THRESH_MAX_CHUNK ? sfirst[t] : slast[t]];
+        const float2 l = sms[sfirst[t] < MAXB ? sfirst[t] : slast[t]];
         latch[2 * t] = l.x;
         latch[2 * t + 1] = l.y;
     }
+}
+
+__global__ void __launch_bounds__(256) k_thresh(const double2 *__restrict__ ms, int nbpl,
+                                                const BpDesc *__restrict__ bpd, float *__restrict__ latch,
+                                                float2 *__restrict__ thr) {
+    thresholds<THRESH_MAX_CHUNK>(ms, nbpl, bpd, latch, thr);
+}
+
+// Statistics and thresholds of up to STATS_ONE block-pols in one workgroup, a
+// wave each, so that a small call with a REFERENCE stream launches one kernel for
+// both (4.7 us each).  A lane holds threads l, l + 64, .. of k_stats and adds them
+// in its order: the same sums, bit for bit.
+constexpr int STATS_ONE = 16;
+__global__ void __launch_bounds__(64 * STATS_ONE)
+k_stats_thresh(const double *__restrict__ part, int nb, int bp0, double2 *__restrict__ ms,
+               double *__restrict__ stats_out, const BpDesc *__restrict__ bpd, float *__restrict__ latch,
+               float2 *__restrict__ thr) {
+    __shared__ double2 sms[STATS_ONE];
+    const int l = threadIdx.x & 63, b = threadIdx.x >> 6;
+    if (b < nb) {
+        double v[4][2];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            v[j][0] = v[j][1] = 0.0;
+#pragma unroll
+            for (int i = 0; i < (C1_TILES + 255) / 256; ++i) {
+                const int e = l + 64 * j + 256 * i;
+                if (e < C1_TILES) {
+                    v[j][0] += part[((size_t)b * C1_TILES + e) * 2];
+                    v[j][1] += part[((size_t)b * C1_TILES + e) * 2 + 1];
+                }
+            }
+        }
+        double a = (v[0][0] + v[2][0]) + (v[1][0] + v[3][0]), d = (v[0][1] + v[2][1]) + (v[1][1] + v[3][1]);
+#pragma unroll
+        for (int s = 32; s > 0; s >>= 1) {
+            a += __shfl_down(a, s);
+            d += __shfl_down(d, s);
+        }
+        if (l == 0) {
+            const double2 m = block_moments(a, d);
+            ms[b] = sms[b] = m;
+            if (stats_out) {
+                stats_out[(size_t)(bp0 + b) * 2] = m.x;
+                stats_out[(size_t)(bp0 + b) * 2 + 1] = m.y;
+            }
+        }
+    }
+    __syncthreads();
+    thresholds<STATS_ONE>(sms, nb, bpd, latch, thr);
 }
 
 struct OutDesc {
@@ -1264,7 +1337,9 @@ k_stage_c2(float *Bc, const float2 *__restrict__ thr, uint8_t *__restrict__ stag
 // HBM-bound transpose through LDS, 64 rows x 64 columns per workgroup: 512-byte
 // runs in, one 32 KB run out.  33 block-pols: 85 us
 // beside a C2 of 153, where C2 storing them itself took 530.
-__global__ void __launch_bounds__(256) k_samples(const float *__restrict__ Bc, const BpDesc *__restrict__ bpd) {
+__global__ void __launch_bounds__(256) k_samples(const float *__restrict__ Bc, const BpDesc *__restrict__ bpd,
+                                                 Mirror mir) {
+    mirror_out(mir);
     __shared__ float2 tile[64][65];
     const int t = threadIdx.x, l = t & 63, r0 = t >> 6, ty0 = 64 * blockIdx.x, bpl = blockIdx.y;
     const float *src = Bc + (size_t)bpl * KHI * 2 * BC_ROW;
@@ -1321,7 +1396,8 @@ __device__ __forceinline__ uint32_t pack_word(const uint32_t (&M)[32], int w) {
 // SINGLE: stage C2 stored its rows one by one, M_i = S[2i] | S[2i+1] << 4 is formed here.
 template <bool SINGLE>
 __global__ void __launch_bounds__(256)
-k_pack(const uint8_t *__restrict__ stage, const BpDesc *__restrict__ bpd, int nb, OutDesc od) {
+k_pack(const uint8_t *__restrict__ stage, const BpDesc *__restrict__ bpd, int nb, OutDesc od, Mirror mir) {
+    mirror_out(mir);
     const int bpl = blockIdx.x >> 4, c = ((blockIdx.x & 15) << 8) + threadIdx.x;   // 4096 column quads
     // the block-pol's 64 frame headers (FRAMES mode), by its first workgroup
     if (od.hdr_bytes && od.bp_headers && (blockIdx.x & 15) == 0 && threadIdx.x < OUT_FRAMES_BLOCK)
@@ -1430,8 +1506,12 @@ struct SpecDescArgs {
     int32_t policy, fpb;
     float fixed_th, fixed_off;
 };
-__global__ void __launch_bounds__(64) k_spectra_desc(SpecDescArgs a, int n_bp, BpDesc *__restrict__ bpd) {
+__global__ void __launch_bounds__(64) k_spectra_desc(SpecDescArgs a, int n_bp, BpDesc *__restrict__ bpd,
+                                                     int *__restrict__ cnt, float *__restrict__ latch) {
     const int b = blockIdx.x * blockDim.x + threadIdx.x;
+    // counters and latch slot 0 to zero
+    if (b < CNT_N) cnt[b] = 0;
+    if (b < 2) latch[b] = 0.0f;
     if (b >= n_bp) return;
     const uint64_t n = (uint64_t)b * (uint64_t)a.fpb;
     const uint64_t dft = (uint64_t)a.df + n;
@@ -1462,13 +1542,13 @@ __global__ void __launch_bounds__(64) k_spectra_desc(SpecDescArgs a, int n_bp, B
 enum KernelId {
     KID_FILL, KID_MAP, KID_REORDER, KID_A, KID_B, KID_C1, KID_STATS, KID_THRESH, KID_C2,
     KID_PACK, KID_HEADERS, KID_TRIM_C2R, KID_TRIM_SEG, KID_TRIM_PACK, KID_A_PK, KID_BITMAP,
-    KID_REORDER8, KID_A_PK8, KID_BITMAP8, KID_TRIM_C2R_PK, KID_CLEAR, KID_SAMPLES, KID_N
+    KID_REORDER8, KID_A_PK8, KID_BITMAP8, KID_TRIM_C2R_PK, KID_BEGIN, KID_SAMPLES, KID_N
 };
 static const char *const kKernelNames[KID_N] = {
     "k_fill_i32", "k_packet_map", "k_reorder", "k_stage_a", "k_stage_b",
     "k_stage_c1", "k_stats", "k_thresh", "k_stage_c2", "k_pack", "k_headers", "k_trim_c2r", "k_trim_seg",
     "k_trim_pack", "k_stage_a_pk", "k_group_bitmap", "k_reorder_8x1024", "k_stage_a_pk8",
-    "k_group_bitmap_8x1024", "k_trim_c2r_pk", "k_clear_map", "k_samples"};
+    "k_group_bitmap_8x1024", "k_trim_c2r_pk", "k_begin", "k_samples"};
 
 struct ProfRec {
     int kid;
@@ -1801,13 +1881,15 @@ int run_trim(sdbe_handle_t *h, const BpDesc *d_bpd, int n_bp, const OutDesc &od,
             LAUNCH(h, KID_TRIM_SEG, nb, s, kseg_c, dim3(trim::NSEG * nb), dim3(trim::seg_threads(D)),
                    (const float *)h->V, bpd, (float *)h->Zf, h->part, h->trim_tabs, h->trim.skip,
                    (const float2 *)h->tb.fft);
+        // the counters and latch go to the host with the call's last kernel
+        const Mirror none{nullptr, nullptr}, mir = bp0 + nb == n_bp ? Mirror{h->cnt, h->h_cnt} : none;
         LAUNCH(h, KID_STATS, nb, s, k_trim_stats, dim3(nb), dim3(trim::NSEG), (const double *)h->part, P, bp0, h->ms,
-               d_stats);
+               d_stats, f32 ? mir : none);
         if (!f32) {
             LAUNCH(h, KID_THRESH, nb, s, k_thresh, dim3(1), dim3(256), (const double2 *)h->ms, nb, bpd, h->latch,
                    h->thr);
             LAUNCH(h, KID_TRIM_PACK, nb, s, k_trim_pack, dim3(nb * (trim::NSEG * P / 16 / 256)), dim3(256),
-                   (const float *)h->Zf, (const float2 *)h->thr, bpd, P, od);
+                   (const float *)h->Zf, (const float2 *)h->thr, bpd, P, od, mir);
         }
         HIP_TRY(h, hipGetLastError());
     }
@@ -1867,22 +1949,31 @@ int run_resampler(sdbe_handle_t *h, const BpDesc *d_bpd, int n_bp, const OutDesc
         const int c1_wgs = (C1_TILES * nb + per_grp - 1) / per_grp * h->c1_ilv;
         LAUNCH(h, KID_C1, nb, s, k_stage_c1, dim3(c1_wgs), dim3(256), (const float2 *)h->Zf, (float *)h->Bc, h->part, h->tb,
                nb, tpw, h->c1_ilv);
-        LAUNCH(h, KID_STATS, nb, s, k_stats, dim3(nb), dim3(256), (const double *)h->part, bp0, h->ms, d_stats, bpd,
-               h->thr);
-        if (ref_walk)   // some block-pol of the call has the REFERENCE policy
-            LAUNCH(h, KID_THRESH, nb, s, k_thresh, dim3(1), dim3(256), (const double2 *)h->ms, nb, bpd, h->latch,
+        // ref_walk: some block-pol of the call has the REFERENCE policy
+        if (ref_walk && nb <= STATS_ONE) {
+            LAUNCH(h, KID_STATS, nb, s, k_stats_thresh, dim3(1), dim3(64 * STATS_ONE), (const double *)h->part, nb, bp0,
+                   h->ms, d_stats, bpd, h->latch, h->thr);
+        } else {
+            LAUNCH(h, KID_STATS, nb, s, k_stats, dim3(nb), dim3(256), (const double *)h->part, bp0, h->ms, d_stats, bpd,
                    h->thr);
+            if (ref_walk)
+                LAUNCH(h, KID_THRESH, nb, s, k_thresh, dim3(1), dim3(256), (const double2 *)h->ms, nb, bpd, h->latch,
+                       h->thr);
+        }
+        const Mirror mir = bp0 + nb == n_bp ? Mirror{h->cnt, h->h_cnt} : Mirror{nullptr, nullptr};
         if (f32) {
             launch_c2<true>(h, nb, s, true);
-            LAUNCH(h, KID_SAMPLES, nb, s, k_samples, dim3(NCH / 64, nb), dim3(256), (const float *)h->Bc, bpd);
+            LAUNCH(h, KID_SAMPLES, nb, s, k_samples, dim3(NCH / 64, nb), dim3(256), (const float *)h->Bc, bpd, mir);
         } else {
             const bool single = c2_single(h, nb);
             launch_c2<false>(h, nb, s, single);
             // with the block-pols' headers (FRAMES mode)
             if (single)
-                LAUNCH(h, KID_PACK, nb, s, k_pack<true>, dim3(16 * nb), dim3(256), (const uint8_t *)h->stage, bpd, nb, od);
+                LAUNCH(h, KID_PACK, nb, s, k_pack<true>, dim3(16 * nb), dim3(256), (const uint8_t *)h->stage, bpd, nb, od,
+                       mir);
             else
-                LAUNCH(h, KID_PACK, nb, s, k_pack<false>, dim3(16 * nb), dim3(256), (const uint8_t *)h->stage, bpd, nb, od);
+                LAUNCH(h, KID_PACK, nb, s, k_pack<false>, dim3(16 * nb), dim3(256), (const uint8_t *)h->stage, bpd, nb, od,
+                       mir);
         }
         HIP_TRY(h, hipGetLastError());
     }
@@ -1931,10 +2022,10 @@ int ring_acquire(sdbe_handle_t *h, int &slot) {
     return SDBE_OK;
 }
 
-int ring_upload(sdbe_handle_t *h, int slot, int n_bp, hipStream_t s) {
-    HIP_TRY(h, hipMemcpyAsync(h->d_bpd[slot], h->h_bpd[slot], (size_t)n_bp * sizeof(BpDesc),
-                              hipMemcpyHostToDevice, s));
-    return SDBE_OK;
+// First kernel of a call: descriptors (pinned host -> device), counters, packet map.
+void launch_begin(sdbe_handle_t *h, const BpDesc *src, BpDesc *dst, int n_bp, int n_map, hipStream_t s) {
+    const int words = n_bp * (int)(sizeof(BpDesc) / 16), n = words > n_map ? words : n_map > CNT_N ? n_map : CNT_N;
+    LAUNCH(h, KID_BEGIN, 1, s, k_begin, dim3((n + 255) / 256), dim3(256), src, dst, n_bp, h->map, n_map, h->cnt);
 }
 
 int ring_release(sdbe_handle_t *h, int slot, hipStream_t s) {
@@ -1951,11 +2042,12 @@ sdbe_stream_state_t state_plus(const sdbe_stream_state_t &st, int64_t n_frames) 
     return t;
 }
 
-// The group's packet index map [frame][cid][fid] and counters; then either
+// The group's n_bp descriptors (ring slot), packet index map [frame][cid][fid] and counters; then either
 // the int8 rows (k_reorder) or, for the packet-reading stage A, only the fid
 // bitmap and the unique count.
-int unpack_map(sdbe_handle_t *h, const void *d_pkts, int32_t n_pkts, uint64_t b_zero, hipStream_t s) {
-    LAUNCH(h, KID_CLEAR, 1, s, k_clear_map, dim3((h->map_n + 255) / 256), dim3(256), h->map, h->map_n, h->cnt);
+int unpack_map(sdbe_handle_t *h, const void *d_pkts, int32_t n_pkts, uint64_t b_zero, int slot, int n_bp,
+               hipStream_t s) {
+    launch_begin(h, n_bp ? h->h_bpd[slot] : nullptr, n_bp ? h->d_bpd[slot] : nullptr, n_bp, h->map_n, s);
     if (n_pkts > 0)
         LAUNCH(h, KID_MAP, 1, s, k_packet_map, dim3((n_pkts + MAP_WG - 1) / MAP_WG), dim3(MAP_WG), (const uint32_t *)d_pkts,
                n_pkts, (uint32_t)(b_zero & 0xFFFFFFFFull), h->nfr, h->n_cid, h->n_fid, h->pkt_words, h->map,
@@ -1970,8 +2062,8 @@ bool overlap(const void *a, size_t na, const void *b, size_t nb) {
 }
 
 int unpack_to_rows(sdbe_handle_t *h, const void *d_pkts, int32_t n_pkts, uint64_t b_zero,
-                   int8_t *beng0, int8_t *beng1, uint8_t *d_bitmap, hipStream_t s) {
-    int rc = unpack_map(h, d_pkts, n_pkts, b_zero, s);
+                   int8_t *beng0, int8_t *beng1, uint8_t *d_bitmap, int slot, int n_bp, hipStream_t s) {
+    int rc = unpack_map(h, d_pkts, n_pkts, b_zero, slot, n_bp, s);
     if (rc) return rc;
     if (h->geom == SDBE_GEOM_8X1024)
         LAUNCH(h, KID_REORDER8, 1, s, k_reorder_8x1024, dim3(G2_CIDS, G2_FIDS, h->nfr), dim3(256),
@@ -1985,8 +2077,8 @@ int unpack_to_rows(sdbe_handle_t *h, const void *d_pkts, int32_t n_pkts, uint64_
 }
 
 int unpack_bitmap(sdbe_handle_t *h, const void *d_pkts, int32_t n_pkts, uint64_t b_zero,
-                  uint8_t *d_bitmap, hipStream_t s) {
-    int rc = unpack_map(h, d_pkts, n_pkts, b_zero, s);
+                  uint8_t *d_bitmap, int slot, int n_bp, hipStream_t s) {
+    int rc = unpack_map(h, d_pkts, n_pkts, b_zero, slot, n_bp, s);
     if (rc) return rc;
     if (h->geom == SDBE_GEOM_8X1024)
         LAUNCH(h, KID_BITMAP8, 1, s, k_group_bitmap_8x1024, dim3(h->nfr), dim3(256), (const int *)h->map,
@@ -2005,9 +2097,11 @@ void advance_state(sdbe_stream_state_t &st, int64_t n_frames) {
     st.psn += (uint64_t)n_frames;
 }
 
-int finish_call(sdbe_handle_t *h, hipStream_t s) {
-    // the counters and latch slot 0 lie back to back on both sides: one copy
-    HIP_TRY(h, hipMemcpyAsync(h->h_cnt, h->cnt, CNT_N * sizeof(int) + 2 * sizeof(float), hipMemcpyDeviceToHost, s));
+// copy: no kernel of the call wrote the host mirror (Mirror).  The counters and
+// latch slot 0 lie back to back on both sides: one copy.
+int finish_call(sdbe_handle_t *h, hipStream_t s, bool copy = false) {
+    if (copy)
+        HIP_TRY(h, hipMemcpyAsync(h->h_cnt, h->cnt, MIRROR_N * sizeof(int), hipMemcpyDeviceToHost, s));
     h->last_stream = s;
     return SDBE_OK;
 }
@@ -2175,21 +2269,23 @@ int sdbe_create(const sdbe_config_t *cfg_in, int device, sdbe_handle_t **out) {
     ALLOC(h->stage, (C > 2 * C2_SINGLE_MAX ? C : C < C2_SINGLE_MAX ? 2 * C : 2 * C2_SINGLE_MAX) * (KHI / 2) * NCH);
     ALLOC(h->ms, C * sizeof(double2));
 #undef ALLOC
-    if (hipHostMalloc((void **)&h->h_cnt, CNT_N * sizeof(int) + 2 * sizeof(float), hipHostMallocDefault) !=
+    // pinned tables the kernels read and write: coherent, so that no GPU cache
+    // holds them from one call to the next
+    if (hipHostMalloc((void **)&h->h_cnt, MIRROR_N * sizeof(int), hipHostMallocCoherent) !=
         hipSuccess) {
         rc = SDBE_ERR_NOMEM;
         goto fail;
     }
     h->h_latch = reinterpret_cast<float *>(h->h_cnt + CNT_N);
     for (int i = 0; i < sdbe_handle::RING; ++i) {
-        if (hipHostMalloc((void **)&h->h_bpd[i], (size_t)h->cap_bp * sizeof(BpDesc), hipHostMallocDefault) !=
+        if (hipHostMalloc((void **)&h->h_bpd[i], (size_t)h->cap_bp * sizeof(BpDesc), hipHostMallocCoherent) !=
                 hipSuccess ||
             hipEventCreateWithFlags(&h->bpd_done[i], hipEventDisableTiming) != hipSuccess) {
             rc = SDBE_ERR_NOMEM;
             goto fail;
         }
     }
-    if (hipHostMalloc((void **)&h->g_h, (size_t)h->cap_bp * sizeof(BpDesc), hipHostMallocDefault) != hipSuccess ||
+    if (hipHostMalloc((void **)&h->g_h, (size_t)h->cap_bp * sizeof(BpDesc), hipHostMallocCoherent) != hipSuccess ||
         hipEventCreateWithFlags(&h->g_done, hipEventDisableTiming) != hipSuccess) {
         rc = SDBE_ERR_NOMEM;
         goto fail;
@@ -2278,8 +2374,8 @@ int sdbe_unpack_group_int8(sdbe_handle_t *h, const void *d_pkts, int32_t n_pkts,
                         !overlap(d_beng1, pol_bytes, d_pkts, pkt_bytes) &&
                         !overlap(d_beng0, pol_bytes, d_bitmap, bm_bytes) &&
                         !overlap(d_beng1, pol_bytes, d_bitmap, bm_bytes);
-    int rc = direct ? unpack_to_rows(h, d_pkts, n_pkts, b_zero, d_beng0, d_beng1, d_bitmap, s)
-                    : unpack_to_rows(h, d_pkts, n_pkts, b_zero, h->beng, h->beng + pol_bytes, d_bitmap, s);
+    int rc = direct ? unpack_to_rows(h, d_pkts, n_pkts, b_zero, d_beng0, d_beng1, d_bitmap, 0, 0, s)
+                    : unpack_to_rows(h, d_pkts, n_pkts, b_zero, h->beng, h->beng + pol_bytes, d_bitmap, 0, 0, s);
     if (rc) return rc;
     if (!direct) {
         HIP_TRY(h, hipMemcpyAsync(d_beng0, h->beng, pol_bytes, hipMemcpyDeviceToDevice, s));
@@ -2288,7 +2384,7 @@ int sdbe_unpack_group_int8(sdbe_handle_t *h, const void *d_pkts, int32_t n_pkts,
     h->n_packets_last = n_pkts;
     h->n_bp_last = 0;
     h->have_group = 1;
-    return finish_call(h, s);
+    return finish_call(h, s, true);
 }
 
 int sdbe_process_group(sdbe_handle_t *h, const void *d_pkts, int32_t n_pkts, uint64_t b_zero, void *d_out,
@@ -2305,10 +2401,7 @@ int sdbe_process_group(sdbe_handle_t *h, const void *d_pkts, int32_t n_pkts, uin
     // reads the packets in 8- or 16-byte units: with a 16-byte aligned buffer,
     // as device allocations are; otherwise the int8 rows
     const bool direct = n_pkts > 0 && (((uintptr_t)d_pkts) & 15) == 0;
-    int rc = direct ? unpack_bitmap(h, d_pkts, n_pkts, b_zero, d_bitmap, s)
-                    : unpack_to_rows(h, d_pkts, n_pkts, b_zero, h->beng, h->beng + (size_t)nsnap * NCH * 2, d_bitmap, s);
-    if (rc) return rc;
-    int slot;
+    int slot, rc;
     if ((rc = ring_acquire(h, slot))) return rc;
     const int n_bp = 2 * blocks;
     BpDesc *hb = h->h_bpd[slot];
@@ -2322,7 +2415,10 @@ int sdbe_process_group(sdbe_handle_t *h, const void *d_pkts, int32_t n_pkts, uin
                c.fixed_threshold, c.fixed_offset, c.station_id, c.bdc_sideband, c.rx_sideband);
         hb[bp].blk = blk;
     }
-    if ((rc = ring_upload(h, slot, n_bp, s))) return rc;
+    rc = direct ? unpack_bitmap(h, d_pkts, n_pkts, b_zero, d_bitmap, slot, n_bp, s)
+                : unpack_to_rows(h, d_pkts, n_pkts, b_zero, h->beng, h->beng + (size_t)nsnap * NCH * 2, d_bitmap, slot,
+                                 n_bp, s);
+    if (rc) return rc;
     // Re-framed output: the stream of 2048-word frames starts align_words
     // into the first aligned group; a group's last lead_words words open the
     // next group's first frame (the output thread's time alignment,
@@ -2391,8 +2487,7 @@ int spectra_call(sdbe_handle_t *h, const int8_t *d_beng, int32_t n_bp, uint8_t *
         set_bp(hb[bp], d_beng + (size_t)bp * h->snaps * NCH * 2, out + (int64_t)bp * out_bp_stride,
                state_plus(h->st, (int64_t)bp * h->fpb), 0, 0, c.thresh_policy, 0, c.fixed_threshold,
                c.fixed_offset, c.station_id, c.bdc_sideband, c.rx_sideband);
-    if ((rc = ring_upload(h, slot, n_bp, s))) return rc;
-    hipLaunchKernelGGL(k_fill_i32, dim3(1), dim3(256), 0, s, h->cnt, CNT_N, 0);
+    launch_begin(h, hb, h->d_bpd[slot], n_bp, 0, s);
     rc = run_resampler(h, h->d_bpd[slot], n_bp, out_desc(h), f32, d_stats, s, nullptr,
                        c.thresh_policy == SDBE_THRESH_REFERENCE);
     if (rc) return rc;
@@ -2481,11 +2576,8 @@ int batch_graph(sdbe_handle_t *h, int n_bp) {
     HIP_TRY(h, hipStreamBeginCapture(cs, hipStreamCaptureModeThreadLocal));
     h->capturing = 1;
     hipGraph_t g = nullptr;
-    hipError_t e1 = hipMemcpyAsync(h->g_d, h->g_h, (size_t)n_bp * sizeof(BpDesc), hipMemcpyHostToDevice, cs);
-    if (e1 == hipSuccess) {
-        hipLaunchKernelGGL(k_fill_i32, dim3(1), dim3(256), 0, cs, h->cnt, CNT_N, 0);
-        e1 = hipGetLastError();
-    }
+    launch_begin(h, h->g_h, h->g_d, n_bp, 0, cs);
+    hipError_t e1 = hipGetLastError();
     int rc = e1 == hipSuccess ? run_resampler(h, h->g_d, n_bp, out_desc(h), false, nullptr, cs) : SDBE_OK;
     hipError_t e2 = hipStreamEndCapture(cs, &g);
     h->capturing = 0;
@@ -2517,7 +2609,7 @@ int sdbe_process_blocks(sdbe_handle_t *h, const sdbe_stream_desc_t *streams, int
     if (n_bp > 0) {
         if (h->cfg.use_graph) {
             if ((rc = batch_graph(h, n_bp))) return rc;
-            // the graph copies g_h in: wait until its previous launch has done so
+            // the graph's first kernel reads g_h: wait until its previous launch has done so
             if (h->g_used) HIP_TRY(h, hipEventSynchronize(h->g_done));
             fill_batch(h, streams, n_streams, h->g_h);
             HIP_TRY(h, hipGraphLaunch(h->gexec, s));
@@ -2527,8 +2619,7 @@ int sdbe_process_blocks(sdbe_handle_t *h, const sdbe_stream_desc_t *streams, int
             int slot;
             if ((rc = ring_acquire(h, slot))) return rc;
             fill_batch(h, streams, n_streams, h->h_bpd[slot]);
-            if ((rc = ring_upload(h, slot, n_bp, s))) return rc;
-            hipLaunchKernelGGL(k_fill_i32, dim3(1), dim3(256), 0, s, h->cnt, CNT_N, 0);
+            launch_begin(h, h->h_bpd[slot], h->d_bpd[slot], n_bp, 0, s);
             bool any_ref = false;
             for (int i = 0; i < n_streams; ++i)
                 any_ref |= streams[i].n_blocks > 0 && streams[i].thresh_policy == SDBE_THRESH_REFERENCE;
@@ -2541,7 +2632,7 @@ int sdbe_process_blocks(sdbe_handle_t *h, const sdbe_stream_desc_t *streams, int
     h->n_packets_last = 0;
     h->n_bp_last = n_bp;
     h->have_group = 0;
-    return finish_call(h, s);
+    return finish_call(h, s, n_bp == 0);
 }
 
 int sdbe_set_output_alignment(sdbe_handle_t *h, int32_t enable, int32_t skip_int32, int32_t skip_frames) {
@@ -2759,8 +2850,6 @@ extern "C" int sdbe_process_spectra_noalloc(const sdbe_config_t *cfg, sdbe_strea
     const OutDesc od = out_desc(&h);
     // the array keeps the previous call's contents: the counters and the
     // REFERENCE latch (slot 0) start at zero in every call
-    hipLaunchKernelGGL(k_fill_i32, dim3(1), dim3(256), 0, s, h.cnt, CNT_N, 0);
-    hipLaunchKernelGGL(k_fill_i32, dim3(1), dim3(64), 0, s, (int *)h.latch, 2, 0);
     SpecDescArgs a;
     a.rows = d_beng;
     a.out = (uint8_t *)d_out;
@@ -2776,7 +2865,7 @@ extern "C" int sdbe_process_spectra_noalloc(const sdbe_config_t *cfg, sdbe_strea
     a.fpb = OUT_FRAMES_BLOCK;
     a.fixed_th = cfg->fixed_threshold;
     a.fixed_off = cfg->fixed_offset;
-    hipLaunchKernelGGL(k_spectra_desc, dim3((n_bp + 63) / 64), dim3(64), 0, s, a, n_bp, bpd);
+    hipLaunchKernelGGL(k_spectra_desc, dim3((n_bp + 63) / 64), dim3(64), 0, s, a, n_bp, bpd, h.cnt, h.latch);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return SDBE_ERR_HIP;
     rc = run_resampler(&h, bpd, n_bp, od, false, nullptr, s, nullptr, cfg->thresh_policy == SDBE_THRESH_REFERENCE);

@@ -717,7 +717,9 @@ k_trim_seg(const float *__restrict__ T, const BpDesc *__restrict__ bpd, float *_
 
 // Mean and sigma (ddof 1) of each block from the segment sums: ms[b] = (mean, sigma).
 __global__ void __launch_bounds__(128)
-k_trim_stats(const double *__restrict__ part, int P, int bp0, double2 *__restrict__ ms, double *__restrict__ stats_out) {
+k_trim_stats(const double *__restrict__ part, int P, int bp0, double2 *__restrict__ ms, double *__restrict__ stats_out,
+             Mirror mir) {
+    mirror_out(mir);
     __shared__ double red[2][trim::NSEG];
     const int t = threadIdx.x, b = blockIdx.x;
     red[0][t] = part[((size_t)b * trim::NSEG + t) * 2];
@@ -749,7 +751,8 @@ k_trim_stats(const double *__restrict__ part, int P, int bp0, double2 *__restric
 // stream byte q to frame q / 8192 of the block's output.  Thread = one 32-bit word.
 __global__ void __launch_bounds__(256)
 k_trim_pack(const float *__restrict__ stage, const float2 *__restrict__ thr, const BpDesc *__restrict__ bpd, int P,
-            OutDesc od) {
+            OutDesc od, Mirror mir) {
+    mirror_out(mir);
     const int words = trim::NSEG * P / 16;
     const int wpb = words / 256;                      // workgroups per block
     const int bpl = blockIdx.x / wpb, wi = (blockIdx.x - bpl * wpb) * 256 + threadIdx.x;
