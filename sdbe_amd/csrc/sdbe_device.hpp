@@ -509,19 +509,23 @@ __device__ __forceinline__ void fft16k_p3(float2 *v, float *lds, const FftTw *tw
     for (int q = 0; q < 16; ++q) v[q] = lds_get(lds, rd + 2048 * q);
 }
 
+// butterfly b of the thread's four: elements t + 1024 (b + 4 r) in v[b + 4 r]
+template <int S>
+__device__ __forceinline__ void fft16k_p4_one(float2 *v, const FftTw *tw, int t, int b) {
+    const uint32_t j = (uint32_t)(t + 1024 * b);
+    const uint32_t j2 = 2u * j;   // < 8192
+    const float2 w1 = ctw<S>(cmul(tw->h16k[j >> 7], tw->l16k[j & 127]));
+    const float2 w2 = ctw<S>(cmul(tw->h16k[j2 >> 7], tw->l16k[j2 & 127]));
+    v[b + 4] = cmul(v[b + 4], w1);
+    v[b + 8] = cmul(v[b + 8], w2);
+    v[b + 12] = cmul(v[b + 12], cmul(w1, w2));
+    dft4<S>(v[b], v[b + 4], v[b + 8], v[b + 12]);
+}
+
 template <int S>
 __device__ __forceinline__ void fft16k_p4(float2 *v, const FftTw *tw, int t) {
 #pragma unroll
-    for (int b = 0; b < 4; ++b) {
-        const uint32_t j = (uint32_t)(t + 1024 * b);
-        const uint32_t j2 = 2u * j;   // < 8192
-        const float2 w1 = ctw<S>(cmul(tw->h16k[j >> 7], tw->l16k[j & 127]));
-        const float2 w2 = ctw<S>(cmul(tw->h16k[j2 >> 7], tw->l16k[j2 & 127]));
-        v[b + 4] = cmul(v[b + 4], w1);
-        v[b + 8] = cmul(v[b + 8], w2);
-        v[b + 12] = cmul(v[b + 12], cmul(w1, w2));
-        dft4<S>(v[b], v[b + 4], v[b + 8], v[b + 12]);
-    }
+    for (int b = 0; b < 4; ++b) fft16k_p4_one<S>(v, tw, t, b);
 }
 
 }  // namespace sdbe

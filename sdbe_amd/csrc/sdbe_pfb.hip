@@ -13,7 +13,8 @@
 // Kernels:
 //   k_pfb_fold_r2c  one workgroup per spectrum: 4-tap fold, packed R2C
 //                   (16384-point complex FFT in LDS + split post-processing)
-//   k_pfb_c2r       one workgroup per spectrum: packed C2R to the pseudo-timestream
+//   k_pfb_fold2_r2c the same for calls of more spectra than CUs, two at a time
+//   k_pfb_c2r       packed C2R of each spectrum to the pseudo-timestream
 // The solve, for any prototype without zeros together on the unit circle:
 //   k_pfb_spectral  once per plan, one thread per branch: the constant
 //                   minimum-phase factor of P P^T and the tables built on it
@@ -63,6 +64,48 @@ constexpr int SOLVE_WG = 64;
 
 static_assert(NH == NCH, "the PFB reuses the 16384-point FFT");
 
+// s + S i w d, in four fused multiply-adds (two roundings a component)
+template <int S> __device__ __forceinline__ float2 add_i_mul(float2 s, float2 w, float2 d) {
+    constexpr float f = (float)S;
+    return make_float2(fmaf(-f * w.x, d.y, fmaf(-f * w.y, d.x, s.x)), fmaf(f * w.x, d.x, fmaf(-f * w.y, d.y, s.y)));
+}
+
+// e^{2 pi i (t + 1024 q)/L} from T = e^{2 pi i t/L}: the product in FP64, which this
+// chip issues at FP32's rate, so that its one rounding is a table entry's (the
+// product of two FP32 factors raised the error of the whole transform by 3 to 4%).
+__device__ __forceinline__ float2 split_tw(double2 T, int q) {
+    const double c = __builtin_cos(6.283185307179586476925286766559 * q / 32),
+                 s = __builtin_sin(6.283185307179586476925286766559 * q / 32);
+    return make_float2((float)fma(T.x, c, -T.y * s), (float)fma(T.x, s, T.y * c));
+}
+
+// The split of a packed transform, Z (element t + 1024 q in v[q]) to bins k = t +
+// 1024 q of out: X[k] = 1/2 (Z[k] + conj Z[N-k]) - 1/2 i e^{-2 pi i k/L} (Z[k] - conj Z[N-k]),
+// the mirror bins through LDS.
+__device__ __forceinline__ void r2c_split(float2 (&v)[16], float *lds, int t, const double2 *__restrict__ tw1k,
+                                          float2 *__restrict__ out) {
+    const double2 T = tw1k[t];
+    __syncthreads();                         // the FFT's last LDS reads are done
+    const int rd = lds_re(t);
+#pragma unroll
+    for (int q = 0; q < 16; ++q) lds_put(lds, rd + 2048 * q, v[q]);
+    __syncthreads();
+    // mirror of t + 1024 q: (1024 - t) + 1024 (15 - q); t = 0: 1024 ((16 - q) & 15)
+    const int rm = lds_re((1024 - t) & 1023);
+#pragma unroll
+    for (int q = 0; q < 16; ++q) {
+        const int mq = t == 0 ? (16 - q) & 15 : 15 - q;
+        const float2 zm = cconj(lds_get(lds, rm + 2048 * mq));   // conj Z[N - k]
+        const float2 E = cscale(cadd(v[q], zm), 0.5f);
+        const float2 D = cscale(csub(v[q], zm), 0.5f);
+        // streamed out: ordinary stores evict the blocks the neighbours read again
+        __builtin_nontemporal_store(
+            __builtin_bit_cast(uint64_t, add_i_mul<-1>(E, cconj(split_tw(T, q)), D)),
+            reinterpret_cast<uint64_t *>(out + t + 1024 * q));
+    }
+    if (t == 0) out[NH] = make_float2(v[0].x - v[0].y, 0.f);
+}
+
 // Forward PFB of spectrum i.  z[m] = y[2m] + i y[2m+1] of the folded block;
 // Z = FFT_16384(z); X[k] = 1/2 (Z[k] + conj Z[N-k]) - 1/2 i e^{-2 pi i k/L} (Z[k] - conj Z[N-k]),
 // X[N] = Re Z[0] - Im Z[0].
@@ -71,7 +114,7 @@ static_assert(NH == NCH, "the PFB reuses the 16384-point FFT");
 // blocks, so most block reads are hits in that XCD's L2.
 __global__ void __launch_bounds__(1024)
 k_pfb_fold_r2c(const float *__restrict__ x, const float *__restrict__ win, float2 *__restrict__ spec,
-               const float2 *__restrict__ fft_img, const float2 *__restrict__ tw32k) {
+               const float2 *__restrict__ fft_img, const double2 *__restrict__ tw1k) {
     __shared__ float lds[LDS_FFT_N];
     __shared__ FftTw ftw;
     fft_tw_load(&ftw, fft_img);
@@ -93,54 +136,144 @@ k_pfb_fold_r2c(const float *__restrict__ x, const float *__restrict__ win, float
         v[q] = acc;
     }
     fft16k<-1>(v, lds, &ftw);
-    __syncthreads();    // the FFT's last LDS reads are done
+    r2c_split(v, lds, t, tw1k, spec + (size_t)i * NBIN);
+}
+
+// The forward transform of calls of more spectra than CUs: persistent, two
+// consecutive spectra at a time.  Folding one spectrum reads 4 blocks and 4 blocks
+// of taps, 1 MB through the CU's L1 (7 us at its 64 bytes a clock, beside 9 us of
+// transform); two read 5 and 4 together, and the second's folded samples wait in
+// 32 registers while the first is transformed (one copy of the transform's code,
+// looped: with two the allocator spills 200 registers).  The pairs of an XCD are
+// neighbours, whose blocks overlap.  4096 spectra: 383 us (424 with ordinary
+// stores); one spectrum per workgroup 567; a fold pass of its own and a
+// persistent transform 186 + 247.  400 spectra: 42 and 53 us.
+__global__ void __launch_bounds__(1024)
+k_pfb_fold2_r2c(const float *__restrict__ x, int n, const float *__restrict__ win, float2 *__restrict__ spec,
+                const float2 *__restrict__ fft_img, const double2 *__restrict__ tw1k) {
+    __shared__ float lds[LDS_FFT_N];
+    __shared__ FftTw ftw;
+    fft_tw_load(&ftw, fft_img);
+    const int pairs = (n + 1) >> 1;
+    const __amdgpu_buffer_rsrc_t rw =
+        __builtin_amdgcn_make_buffer_rsrc((void *)win, 0, NT * LB * (int)sizeof(float), 0x00020000);
+    for (int p = xcd_contig((int)blockIdx.x, (int)gridDim.x); p < pairs; p += (int)gridDim.x) {
+        const int i = 2 * p;
+        const int blocks = min(NT + 1, n + NT - 1 - i);       // 4 when spectrum i + 1 does not exist
+        const __amdgpu_buffer_rsrc_t rx = __builtin_amdgcn_make_buffer_rsrc(
+            (void *)(x + (size_t)i * LB), 0, blocks * LB * (int)sizeof(float), 0x00020000);
+        const int last = 4 * LB * (blocks - 1);
+        float2 a[16], b[16], w[2][NT], v[2][NT + 1];
+        const int t0 = row_tid();
+        // one q ahead: with more in flight the sums spill (2 ahead 462 us, 3 475)
+        auto fetch = [&](int q) {
 #pragma unroll
-    for (int q = 0; q < 16; ++q) {
-        const int k = t + 1024 * q;
-        lds_put(lds, lds_re(k), v[q]);
-    }
-    __syncthreads();
-    float2 *out = spec + (size_t)i * NBIN;
+            for (int k = 0; k < NT; ++k)
+                w[q & 1][k] = __builtin_bit_cast(
+                    float2, __builtin_amdgcn_raw_buffer_load_b64(rw, 8 * t0, 4 * LB * k + 8192 * q, 0));
 #pragma unroll
-    for (int q = 0; q < 16; ++q) {
-        const int k = t + 1024 * q;
-        const int km = (NH - k) & (NH - 1);
-        const float2 zm = cconj(lds_get(lds, lds_re(km)));   // conj Z[N - k]
-        const float2 E = cscale(cadd(v[q], zm), 0.5f);
-        const float2 D = cscale(csub(v[q], zm), 0.5f);
-        out[k] = cadd(E, mul_si<-1>(cmul(cconj(tw32k[k]), D)));
+            for (int k = 0; k <= NT; ++k)
+                v[q & 1][k] = __builtin_bit_cast(
+                    float2, __builtin_amdgcn_raw_buffer_load_b64(rx, 8 * t0, (k < NT ? 4 * LB * k : last) + 8192 * q, 0));
+        };
+        fetch(0);
+#pragma unroll
+        for (int q = 0; q < 16; ++q) {
+            if (q < 15) fetch(q + 1);
+            __builtin_amdgcn_sched_barrier(0);
+            a[q] = b[q] = make_float2(0.f, 0.f);
+#pragma unroll
+            for (int k = 0; k < NT; ++k) {
+                const float2 wk = w[q & 1][k], va = v[q & 1][k], vb = v[q & 1][k + 1];
+                a[q].x = fmaf(wk.x, va.x, a[q].x);
+                a[q].y = fmaf(wk.y, va.y, a[q].y);
+                b[q].x = fmaf(wk.x, vb.x, b[q].x);
+                b[q].y = fmaf(wk.y, vb.y, b[q].y);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+#pragma unroll 1
+        for (int h = 0; h < 2 && i + h < n; ++h) {            // workgroup-uniform
+            const int t = row_tid();
+            fft16k_p123<-1>(a, lds, &ftw, t);
+            fft16k_p4<-1>(a, &ftw, t);
+            r2c_split(a, lds, t, tw1k, spec + (size_t)(i + h) * NBIN);
+#pragma unroll
+            for (int q = 0; q < 16; ++q) a[q] = b[q];
+        }
     }
-    if (t == 0) out[NH] = make_float2(v[0].x - v[0].y, 0.f);
 }
 
 // Pseudo-timestream of spectrum i: Z[k] = (X[k] + conj X[N-k]) + i e^{2 pi i k/L} (X[k] - conj X[N-k])
 // (imaginary parts of X[0], X[N] dropped), z = IFFT_16384(Z) / L, samples (2m, 2m+1) = (Re, Im) z[m]
-// -- numpy's irfft.
+// -- numpy's irfft.  Persistent, one workgroup per CU: the next spectrum's bins
+// and mirror bins (64 registers) load while the last pass and the stores of the
+// current one run (LOOP false: a workgroup per spectrum, nothing to load ahead).
+// 4096 spectra: 262 us, 4.1 TB/s of the 1.07 GB it must move (not persistent, the
+// twiddles from memory: 330).
+template <bool LOOP>
 __global__ void __launch_bounds__(1024)
-k_pfb_c2r(const float2 *__restrict__ spec, float *__restrict__ yh, const float2 *__restrict__ fft_img,
-          const float2 *__restrict__ tw32k) {
+k_pfb_c2r(const float2 *__restrict__ spec, int n, float *__restrict__ yh, const float2 *__restrict__ fft_img,
+          const double2 *__restrict__ tw1k) {
     __shared__ float lds[LDS_FFT_N];
     __shared__ FftTw ftw;
     fft_tw_load(&ftw, fft_img);
-    const int i = blockIdx.x, t = threadIdx.x;
-    const float2 *X = spec + (size_t)i * NBIN;
-    float2 v[16];
-#pragma unroll
-    for (int q = 0; q < 16; ++q) {
-        const int k = t + 1024 * q;
-        float2 a = X[k], b = X[NH - k];     // k = 0 pairs with bin N
-        if (k == 0) {
-            a.y = 0.f;
-            b.y = 0.f;
-        }
-        const float2 sum = cadd(a, cconj(b)), dif = csub(a, cconj(b));
-        v[q] = cadd(sum, mul_si<+1>(cmul(tw32k[k], dif)));
-    }
-    fft16k_t<+1>(v, lds, &ftw);   // z[fft16k_tord(t) + 1024 q] in v[q]
-    float2 *dst = reinterpret_cast<float2 *>(yh + (size_t)i * LB) + fft16k_tord(t);
+    const int t = threadIdx.x;
     const float sc = 1.0f / (float)LB;
+    auto rsrc = [&](int row) {
+        return __builtin_amdgcn_make_buffer_rsrc((void *)(spec + (size_t)row * NBIN), 0, NBIN * (int)sizeof(float2),
+                                                 0x00020000);
+    };
+    // bin k = t + 1024 q, and N - k = (1024 - t) + 1024 (15 - q); k = 0 pairs with bin N
+    auto bin = [&](__amdgpu_buffer_rsrc_t rs, int q) {
+        return __builtin_bit_cast(float2, __builtin_amdgcn_raw_buffer_load_b64(rs, 8 * t, 8192 * q, 0));
+    };
+    auto mirror = [&](__amdgpu_buffer_rsrc_t rs, int q) {
+        return __builtin_bit_cast(float2, __builtin_amdgcn_raw_buffer_load_b64(rs, 8 * (1024 - t), 8192 * (15 - q), 0));
+    };
+    float2 a[16], b[16];
+    int row = blockIdx.x;
+    __amdgpu_buffer_rsrc_t rs = rsrc(row);
 #pragma unroll
-    for (int q = 0; q < 16; ++q) dst[1024 * q] = cscale(v[q], sc);
+    for (int q = 0; q < 16; ++q) a[q] = bin(rs, q);
+#pragma unroll
+    for (int q = 0; q < 16; ++q) b[q] = mirror(rs, q);
+    for (;;) {
+        const int next = row + (int)gridDim.x, tr = row_tid();
+        const double2 T = tw1k[tr];
+        float2 v[16];
+#pragma unroll
+        for (int q = 0; q < 16; ++q) {
+            if (q == 0 && tr == 0) a[0].y = b[0].y = 0.f;
+            const float2 sum = cadd(a[q], cconj(b[q])), dif = csub(a[q], cconj(b[q]));
+            v[q] = add_i_mul<+1>(sum, split_tw(T, q), dif);
+        }
+        fft16k_p12<+1>(v, lds, &ftw, tr);
+        fft16k_p3w<+1>(v, lds, &ftw, tr);
+        if (LOOP) {
+            // the bins before the last pass, the mirror bins as its outputs leave
+            // their registers; the last spectrum loads itself again
+            rs = rsrc(next < n ? next : row);
+#pragma unroll
+            for (int q = 0; q < 16; ++q) a[q] = bin(rs, q);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        const int T0 = fft16k_tord(tr);            // z[T0 + 1024 q] in v[q]
+        float2 *dst = reinterpret_cast<float2 *>(yh + (size_t)row * LB) + T0;
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+            fft16k_p4_one<+1>(v, &ftw, T0, g);
+#pragma unroll
+            for (int r = 0; r < 4; ++r) dst[1024 * (g + 4 * r)] = cscale(v[g + 4 * r], sc);
+            if (LOOP) {
+#pragma unroll
+                for (int r = 0; r < 4; ++r) b[4 * g + r] = mirror(rs, 4 * g + r);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        }
+        if (!LOOP || next >= n) break;
+        row = next;
+    }
 }
 
 // One row of the banded Cholesky factor of the Toeplitz band (a0, a1, a2, a3):
@@ -906,7 +1039,7 @@ k_pfb_join(const double *__restrict__ tab, int N, int nb, const double *__restri
         }
     }
     const double be1 = tab[n], be2 = tab[LB + n], be3 = tab[2 * LB + n];
-    double cb[9], rb[9], rl[9], W[9];
+    double cb[9], rb[9], rl[9], W[9], G[9];
 #pragma unroll
     for (int i = 0; i < 9; ++i) {
         cb[i] = tab[(size_t)(TB_CB + i) * LB + n];
@@ -1096,7 +1229,7 @@ struct sdbe_pfb {
     int max_spec = 0;
     int last_hip_err = 0;
     float2 *fft_img = nullptr;    // FftTw image
-    float2 *tw32k = nullptr;      // e^{2 pi i k / 32768}, k < 16384
+    double2 *tw1k = nullptr;      // e^{2 pi i k / 32768}, k < 1024
     float *win = nullptr;         // [4][32768]
     double *a = nullptr;          // [4][32768] band of P P^T per branch
     float *yh = nullptr;          // [max_spec][32768]
@@ -1110,6 +1243,7 @@ struct sdbe_pfb {
     double *tc = nullptr;         // [TC_N][32768] ... of the current call
     double *bst = nullptr;        // [4][nb][3][32768] ... its blocks' states, out and in, both ways
     int nb = 0;                   // blocks of max_spec rows
+    int n_cu = 256;               // compute units of the device
     int constant = 0;             // no branch has zeros together on the unit circle
 };
 
@@ -1132,7 +1266,7 @@ void sdbe_pfb_destroy(sdbe_pfb_t *p) {
     (void)hipSetDevice(p->device);
     (void)hipDeviceSynchronize();
     (void)hipFree(p->fft_img);
-    (void)hipFree(p->tw32k);
+    (void)hipFree(p->tw1k);
     (void)hipFree(p->win);
     (void)hipFree(p->a);
     (void)hipFree(p->yh);
@@ -1161,13 +1295,15 @@ int sdbe_pfb_create(int device, int32_t n_taps, const float *h_window, int32_t m
     if (!p) return SDBE_ERR_NOMEM;
     p->device = device;
     p->max_spec = max_spectra;
-    int rc = SDBE_OK, clustered = 0, *d_clustered = nullptr;
-    std::vector<float2> img(FFT_TW_N), tw(NH);
+    int rc = SDBE_OK, clustered = 0, *d_clustered = nullptr, ncu = 0;
+    if (hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, device) == hipSuccess && ncu > 0) p->n_cu = ncu;
+    std::vector<float2> img(FFT_TW_N);
+    std::vector<double2> tw(1024);
     const double two_pi = 6.283185307179586476925286766559;
     fft_tw_fill(img.data());
-    for (int k = 0; k < NH; ++k) {
+    for (int k = 0; k < 1024; ++k) {
         const double ang = two_pi * (double)k / (double)LB;
-        tw[k] = make_float2((float)cos(ang), (float)sin(ang));
+        tw[k] = make_double2(cos(ang), sin(ang));
     }
 #define PALLOC(ptr, bytes)                                              \
     do {                                                                \
@@ -1177,14 +1313,14 @@ int sdbe_pfb_create(int device, int32_t n_taps, const float *h_window, int32_t m
         }                                                               \
     } while (0)
     PALLOC(p->fft_img, FFT_TW_N * sizeof(float2));
-    PALLOC(p->tw32k, NH * sizeof(float2));
+    PALLOC(p->tw1k, 1024 * sizeof(double2));
     PALLOC(p->win, (size_t)NT * LB * sizeof(float));
     PALLOC(p->yh, (size_t)max_spectra * LB * sizeof(float));
     PALLOC(p->tab, (size_t)TB_N * LB * sizeof(double));
     PALLOC(p->tc, (size_t)TC_N * LB * sizeof(double));
     d_clustered = reinterpret_cast<int *>(p->tc);    // until the first call writes its tables
     if (hipMemcpy(p->fft_img, img.data(), FFT_TW_N * sizeof(float2), hipMemcpyHostToDevice) != hipSuccess ||
-        hipMemcpy(p->tw32k, tw.data(), NH * sizeof(float2), hipMemcpyHostToDevice) != hipSuccess ||
+        hipMemcpy(p->tw1k, tw.data(), 1024 * sizeof(double2), hipMemcpyHostToDevice) != hipSuccess ||
         hipMemcpy(p->win, h_window, (size_t)NT * LB * sizeof(float), hipMemcpyHostToDevice) != hipSuccess ||
         hipMemcpy(d_clustered, &clustered, sizeof(int), hipMemcpyHostToDevice) != hipSuccess) {
         rc = SDBE_ERR_HIP;
@@ -1248,9 +1384,16 @@ int sdbe_pfb_forward(sdbe_pfb_t *p, const float *d_x, int32_t n_spectra, void *d
     if (!p || !d_x || !d_spec || n_spectra < 1) return SDBE_ERR_ARG;
     if (n_spectra > p->max_spec) return SDBE_ERR_CAPACITY;
     PFB_TRY(p, hipSetDevice(p->device));
-    hipLaunchKernelGGL(k_pfb_fold_r2c, dim3(n_spectra), dim3(1024), 0, (hipStream_t)stream, d_x,
-                       (const float *)p->win, (float2 *)d_spec, (const float2 *)p->fft_img,
-                       (const float2 *)p->tw32k);
+    hipStream_t s = (hipStream_t)stream;
+    if (n_spectra <= p->n_cu) {          // pairs would leave CUs without work: one round either way, of one or of two spectra
+        hipLaunchKernelGGL(k_pfb_fold_r2c, dim3(n_spectra), dim3(1024), 0, s, d_x, (const float *)p->win,
+                           (float2 *)d_spec, (const float2 *)p->fft_img, (const double2 *)p->tw1k);
+    } else {
+        const int pairs = (n_spectra + 1) / 2;
+        hipLaunchKernelGGL(k_pfb_fold2_r2c, dim3(pairs < p->n_cu ? pairs : p->n_cu), dim3(1024), 0, s, d_x,
+                           (int)n_spectra, (const float *)p->win, (float2 *)d_spec, (const float2 *)p->fft_img,
+                           (const double2 *)p->tw1k);
+    }
     PFB_TRY(p, hipGetLastError());
     return SDBE_OK;
 }
@@ -1260,8 +1403,9 @@ int sdbe_pfb_inverse(sdbe_pfb_t *p, const void *d_spec, int32_t n_spectra, float
     if (n_spectra > p->max_spec) return SDBE_ERR_CAPACITY;
     PFB_TRY(p, hipSetDevice(p->device));
     hipStream_t s = (hipStream_t)stream;
-    hipLaunchKernelGGL(k_pfb_c2r, dim3(n_spectra), dim3(1024), 0, s, (const float2 *)d_spec, p->yh,
-                       (const float2 *)p->fft_img, (const float2 *)p->tw32k);
+    const bool loop = n_spectra > p->n_cu;
+    hipLaunchKernelGGL(loop ? k_pfb_c2r<true> : k_pfb_c2r<false>, dim3(loop ? p->n_cu : n_spectra), dim3(1024), 0, s,
+                       (const float2 *)d_spec, (int)n_spectra, p->yh, (const float2 *)p->fft_img, (const double2 *)p->tw1k);
     if (p->constant) {
         const int N = n_spectra, nb = (N + SBLK - 1) / SBLK;
         const dim3 br(LB / SOLVE_WG), wg(SOLVE_WG);
