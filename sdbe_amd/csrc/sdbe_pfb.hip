@@ -689,10 +689,13 @@ k_pfb_bfin(const float *__restrict__ yh, const double *__restrict__ uck, int nbl
 // block of (B B^T)^-1.  In scaled units v = b0 B^-1 y, zeta = b0^2 z:
 //   v_i = y_i - beta1 v_{i-1} - beta2 v_{i-2} - beta3 v_{i-3},
 //   zeta_i = v_i - beta1 zeta_{i+1} - beta2 zeta_{i+2} - beta3 zeta_{i+3}.
-// Rounding grows with the rows like the factor-row recurrences' does (both below
-// 1e-8 of the result for 4096 rows of the Hamming and Hann-sinc prototypes, far
-// under the FP32 rounding of yh), except where two zeros fall together on the
-// unit circle: taps 1, 2, 1 lose 5e-5 in 1000 rows here and 1e-8 by factor rows.
+// Rounding: the tables are computed in double-double and the corner takes one
+// refinement step, so the FP32 rounding of yh is all that is left in the result.
+// Against an 80-bit solve, over the 280 worst branches of a Hamming prototype
+// (double zeros near -0.995): 1.65e-7 to 1.79e-7 at 256 to 4096 rows, where the
+// FP64 factor rows are themselves off by up to 3.0e-7 (4096 rows).  The exception is
+// two zeros together on the unit circle: taps 1, 2, 1 lose 5e-5 in 1000 rows here
+// and 1e-8 by factor rows.
 // k_pfb_spectral counts such branches, and a plan that has any takes those.
 //
 // Thread (branch, span of 32 rows) keeps its rows' v in registers; a workgroup
@@ -702,7 +705,7 @@ k_pfb_bfin(const float *__restrict__ yh, const double *__restrict__ uck, int nbl
 // one read of yh, k_pfb_join composes them per branch into the blocks' true
 // incoming states with the corner, and k_pfb_solve finishes the blocks: two
 // reads of yh and one write of x, all in 256-byte runs.  4096 spectra: span 130 us
-// (4.1 TB/s), join 22, solve 225 (4.8 TB/s, the rate of a large copy); the
+// (4.1 TB/s), join 27, solve 225 (4.8 TB/s, the rate of a large copy); the
 // factor-row kernels, which read yh four times beside 0.8 GB of checkpoints and
 // recompute every factor row four times, take 890.  (Tiles of 8 branches over
 // all 4096 rows read yh once, but in 32-byte runs: 700 us.)
@@ -716,7 +719,8 @@ constexpr int TB_RS = 25;                 // a span's head zeta per unit incomin
 constexpr int TB_HS = 34;                 // its impulse response h27..h31
 constexpr int TB_RB = 39;                 // the same of a block: head zeta
 constexpr int TB_HB = 48;                 // ... h251..h255
-constexpr int TB_N = 53;
+constexpr int TB_GB = 53;                 // ... first 3 x 3 block of (B B^T)^-1
+constexpr int TB_N = 62;
 // ... and of a call
 constexpr int TC_W = 0;                   // corner matrix W (scaled)
 constexpr int TC_RS = 9;                  // TB_RS of the partial last span
@@ -730,6 +734,25 @@ __device__ __forceinline__ void mat_mul(double (&o)[9], const double (&a)[9], co
 #pragma unroll
         for (int c = 0; c < 3; ++c) o[3 * r + c] = a[3 * r] * b[c] + a[3 * r + 1] * b[3 + c] + a[3 * r + 2] * b[6 + c];
 }
+
+// Double-double: h + l, |l| at most half an ulp of h.
+struct Dd {
+    double h = 0.0, l = 0.0;
+};
+__device__ __forceinline__ Dd dd_norm(double h, double l) {
+    const double s = h + l;
+    return Dd{s, l - (s - h)};
+}
+__device__ __forceinline__ Dd dd_add(Dd a, Dd b) {
+    const double s = a.h + b.h, t = s - a.h;
+    return dd_norm(s, (a.h - (s - t)) + (b.h - t) + (a.l + b.l));
+}
+__device__ __forceinline__ Dd dd_mul(Dd a, Dd b) {
+    const double p = a.h * b.h;
+    return dd_norm(p, fma(a.h, b.h, -p) + fma(a.h, b.l, a.l * b.h));
+}
+// a - b c
+__device__ __forceinline__ Dd dd_sub_mul(Dd a, Dd b, double c) { return dd_add(a, dd_mul(b, Dd{-c, 0.0})); }
 
 // sum_{k < n} C^k X (C^k)^T (TR) or sum_{k < n} C^k X C^k, by doubling over the
 // bits of n.
@@ -840,18 +863,21 @@ k_pfb_spectral(const float *__restrict__ win, double *__restrict__ tab, int *__r
         };
         auto inside = [](double x) { return fabs(x) > 1.0 ? 1.0 / x : x; };
         times(r);
+        bool any = fabs(r) > 1.0;              // a zero was reflected
         const double disc = d1 * d1 - 4.0 * d0, ri = inside(r);
         constexpr double NEAR = 0.998, GAP = 0.02;
         if (disc >= 0.0) {
             const double s = -0.5 * (d1 + copysign(sqrt(disc), d1)), x2 = s != 0.0 ? d0 / s : 0.0;
             times(s);
             times(x2);
+            any = any || fabs(s) > 1.0 || fabs(x2) > 1.0;
             const double si = inside(s), xi = inside(x2);
             close = (fmin(fabs(ri), fabs(si)) > NEAR && fabs(ri - si) < GAP) ||
                     (fmin(fabs(ri), fabs(xi)) > NEAR && fabs(ri - xi) < GAP) ||
                     (fmin(fabs(si), fabs(xi)) > NEAR && fabs(si - xi) < GAP);
         } else {
             const bool out = d0 > 1.0;
+            any = any || out;
             const double e0 = out ? d0 : 1.0, e2 = out ? 1.0 : d0;
             const double p0 = pol[0], p1 = pol[1];
             pol[0] = p0 * e0;
@@ -861,8 +887,9 @@ k_pfb_spectral(const float *__restrict__ win, double *__restrict__ tab, int *__r
             const double re = -0.5 * d1 / e0, im = 0.5 * sqrt(-disc) / e0, mod = sqrt(fmin(d0, 1.0 / d0));
             close = mod > NEAR && (2.0 * im < GAP || (fabs(ri) > NEAR && hypot(ri - re, im) < GAP));
         }
+        // taps that are minimum phase already (in either order) are the factor, exactly
 #pragma unroll
-        for (int i = 0; i < 4; ++i) b[i] = pol[i];
+        for (int i = 0; i < 4; ++i) b[i] = any ? pol[i] : c[i];
     }
     if (close) atomicAdd(clustered, 1);
     const double be1 = b[1] / b[0], be2 = b[2] / b[0], be3 = b[3] / b[0], b0 = b[0] * sc;
@@ -872,38 +899,55 @@ k_pfb_spectral(const float *__restrict__ win, double *__restrict__ tab, int *__r
     o[(size_t)(TB_BETA + 2) * LB] = be3;
 #pragma unroll
     for (int i = 0; i < 4; ++i) o[(size_t)(TB_WZ + i) * LB] = w[i] / b0 / b0;
-    double m[9] = {-be1, -be2, -be3, 1.0, 0.0, 0.0, 0.0, 1.0, 0.0};
-    for (int k = 1; k <= 8; ++k) {          // C^2, C^4, .. C^256
-        double q[9];
-        mat_mul(q, m, m);
+    // The span's and the block's responses, by recursion over their rows in
+    // double-double: near-double zeros close to the unit circle (the Hamming
+    // prototype has some around branches 4050 and 28720) amplify the tables'
+    // rounding into the result, 3e-7 of it with powers by squaring in FP64.
+    Dd v[3][3] = {{{1.0, 0.0}, {}, {}}, {{}, {1.0, 0.0}, {}}, {{}, {}, {1.0, 0.0}}};   // chain c: its last three values
+    Dd h[3] = {}, rm[9] = {}, g[6] = {};
+    for (int k = 0; k < SBLK; ++k) {
+        const Dd in{k == 0 ? 1.0 : 0.0, 0.0};
+        const Dd hk = dd_sub_mul(dd_sub_mul(dd_sub_mul(in, h[0], be1), h[1], be2), h[2], be3);
+        h[2] = h[1];
+        h[1] = h[0];
+        h[0] = hk;
 #pragma unroll
-        for (int i = 0; i < 9; ++i) m[i] = q[i];
-        if (k == 5 || k == 8)
+        for (int c = 0; c < 3; ++c) {
+            const Dd x = dd_sub_mul(dd_sub_mul(dd_sub_mul(Dd{}, v[c][0], be1), v[c][1], be2), v[c][2], be3);
+            v[c][2] = v[c][1];
+            v[c][1] = v[c][0];
+            v[c][0] = x;
 #pragma unroll
-            for (int i = 0; i < 9; ++i) o[(size_t)((k == 5 ? TB_CS : TB_CB) + i) * LB] = m[i];
-    }
-    for (int v = 0; v < 2; ++v) {
-        const int rows = v ? SBLK : SR;
-        double rm[9];
-        head_response(rows, be1, be2, be3, rm);
+            for (int r = 0; r < 3; ++r) rm[3 * r + c] = dd_add(rm[3 * r + c], dd_mul(x, h[r]));
+        }
 #pragma unroll
-        for (int i = 0; i < 9; ++i) o[(size_t)((v ? TB_RB : TB_RS) + i) * LB] = rm[i];
-        double h1 = 0.0, h2 = 0.0, h3 = 0.0;
-        for (int k = 0; k < rows; ++k) {
-            const double h = (k == 0 ? 1.0 : 0.0) - be1 * h1 - be2 * h2 - be3 * h3;
-            if (k >= rows - 5) o[(size_t)((v ? TB_HB : TB_HS) + k - (rows - 5)) * LB] = h;
-            h3 = h2;
-            h2 = h1;
-            h1 = h;
+        for (int r = 0, i = 0; r < 3; ++r)
+#pragma unroll
+            for (int c = r; c < 3; ++c, ++i) g[i] = dd_add(g[i], dd_mul(h[r], h[c]));
+        if (k < SR && k >= SR - 5) o[(size_t)(TB_HS + k - (SR - 5)) * LB] = hk.h;
+        if (k >= SBLK - 5) o[(size_t)(TB_HB + k - (SBLK - 5)) * LB] = hk.h;
+        if (k == SR - 1 || k == SBLK - 1) {
+            const int cr = k == SR - 1 ? TB_CS : TB_CB, rr = k == SR - 1 ? TB_RS : TB_RB;
+#pragma unroll
+            for (int r = 0; r < 3; ++r)
+#pragma unroll
+                for (int c = 0; c < 3; ++c) {
+                    o[(size_t)(cr + 3 * r + c) * LB] = v[c][r].h;
+                    o[(size_t)(rr + 3 * r + c) * LB] = rm[3 * r + c].h;
+                }
         }
     }
+#pragma unroll
+    for (int r = 0, i = 0; r < 3; ++r)
+#pragma unroll
+        for (int c = r; c < 3; ++c, ++i) o[(size_t)(TB_GB + 3 * r + c) * LB] = o[(size_t)(TB_GB + 3 * c + r) * LB] = g[i].h;
 }
 
-// The corner matrix W of N rows.  G = sum_{i < N} s_i s_i^T with s_i = C^i e_0.
-__device__ __forceinline__ void corner(int N, double be1, double be2, double be3, double (&W)[9]) {
+// The corner matrix W of N rows, and G = sum_{i < N} s_i s_i^T with s_i = C^i e_0.
+__device__ __forceinline__ void corner(int N, double be1, double be2, double be3, double (&W)[9], double (&G)[9]) {
     const double C[9] = {-be1, -be2, -be3, 1.0, 0.0, 0.0, 0.0, 1.0, 0.0};
     const double X[9] = {1.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
-    double G[9], t[9];
+    double t[9];
     power_sum<true>(N, C, X, G);
     // H (scaled by 1 / b0), rows past N zero
     const double H[9] = {be1, be2, be3, N > 1 ? be2 : 0.0, N > 1 ? be3 : 0.0, 0.0, N > 2 ? be3 : 0.0, 0.0, 0.0};
@@ -935,8 +979,8 @@ __global__ void __launch_bounds__(SOLVE_WG)
 k_pfb_corner(const double *__restrict__ tab, int N, double *__restrict__ tc) {
     const int n = blockIdx.x * SOLVE_WG + threadIdx.x;
     const double be1 = tab[n], be2 = tab[LB + n], be3 = tab[2 * LB + n];
-    double W[9], rm[9];
-    corner(N, be1, be2, be3, W);
+    double W[9], G[9], rm[9];
+    corner(N, be1, be2, be3, W, G);
     head_response(N & (SR - 1), be1, be2, be3, rm);
 #pragma unroll
     for (int i = 0; i < 9; ++i) {
@@ -1049,7 +1093,7 @@ k_pfb_join(const double *__restrict__ tab, int N, int nb, const double *__restri
 #pragma unroll
     for (int i = 0; i < 9; ++i) tc[(size_t)(TC_RS + i) * LB + n] = rl[i];
     head_response((N - 1) % SBLK + 1, be1, be2, be3, rl);     // the last block's
-    corner(N, be1, be2, be3, W);
+    corner(N, be1, be2, be3, W, G);
     const V3 zero{0.0, 0.0, 0.0};
     V3 a = zero;
     for (int k = 0; k < nb; ++k) {
@@ -1060,19 +1104,43 @@ k_pfb_join(const double *__restrict__ tab, int N, int nb, const double *__restri
     }
     V3 z = zero;                                               // zeta at the head of block k
     for (int k = nb - 1; k >= 0; --k) z = mv_add<1>(get(1, k), cb, z);
-    const V3 g = mv_add<1>(zero, W, z);
-    v3_store(tc + (size_t)TC_G * LB, n, g);
     const double *h = tab + (size_t)TB_HB * LB + n;
     const double h0 = h[0], h1 = h[LB], h2 = h[2 * LB], h3 = h[3 * LB], h4 = h[4 * LB];
-    // state after the first block from -g on its first three rows
-    V3 d{-(g.a * h4 + g.b * h3 + g.c * h2), -(g.a * h3 + g.b * h2 + g.c * h1), -(g.a * h2 + g.b * h1 + g.c * h0)};
-    v3_store(A, n, zero);
-    for (int k = 1; k < nb; ++k) {
-        const V3 p = get(0, k), q = get(1, k);
-        v3_store(A + B3 * k, n, V3{p.a + d.a, p.b + d.b, p.c + d.c});
-        put(1, k, k == nb - 1 ? mv_add<1>(q, rl, d) : mv_add<1>(q, rb, d));
-        d = mv_add<1>(zero, cb, d);
+    // -dg on the first three rows: the states it leaves after the first block, and on
+    auto correct = [&](V3 dg) {
+        V3 d{-(dg.a * h4 + dg.b * h3 + dg.c * h2), -(dg.a * h3 + dg.b * h2 + dg.c * h1),
+             -(dg.a * h2 + dg.b * h1 + dg.c * h0)};
+        for (int k = 1; k < nb; ++k) {
+            const V3 p = get(0, k), q = get(1, k);
+            put(0, k, V3{p.a + d.a, p.b + d.b, p.c + d.c});
+            put(1, k, k == nb - 1 ? mv_add<1>(q, rl, d) : mv_add<1>(q, rb, d));
+            d = mv_add<1>(zero, cb, d);
+        }
+    };
+    V3 g = mv_add<1>(zero, W, z);
+    correct(g);
+    // One step of refinement: W comes from a Gram matrix, whose condition is that
+    // of the corner squared.  With the head zeta of the corrected solution, g must
+    // be H H^T zeta; the residual r is corrected by (I + H H^T G)^-1 r = r - W G r.
+    z = zero;
+    for (int k = nb - 1; k > 0; --k) z = mv_add<1>(get(1, k), cb, z);
+    {
+        const double *gb = tab + (size_t)TB_GB * LB + n;
+        V3 q = get(1, 0);
+        q = V3{q.a - (gb[0] * g.a + gb[LB] * g.b + gb[2 * LB] * g.c),
+               q.b - (gb[3 * LB] * g.a + gb[4 * LB] * g.b + gb[5 * LB] * g.c),
+               q.c - (gb[6 * LB] * g.a + gb[7 * LB] * g.b + gb[8 * LB] * g.c)};
+        z = mv_add<1>(q, cb, z);
+        const double H[9] = {be1, be2, be3, be2, be3, 0.0, be3, 0.0, 0.0};          // symmetric
+        const V3 r = mv_add<1>(V3{-g.a, -g.b, -g.c}, H, mv_add<1>(zero, H, z));
+        const V3 wgr = mv_add<1>(zero, W, mv_add<1>(zero, G, r));
+        const V3 dg{r.a - wgr.a, r.b - wgr.b, r.c - wgr.c};
+        correct(dg);
+        g = V3{g.a + dg.a, g.b + dg.b, g.c + dg.c};
     }
+    v3_store(tc + (size_t)TC_G * LB, n, g);
+    if (IN_LDS)
+        for (int k = 0; k < nb; ++k) v3_store(A + B3 * k, n, get(0, k));
     V3 b = zero;
     for (int k = nb - 1; k >= 0; --k) {
         v3_store(B + B3 * k, n, b);
