@@ -1865,6 +1865,7 @@ int run_trim(sdbe_handle_t *h, const BpDesc *d_bpd, int n_bp, const OutDesc &od,
     const auto kc2r_pk = h->geom == SDBE_GEOM_8X1024 ? k_trim_c2r_pk<D, true> : k_trim_c2r_pk<D, false>;
     const auto kseg_f = k_trim_seg<D, E, true>;
     const auto kseg_c = k_trim_seg<D, E, false>;
+    int *packed = reinterpret_cast<int *>(h->stage);     // a flag per block-pol, in the 64/39 path's code buffer
     for (int bp0 = 0; bp0 < n_bp; bp0 += h->chunk) {
         const int nb = (n_bp - bp0) < h->chunk ? (n_bp - bp0) : h->chunk;
         const BpDesc *bpd = d_bpd + bp0;
@@ -1876,11 +1877,11 @@ int run_trim(sdbe_handle_t *h, const BpDesc *d_bpd, int n_bp, const OutDesc &od,
         if (f32)
             LAUNCH(h, KID_TRIM_SEG, nb, s, kseg_f, dim3(trim::NSEG * nb), dim3(trim::seg_threads(D)),
                    (const float *)h->V, bpd, (float *)h->Zf, h->part, h->trim_tabs, h->trim.skip,
-                   (const float2 *)h->tb.fft);
+                   (const float2 *)h->tb.fft, (const float *)h->latch, packed, od);
         else
             LAUNCH(h, KID_TRIM_SEG, nb, s, kseg_c, dim3(trim::NSEG * nb), dim3(trim::seg_threads(D)),
                    (const float *)h->V, bpd, (float *)h->Zf, h->part, h->trim_tabs, h->trim.skip,
-                   (const float2 *)h->tb.fft);
+                   (const float2 *)h->tb.fft, (const float *)h->latch, packed, od);
         // the counters and latch go to the host with the call's last kernel
         const Mirror none{nullptr, nullptr}, mir = bp0 + nb == n_bp ? Mirror{h->cnt, h->h_cnt} : none;
         LAUNCH(h, KID_STATS, nb, s, k_trim_stats, dim3(nb), dim3(trim::NSEG), (const double *)h->part, P, bp0, h->ms,
@@ -1889,7 +1890,7 @@ int run_trim(sdbe_handle_t *h, const BpDesc *d_bpd, int n_bp, const OutDesc &od,
             LAUNCH(h, KID_THRESH, nb, s, k_thresh, dim3(1), dim3(256), (const double2 *)h->ms, nb, bpd, h->latch,
                    h->thr);
             LAUNCH(h, KID_TRIM_PACK, nb, s, k_trim_pack, dim3(nb * (trim::NSEG * P / 16 / 256)), dim3(256),
-                   (const float *)h->Zf, (const float2 *)h->thr, bpd, P, od, mir);
+                   (const float *)h->Zf, (const float2 *)h->thr, bpd, P, (const int *)packed, od, mir);
         }
         HIP_TRY(h, hipGetLastError());
     }

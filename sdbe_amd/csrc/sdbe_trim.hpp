@@ -422,6 +422,51 @@ __device__ __forceinline__ void c2r_inputs(const Tw2 &n32k, float2 (&v)[16], Val
     }
 }
 
+// The threshold and offset a block's codes take, where they do not depend on the
+// block's own samples: FIXED, and REFERENCE once its slot has latched.
+__device__ __forceinline__ bool known_threshold(const BpDesc &d, const float *__restrict__ latch, float2 &to) {
+    if (d.policy == SDBE_THRESH_REFERENCE) {
+        to = make_float2(latch[2 * d.slot], latch[2 * d.slot + 1]);
+        return !(to.x == 0.0f);
+    }
+    to = make_float2(d.fixed_th, d.fixed_off);
+    return d.policy == SDBE_THRESH_FIXED;
+}
+
+// 2-bit code of a sample: v = x - off; ((|v| >= th) | 2) ^ 3 (v < 0)
+// (vdif_inout_gpu_thread.cu:565-583), shifted up by the position of `one` = 1 << shift.
+// The difference is rounded by itself wherever x comes from.
+__device__ __forceinline__ uint32_t code2(float x, float2 to, uint32_t one) {
+#pragma clang fp contract(off)
+    const float v = x - to.y;
+    return (fabsf(v) >= to.x ? 3u * one : 2u * one) ^ (v < 0.f ? 3u * one : 0u);
+}
+
+// Codes of a segment straight from the registers of its last pass: x(q), q < JT, is
+// the pair of samples of element m0 + STEP q (m0 = the thread's, whose low three
+// bits are those of t).  8 elements are a word; its lanes OR their nibbles, and of
+// 8 consecutive q lane r keeps and stores that of q = r.
+template <int JT, int STEP, typename X>
+__device__ __forceinline__ void store_codes(uint8_t *dst, int m0, float2 to, X x) {
+    static_assert(JT % 8 == 0 && STEP % 8 == 0, "whole words");
+    const uint32_t r = m0 & 7, one = 1u << (4 * r);
+    uint32_t *w = reinterpret_cast<uint32_t *>(dst) + (m0 >> 3) + (STEP / 8) * r;
+#pragma unroll
+    for (int h = 0; h < JT; h += 8) {
+        uint32_t keep = 0;
+#pragma unroll
+        for (int q = 0; q < 8; ++q) {
+            const float2 v = x(h + q);
+            int c = (int)(code2(v.x, to, one) | code2(v.y, to, 4u * one));
+            c |= __builtin_amdgcn_mov_dpp(c, 0xB1, 0xF, 0xF, true);      // lanes ^ 1
+            c |= __builtin_amdgcn_mov_dpp(c, 0x4E, 0xF, 0xF, true);      // lanes ^ 2
+            c |= __builtin_amdgcn_mov_dpp(c, 0x141, 0xF, 0xF, true);     // the other four of 8
+            keep = r == (uint32_t)q ? (uint32_t)c : keep;
+        }
+        w[(STEP / 8) * h] = keep;
+    }
+}
+
 }  // namespace trim
 
 // SwarmC2R of one snapshot (workgroup = snapshot s of block bpl, 1024 threads):
@@ -580,7 +625,8 @@ k_trim_c2r_pk(const BpDesc *__restrict__ bpd, float2 *__restrict__ T, Tables tb,
 template <int D, int E, bool F32>
 __global__ void __launch_bounds__(trim::seg_threads(D))
 k_trim_seg(const float *__restrict__ T, const BpDesc *__restrict__ bpd, float *__restrict__ stage,
-           double *__restrict__ part, trim::Tabs tt, int skip, const float2 *__restrict__ fft_tw) {
+           double *__restrict__ part, trim::Tabs tt, int skip, const float2 *__restrict__ fft_tw,
+           const float *__restrict__ latch, int *__restrict__ packed, OutDesc od) {
     constexpr int R = 256 * D, P = 256 * E, NR = R / 2, NP = P / 2;
     constexpr int NBUF = NR > NP ? NR : NP;
     constexpr int NT = trim::seg_threads(D);
@@ -598,6 +644,13 @@ k_trim_seg(const float *__restrict__ T, const BpDesc *__restrict__ bpd, float *_
         ftwp = &ftw;
     }
     const int bpl = blockIdx.x / trim::NSEG, g = blockIdx.x - bpl * trim::NSEG, t = threadIdx.x;
+    // With a known threshold the samples leave as codes and not as floats: 1/16 of
+    // the stores, and k_trim_pack has nothing to do for the block.  256 block-pols
+    // at 6/11, segments and packing: 806 + 5 us, as floats 800 + 217; at 11/11 3895 +
+    // 10 and 3965 + 833.  (Decided here, ahead of the transforms: a branch between
+    // them splits the schedule and takes 130 registers more.)
+    float2 to;
+    const bool codes = !F32 && trim::known_threshold(bpd[bpl], latch, to);
     const float2 *z = reinterpret_cast<const float2 *>(T + (size_t)bpl * D * 2 * NCH + (size_t)g * R);
     trim::pass1_global<NR, -1, NT>(buf, z);   // the input goes to registers, not through LDS
     trim::fft_tail<NR, -1, NT>(buf, tt.zr);   // Z in natural order, plain layout
@@ -648,6 +701,9 @@ k_trim_seg(const float *__restrict__ T, const BpDesc *__restrict__ bpd, float *_
     const float sc = 1.0f / (65536.0f * (float)P);
     float2 *dst = reinterpret_cast<float2 *>((F32 ? (float *)bpd[bpl].out : stage + (size_t)bpl * trim::NSEG * P) +
                                              (size_t)g * P);
+    uint8_t *cdst = bpd[bpl].out + (size_t)(g * (P / 4) / OUT_FRAME_PAYLOAD) * od.frame_bytes + od.hdr_bytes +
+                    g * (P / 4) % OUT_FRAME_PAYLOAD;
+    static_assert(OUT_FRAME_PAYLOAD % (P / 4) == 0, "a segment's codes are in one frame");
     // the segment's sums of x and x^2: FP32 over the thread's 2 JT samples,
     // then FP64 across threads and segments
     float s1f = 0.f, s2f = 0.f;
@@ -655,13 +711,18 @@ k_trim_seg(const float *__restrict__ T, const BpDesc *__restrict__ bpd, float *_
         // wv[q] is element t + 1024 q, fft16k_t's input layout; it waits at its
         // first barrier until every read of Z is done
         fft16k_t<+1>(wv, reinterpret_cast<float *>(buf), ftwp);   // element fft16k_tord(t) + 1024 q in wv[q]
-        float2 *d = dst + fft16k_tord(t);
-#pragma unroll
-        for (int q = 0; q < JT; ++q) {
+        const int m0 = fft16k_tord(t);
+        auto sample = [&](int q) {
             const float2 x = cscale(wv[q], sc);
-            d[1024 * q] = x;
             s1f += x.x + x.y;
             s2f = fmaf(x.x, x.x, fmaf(x.y, x.y, s2f));
+            return x;
+        };
+        if (codes) {
+            trim::store_codes<JT, 1024>(cdst, m0, to, sample);
+        } else {
+#pragma unroll
+            for (int q = 0; q < JT; ++q) dst[m0 + 1024 * q] = sample(q);
         }
     } else {
         if constexpr (NP / 16 == NT) {
@@ -685,12 +746,18 @@ k_trim_seg(const float *__restrict__ T, const BpDesc *__restrict__ bpd, float *_
         trim::pass_to_regs<NP, LR, LNS, +1, NT>(buf, tt.zp, o);
         const __amdgpu_buffer_rsrc_t rd =
             __builtin_amdgcn_make_buffer_rsrc((void *)dst, 0, NP * (int)sizeof(float2), BUF_RSRC_WORD3);
-#pragma unroll
-        for (int q = 0; q < JT; ++q) {
+        auto sample = [&](int q) {
             const float2 x = cscale(o[q % QS][q / QS], sc);
-            __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32v2, x), rd, 8 * t, 8 * NT * q, 0);
             s1f += x.x + x.y;
             s2f = fmaf(x.x, x.x, fmaf(x.y, x.y, s2f));
+            return x;
+        };
+        if (codes) {
+            trim::store_codes<JT, NT>(cdst, t, to, sample);
+        } else {
+#pragma unroll
+            for (int q = 0; q < JT; ++q)
+                __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32v2, sample(q)), rd, 8 * t, 8 * NT * q, 0);
         }
     }
     double s1 = (double)s1f, s2 = (double)s2f;
@@ -705,6 +772,7 @@ k_trim_seg(const float *__restrict__ T, const BpDesc *__restrict__ bpd, float *_
     }
     __syncthreads();
     if (t == 0) {
+        if (!F32 && g == 0) packed[bpl] = codes;
         double a = 0.0, b = 0.0;
         for (int i = 0; i < NT / 64; ++i) {
             a += red[0][i];
@@ -746,31 +814,36 @@ k_trim_stats(const double *__restrict__ part, int P, int bp0, double2 *__restric
     }
 }
 
-// 2-bit codes of block bpl in natural sample order (vdif_inout_gpu_thread.cu:565-583:
-// v = x - off; ((|v| >= th) | 2) ^ 3 (v < 0); sample i of a word at bits 2i),
-// stream byte q to frame q / 8192 of the block's output.  Thread = one 32-bit word.
+// 2-bit codes of block bpl in natural sample order (sample i of a word at bits 2i),
+// stream byte q to frame q / 8192 of the block's output, unless k_trim_seg stored
+// them.  Bound by its reads, 64 bytes a word (256 block-pols at 6/11: 219 us, 4.9
+// TB/s): a wave reads 4 KB in four coalesced loads of 16 bytes a lane, each lane's
+// four codes are a byte of a word of its four lanes, and of four lanes lane i
+// stores the word of load i.  One such piece a wave; with 2 to 8 a launch that finds
+// the codes stored is shorter (256 block-pols at 11/11: 45 and 10 us), but one that
+// does not takes 15 to 50 us more.
 __global__ void __launch_bounds__(256)
 k_trim_pack(const float *__restrict__ stage, const float2 *__restrict__ thr, const BpDesc *__restrict__ bpd, int P,
-            OutDesc od, Mirror mir) {
+            const int *__restrict__ packed, OutDesc od, Mirror mir) {
     mirror_out(mir);
-    const int words = trim::NSEG * P / 16;
-    const int wpb = words / 256;                      // workgroups per block
-    const int bpl = blockIdx.x / wpb, wi = (blockIdx.x - bpl * wpb) * 256 + threadIdx.x;
-    const float4 *src = reinterpret_cast<const float4 *>(stage + (size_t)bpl * trim::NSEG * P) + (size_t)wi * 4;
+    const int wpb = trim::NSEG * P / 16 / 256;                                   // workgroups per block
+    const int bpl = blockIdx.x / wpb, l = threadIdx.x & 63;
+    if (packed[bpl]) return;
     const float2 to = thr[bpl];
+    const int w0 = (blockIdx.x - bpl * wpb) * 256 + 64 * (threadIdx.x >> 6);     // the wave's first word
+    const float4 *src = reinterpret_cast<const float4 *>(stage + (size_t)bpl * trim::NSEG * P) + (size_t)w0 * 4 + l;
+    const uint32_t one = 1u << (8 * (l & 3));
     uint32_t word = 0;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-        const float4 f = src[i];
-        const float x[4] = {f.x, f.y, f.z, f.w};
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const float v = x[j] - to.y;
-            const uint32_t c = ((((fabsf(v) >= to.x) ? 1u : 0u) | 2u) ^ (v < 0.f ? 3u : 0u)) & 3u;
-            word |= c << (2 * (4 * i + j));
-        }
+        const float4 f = src[64 * i];
+        int c = (int)(trim::code2(f.x, to, one) | trim::code2(f.y, to, 4 * one) | trim::code2(f.z, to, 16 * one) |
+                      trim::code2(f.w, to, 64 * one));
+        c |= __builtin_amdgcn_mov_dpp(c, 0xB1, 0xF, 0xF, true);      // lanes ^ 1
+        c |= __builtin_amdgcn_mov_dpp(c, 0x4E, 0xF, 0xF, true);      // lanes ^ 2
+        word = (l & 3) == i ? (uint32_t)c : word;
     }
-    const int64_t q = (int64_t)wi * 4;
+    const int64_t q = (int64_t)(w0 + 16 * (l & 3) + (l >> 2)) * 4;
     uint8_t *dst = bpd[bpl].out + (q / OUT_FRAME_PAYLOAD) * od.frame_bytes + od.hdr_bytes + (q % OUT_FRAME_PAYLOAD);
     *reinterpret_cast<uint32_t *>(dst) = word;
 }
