@@ -612,6 +612,20 @@ k_group_bitmap(const int *__restrict__ map, uint8_t *__restrict__ bitmap, int *_
 }
 
 
+// Work item lin (of `per` in each of nb block-pols) of a kernel that runs its
+// block-pols in the opposite order to the kernel before it, whose last output is
+// then still in the memory-side cache (256 MB): block-pol and item.  Stages A and C1
+// go forward over a contiguous range of block-pols per XCD (xcd_contig), stages B
+// and C2 backward over the same ranges (xcd_map: nb and the grid are multiples of 8;
+// workgroups are dealt round-robin over the 8 XCDs).  All in one order: 33
+// block-pols 524 us (now 509), 64: 718 (708), 256: 2551 (2541).
+__device__ __forceinline__ int back_bp(int lin, int per, int nb, int xcd_map, int &item) {
+    lin = __builtin_amdgcn_readfirstlane(lin);
+    const int slot = xcd_map ? lin >> 3 : lin, n = xcd_map ? nb >> 3 : nb, b = slot / per;
+    item = slot - b * per;
+    return (xcd_map ? (lin & 7) * n : 0) + n - 1 - b;
+}
+
 // Stage B: row k1 of block-pol bpl: w = IFFT16384(V[k1]); w[n] *= e^{-2 pi i n k1/638976};
 // Zf[k1 + 39 k2] = FFT16384(w)[k2]   (packed forward DFT of the 1,277,952 samples)
 // for k1 = 1..38 (stage A writes row 0, whose transforms cancel).
@@ -619,21 +633,14 @@ k_group_bitmap(const int *__restrict__ map, uint8_t *__restrict__ bitmap, int *_
 // P = 0: FP32 VALU FFTs; P = FftMode: radix-16 passes on the matrix cores
 // (fft16k_mfma).
 // The workgroups are persistent (one per CU: the FFT's LDS fills a CU) and take
-// row slots lin = blockIdx.x, blockIdx.x + gridDim.x, ...  With xcd_map the
-// 38 rows of a block-pol all run on one XCD (workgroups are dealt round-robin
-// over the 8 XCDs; requires the chunk and the grid to be multiples of 8).  The
+// row slots lin = blockIdx.x, blockIdx.x + gridDim.x, ... (back_bp: with xcd_map the
+// 38 rows of a block-pol all run on one XCD).  The
 // next row is loaded (buffer loads, no VALU address arithmetic) while the last
 // pass, the conjugation and the stores of the current row run.
 constexpr int B_ROWS = NBLK - 1;   // rows k1 = 1..38 of a block-pol
-__device__ __forceinline__ void b_row(int lin, int xcd_map, int &bpl, int &k1) {
-    if (xcd_map) {
-        const int slot = lin >> 3;
-        bpl = (lin & 7) + 8 * (slot / B_ROWS);
-        k1 = 1 + slot % B_ROWS;
-    } else {
-        bpl = lin / B_ROWS;
-        k1 = 1 + lin % B_ROWS;
-    }
+__device__ __forceinline__ void b_row(int lin, int xcd_map, int nb, int &bpl, int &k1) {
+    bpl = back_bp(lin, B_ROWS, nb, xcd_map, k1);
+    k1 += 1;
 }
 
 __device__ __forceinline__ void b_load(const float2 *__restrict__ V, int bpl, int k1, float2 (&x)[16]) {
@@ -649,28 +656,20 @@ __device__ __forceinline__ void b_load(const float2 *__restrict__ V, int bpl, in
 
 template <int P>
 __global__ void __launch_bounds__(1024)
-k_stage_b(const float2 *__restrict__ V, float2 *__restrict__ Zf, Tables tb, int xcd_map, int n_rows) {
+k_stage_b(const float2 *__restrict__ V, float2 *__restrict__ Zf, Tables tb, int xcd_map, int nb) {
+    const int n_rows = B_ROWS * nb;
     __shared__ float lds[LDS_FFT_N];
     __shared__ FftTw ftw;
     fft_tw_load(&ftw, tb.fft);
     int lin = blockIdx.x;
     float2 nx[16];
-    if constexpr (P == 0) {
-        int bpl, k1;
-        b_row(lin, xcd_map, bpl, k1);
-        b_load(V, bpl, k1, nx);
-    }
+    int bpl, k1;      // in scalar registers: the row twiddles below are scalar loads
+    b_row(lin, xcd_map, nb, bpl, k1);
+    if constexpr (P == 0) b_load(V, bpl, k1, nx);
     for (;;) {
-        int k1, bpl;
-        b_row(lin, xcd_map, bpl, k1);
-        // workgroup-uniform: the row twiddles below are scalar loads
-        k1 = __builtin_amdgcn_readfirstlane(k1);
-        bpl = __builtin_amdgcn_readfirstlane(bpl);
         const int next = lin + (int)gridDim.x;
         int nbpl, nk1;
-        b_row(next < n_rows ? next : lin, xcd_map, nbpl, nk1);
-        nbpl = __builtin_amdgcn_readfirstlane(nbpl);
-        nk1 = __builtin_amdgcn_readfirstlane(nk1);
+        b_row(next < n_rows ? next : lin, xcd_map, nb, nbpl, nk1);
         const int t = row_tid();
         float2 v[16];
         if constexpr (P == 0) {
@@ -744,6 +743,8 @@ k_stage_b(const float2 *__restrict__ V, float2 *__restrict__ Zf, Tables tb, int 
         for (int q = 0; q < 16; ++q) dst[1024 * q] = v[q];
         if (next >= n_rows) break;
         lin = next;
+        bpl = nbpl;
+        k1 = nk1;
     }
 }
 
@@ -1163,7 +1164,7 @@ struct OutDesc {
 // the 4-bit pair code (re | im << 2) of t goes to the low nibble of
 // stage[bp][tx / 2][ty] for even tx, the high nibble for odd tx.
 // The workgroups are persistent (one per CU: the FFT's LDS fills a CU) and take
-// the rows of pairs blockIdx.x, blockIdx.x + gridDim.x, ... in turn (pair i =
+// the rows of pairs blockIdx.x, blockIdx.x + gridDim.x, ... in turn (back_bp; a pair is
 // rows 2i, 2i + 1, so that a byte's two nibbles are stored once, by the odd
 // row's pass; SINGLE: the rows one by one, each with a byte per ty of its own).  A row arrives in stage C1's
 // tile-major slot order (planar: real plane then imaginary plane) and is
@@ -1200,7 +1201,8 @@ __device__ __forceinline__ void c2_load(const float *__restrict__ Bc, int row, f
 
 template <bool F32, int P, bool SINGLE>
 __global__ void __launch_bounds__(1024)
-k_stage_c2(float *Bc, const float2 *__restrict__ thr, uint8_t *__restrict__ stage, const int *__restrict__ slot_col, Tables tb, int n_rows) {
+k_stage_c2(float *Bc, const float2 *__restrict__ thr, uint8_t *__restrict__ stage, const int *__restrict__ slot_col,
+           Tables tb, int nb, int xcd_map) {
     // the work array, then a junk row (words LDS_FFT_N + lane, + 64) that takes
     // the slots without a column, so the scatter has no branches
     __shared__ float lds[LDS_FFT_N + 128];
@@ -1227,7 +1229,13 @@ k_stage_c2(float *Bc, const float2 *__restrict__ thr, uint8_t *__restrict__ stag
     // rows go in pairs (2 i, 2 i + 1) of one block-pol, pair blockIdx.x, + gridDim.x, ...:
     // the even row's codes wait in hold (byte q & 3 of hold[q >> 2] for element
     // te + 1024 q) and the odd row stores both as one byte
-    int row = SINGLE ? (int)blockIdx.x : 2 * (int)blockIdx.x;
+    constexpr int PER = SINGLE ? KHI : KHI / 2;
+    auto first_row = [&](int lin) {
+        int item;
+        const int b = back_bp(lin, PER, nb, xcd_map, item);
+        return __builtin_amdgcn_readfirstlane(KHI * b + (SINGLE ? item : 2 * item));
+    };
+    int lin = (int)blockIdx.x, row = first_row(lin);
     uint32_t hold[4] = {0u, 0u, 0u, 0u};
     if constexpr (P == 0) c2_load(Bc, row, pr, pi);
     for (;;) {
@@ -1240,7 +1248,11 @@ k_stage_c2(float *Bc, const float2 *__restrict__ thr, uint8_t *__restrict__ stag
             lds_put(lds, (i & 1) ? (int)(pos2[i >> 1] >> 16) : (int)(pos2[i >> 1] & 0xffffu),
                     make_float2(pr[i], pi[i]));
         __syncthreads();
-        const int next = SINGLE ? row + (int)gridDim.x : (row & 1) ? row - 1 + 2 * (int)gridDim.x : row + 1;
+        int next = row + 1;                       // the pair's odd row
+        if (SINGLE || (row & 1)) {
+            lin += (int)gridDim.x;
+            next = lin < PER * nb ? first_row(lin) : -1;
+        }
         float2 v[16];
         if constexpr (P == 0) {
             const int tr = row_tid();
@@ -1255,7 +1267,7 @@ k_stage_c2(float *Bc, const float2 *__restrict__ thr, uint8_t *__restrict__ stag
             // fft16k_tord (element fft16k_tord(t) + 1024 q in v[q])
             fft16k_p12<+1>(v, lds, &ftw, tr);
             fft16k_p3w<+1>(v, lds, &ftw, tr);
-            c2_load(Bc, next < n_rows ? next : row, pr, pi);
+            c2_load(Bc, next >= 0 ? next : row, pr, pi);
             // keep the loads here: the scheduler would otherwise sink them below
             // the stores at the end of the row, exposing their whole latency
             __builtin_amdgcn_sched_barrier(0);
@@ -1327,7 +1339,7 @@ k_stage_c2(float *Bc, const float2 *__restrict__ thr, uint8_t *__restrict__ stag
                 }
             }
         }
-        if (next >= n_rows) break;
+        if (next < 0) break;
         row = next;
     }
 }
@@ -1809,13 +1821,13 @@ int build_slot_table(sdbe_handle_t *h) {
 template <bool F32, int P>
 void launch_c2_kernel(sdbe_handle_t *h, int nb, hipStream_t s, bool single) {
     const int rows = KHI * nb, units = single ? rows : rows / 2;
-    const int grid = units < h->n_cu ? units : h->n_cu;
+    const int grid = units < h->n_cu ? units : h->n_cu, xm = nb % 8 == 0 && grid % 8 == 0;
     if (F32 || single)
         LAUNCH(h, KID_C2, nb, s, (k_stage_c2<F32, P, true>), dim3(grid), dim3(1024), (float *)h->Bc,
-               (const float2 *)h->thr, h->stage, (const int *)h->slot_col, h->tb, rows);
+               (const float2 *)h->thr, h->stage, (const int *)h->slot_col, h->tb, nb, xm);
     else
         LAUNCH(h, KID_C2, nb, s, (k_stage_c2<F32, P, F32>), dim3(grid), dim3(1024), (float *)h->Bc,
-               (const float2 *)h->thr, h->stage, (const int *)h->slot_col, h->tb, rows);
+               (const float2 *)h->thr, h->stage, (const int *)h->slot_col, h->tb, nb, xm);
 }
 
 template <bool F32>
@@ -1930,19 +1942,19 @@ int run_resampler(sdbe_handle_t *h, const BpDesc *d_bpd, int n_bp, const OutDesc
             switch (h->cfg.fft_precision) {
             case FFT_BF16X3:
                 LAUNCH(h, KID_B, nb, s, k_stage_b<FFT_BF16X3>, dim3(grid), dim3(1024), (const float2 *)h->V, h->Zf,
-                       h->tb, xm, rows);
+                       h->tb, xm, nb);
                 break;
             case FFT_BF16:
                 LAUNCH(h, KID_B, nb, s, k_stage_b<FFT_BF16>, dim3(grid), dim3(1024), (const float2 *)h->V, h->Zf,
-                       h->tb, xm, rows);
+                       h->tb, xm, nb);
                 break;
             case FFT_FP16:
                 LAUNCH(h, KID_B, nb, s, k_stage_b<FFT_FP16>, dim3(grid), dim3(1024), (const float2 *)h->V, h->Zf,
-                       h->tb, xm, rows);
+                       h->tb, xm, nb);
                 break;
             default:
                 LAUNCH(h, KID_B, nb, s, k_stage_b<0>, dim3(grid), dim3(1024), (const float2 *)h->V, h->Zf, h->tb,
-                       xm, rows);
+                       xm, nb);
             }
         }
         // whole groups of c1_ilv workgroups, tpw tiles each

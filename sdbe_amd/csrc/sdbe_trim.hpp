@@ -643,7 +643,11 @@ k_trim_seg(const float *__restrict__ T, const BpDesc *__restrict__ bpd, float *_
         fft_tw_load(&ftw, fft_tw);
         ftwp = &ftw;
     }
-    const int bpl = blockIdx.x / trim::NSEG, g = blockIdx.x - bpl * trim::NSEG, t = threadIdx.x;
+    const int bw = (int)blockIdx.x / trim::NSEG, g = blockIdx.x - bw * trim::NSEG, t = threadIdx.x;
+    // the blocks from the last: what the snapshot transforms wrote last is still in the
+    // memory-side cache (256 MB), and k_trim_pack finds the first blocks' samples there
+    // (256 block-pols at 6/11, as floats: segments 821 -> 804 us, packing 235 -> 223)
+    const int bpl = (int)gridDim.x / trim::NSEG - 1 - bw;
     // With a known threshold the samples leave as codes and not as floats: 1/16 of
     // the stores, and k_trim_pack has nothing to do for the block.  256 block-pols
     // at 6/11, segments and packing: 806 + 5 us, as floats 800 + 217; at 11/11 3895 +
