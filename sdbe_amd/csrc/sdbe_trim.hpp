@@ -213,56 +213,18 @@ __device__ __forceinline__ void pass_writes(float2 *out, int b, const float2 (&x
 // the loads and the DFT (the condition is uniform over a wave, and the barriers
 // stay outside it); the lanes of a partly used wave past NB still run on a
 // clamped butterfly and do not write.  The issue slots a skipping wave gives up
-// go to the other workgroups on its CU (3.2% at 6/11); a 1024-thread workgroup
-// fills its CU alone and gains nothing (11/11: 5594 us a group with, 5600 without).
+// go to the other workgroups on its CU; a 1024-thread workgroup fills its CU
+// alone, where the barrier waits for the busiest wave anyway (measured: 0.5%
+// slower at 11/11 with the skip, 3.2% faster at 6/11).
 template <int NB, int T>
 __device__ __forceinline__ bool wave_has_work(int it) {
-    if constexpr (NB % T == 0 || NB % T > T - 64) return true;   // no skipping wave
+    if constexpr (NB % T == 0 || NB % T > T - 64 || T >= 1024) return true;   // no skipping wave
     const int w0 = __builtin_amdgcn_readfirstlane((int)threadIdx.x & ~63);
     return it < (NB + T - 1) / T - 1 || w0 + it * T < NB;
 }
-// Table entries w, w^2, w^4, w^8 of the thread's butterflies of a pass.
-template <int N, int R, int NS, int T>
-struct PassTw {
-    static constexpr int NB = N / R, IT = (NB + T - 1) / T, STRIDE = N / (NS * R);
-    float2 w[IT][4];
-    __device__ __forceinline__ void load(const float2 *__restrict__ tab) {
-#pragma unroll
-        for (int it = 0; it < IT; ++it) {
-            if (!wave_has_work<NB, T>(it)) continue;
-            const int b0 = threadIdx.x + it * T;
-            const int m = ((NB % T == 0 || it < IT - 1 ? b0 : (b0 < NB ? b0 : NB - 1)) % NS) * STRIDE;
-            w[it][0] = tab[m];
-            if constexpr (R > 2) w[it][1] = tab[2 * m];
-            if constexpr (R > 4) w[it][2] = tab[4 * m];
-            if constexpr (R > 8) w[it][3] = tab[8 * m];
-        }
-    }
-};
-template <int R>
-__device__ __forceinline__ void pass_twiddle(float2 (&x)[R], const float2 (&w)[4]) {
-    float2 pw[16];
-    pw[1] = w[0];
-    if constexpr (R > 2) pw[2] = w[1];
-    if constexpr (R > 4) pw[4] = w[2];
-    if constexpr (R > 8) pw[8] = w[3];
-#pragma unroll
-    for (int i = 3; i < R; ++i) {
-        if (i == 4 || i == 8) continue;
-        const int hi = i >= 8 ? 8 : (i >= 4 ? 4 : 2);
-        pw[i] = cmul(pw[hi], pw[i - hi]);
-    }
-#pragma unroll
-    for (int i = 1; i < R; ++i) x[i] = cmul(x[i], pw[i]);
-}
-// The pass with its table entries loaded; `ahead` issues the loads of what follows,
-// which then have the DFTs, the writes and the barriers to arrive in (the tables are
-// in L2: 500 cycles at the start of every pass otherwise, which fewer, smaller
-// workgroups feel most: 8/11 392 -> 369 us a group, 10/11 2281 -> 2251, 6/11 1240 ->
-// 1224, 11/11 the same).
-template <int N, int R, int NS, int S, int T, bool LIN, typename Ahead>
-__device__ __forceinline__ void pass(float2 *buf, const PassTw<N, R, NS, T> &tw, Ahead ahead) {
-    constexpr int NB = N / R, IT = (NB + T - 1) / T;
+template <int N, int R, int NS, int S, int T, bool LIN = false>
+__device__ __forceinline__ void pass(float2 *buf, const float2 *__restrict__ tab) {
+    constexpr int NB = N / R, IT = (NB + T - 1) / T, STRIDE = N / (NS * R);
     static_assert(!LIN || NS >= 64, "plain output layout needs contiguous writes");
     float2 x[IT][R];
 #pragma unroll
@@ -271,11 +233,24 @@ __device__ __forceinline__ void pass(float2 *buf, const PassTw<N, R, NS, T> &tw,
         const int b0 = threadIdx.x + it * T;
         const int b = (NB % T == 0 || it < IT - 1) ? b0 : (b0 < NB ? b0 : NB - 1);
         pass_reads<N, R, S, T>(buf, b, x[it]);
-        if constexpr (NS > 1) pass_twiddle<R>(x[it], tw.w[it]);
+        if constexpr (NS > 1) {
+            const int m = (b % NS) * STRIDE;
+            float2 pw[16];
+            pw[1] = tab[m];
+            if constexpr (R > 2) pw[2] = tab[2 * m];
+            if constexpr (R > 4) pw[4] = tab[4 * m];
+            if constexpr (R > 8) pw[8] = tab[8 * m];
+#pragma unroll
+            for (int i = 3; i < R; ++i) {
+                if (i == 4 || i == 8) continue;
+                const int hi = i >= 8 ? 8 : (i >= 4 ? 4 : 2);
+                pw[i] = cmul(pw[hi], pw[i - hi]);
+            }
+#pragma unroll
+            for (int i = 1; i < R; ++i) x[it][i] = cmul(x[it][i], pw[i]);
+        }
     }
     __syncthreads();   // every read of the pass is done
-    ahead();
-    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int it = 0; it < IT; ++it) {
         if (!wave_has_work<NB, T>(it)) continue;
@@ -285,40 +260,28 @@ __device__ __forceinline__ void pass(float2 *buf, const PassTw<N, R, NS, T> &tw,
     }
     __syncthreads();
 }
-template <int N, int R, int NS, int S, int T, bool LIN = false>
-__device__ __forceinline__ void pass(float2 *buf, const float2 *__restrict__ tab) {
-    PassTw<N, R, NS, T> tw;
-    if constexpr (NS > 1) tw.load(tab);
-    pass<N, R, NS, S, T, LIN>(buf, tw, [] {});
-}
 
 // The R2C transform sizes after their first pass (pass1_global): radix passes in
 // place, T threads.  The last pass writes the plain layout (element e at e),
 // which the post-processing reads.
 template <int N, int S, int T>
-__device__ __forceinline__ void fft_tail(float2 *a, const float2 *__restrict__ tab, const PassTw<N, 8, 16, T> &t8) {
+__device__ __forceinline__ void fft_tail(float2 *a, const float2 *__restrict__ tab) {
     if constexpr (N == 4992) {
-        PassTw<N, 13, 128, T> t13;
-        pass<N, 8, 16, S, T, false>(a, t8, [&] { t13.load(tab); });
-        pass<N, 13, 128, S, T, false>(a, t13, [] {});
-        pass<N, 3, 1664, S, T, true>(a, tab);         // seven butterflies: no registers to load ahead
+        pass<N, 8, 16, S, T>(a, tab);
+        pass<N, 13, 128, S, T>(a, tab);
+        pass<N, 3, 1664, S, T, true>(a, tab);
     } else if constexpr (N == 1664) {
-        PassTw<N, 13, 128, T> t13;
-        pass<N, 8, 16, S, T, false>(a, t8, [&] { t13.load(tab); });
-        pass<N, 13, 128, S, T, true>(a, t13, [] {});
+        pass<N, 8, 16, S, T>(a, tab);
+        pass<N, 13, 128, S, T, true>(a, tab);
     } else if constexpr (N == 8320) {
-        PassTw<N, 5, 128, T> t5;
-        PassTw<N, 13, 640, T> t13;
-        pass<N, 8, 16, S, T, false>(a, t8, [&] { t5.load(tab); });
-        pass<N, 5, 128, S, T, false>(a, t5, [&] { t13.load(tab); });
-        pass<N, 13, 640, S, T, true>(a, t13, [] {});
+        pass<N, 8, 16, S, T>(a, tab);
+        pass<N, 5, 128, S, T>(a, tab);
+        pass<N, 13, 640, S, T, true>(a, tab);
     } else {
         static_assert(N == 18304, "size");
-        PassTw<N, 11, 128, T> t11;
-        PassTw<N, 13, 1408, T> t13;
-        pass<N, 8, 16, S, T, false>(a, t8, [&] { t11.load(tab); });
-        pass<N, 11, 128, S, T, false>(a, t11, [&] { t13.load(tab); });
-        pass<N, 13, 1408, S, T, true>(a, t13, [] {});
+        pass<N, 8, 16, S, T>(a, tab);
+        pass<N, 11, 128, S, T>(a, tab);
+        pass<N, 13, 1408, S, T, true>(a, tab);
     }
 }
 
@@ -660,7 +623,7 @@ k_trim_c2r_pk(const BpDesc *__restrict__ bpd, float2 *__restrict__ T, Tables tb,
 // stage + bpl * 128 P; FP64 sums of x and x^2 of the segment at
 // part[(bpl * 128 + g) * 2].
 template <int D, int E, bool F32>
-__global__ void __launch_bounds__(trim::seg_threads(D), 4)
+__global__ void __launch_bounds__(trim::seg_threads(D))
 k_trim_seg(const float *__restrict__ T, const BpDesc *__restrict__ bpd, float *__restrict__ stage,
            double *__restrict__ part, trim::Tabs tt, int skip, const float2 *__restrict__ fft_tw,
            const float *__restrict__ latch, int *__restrict__ packed, OutDesc od) {
@@ -693,10 +656,8 @@ k_trim_seg(const float *__restrict__ T, const BpDesc *__restrict__ bpd, float *_
     float2 to;
     const bool codes = !F32 && trim::known_threshold(bpd[bpl], latch, to);
     const float2 *z = reinterpret_cast<const float2 *>(T + (size_t)bpl * D * 2 * NCH + (size_t)g * R);
-    trim::PassTw<NR, 8, 16, NT> t8;
-    t8.load(tt.zr);
-    trim::pass1_global<NR, -1, NT>(buf, z);       // the input goes to registers, not through LDS
-    trim::fft_tail<NR, -1, NT>(buf, tt.zr, t8);   // Z in natural order, plain layout
+    trim::pass1_global<NR, -1, NT>(buf, z);   // the input goes to registers, not through LDS
+    trim::fft_tail<NR, -1, NT>(buf, tt.zr);   // Z in natural order, plain layout
     // bins skip .. skip + NP of the R2C, then the C2R pre-processing; the NP / 256
     // values of a thread stay in registers until every read of Z is done.
     // 2 X[k] = (Z[k] + conj Z[NR-k]) - i xr[k] (Z[k] - conj Z[NR-k]) (twice the
