@@ -29,12 +29,13 @@ namespace {
 constexpr int LW = SDBE_XCORR_WINDOW;     // 32768
 constexpr int NHW = LW / 2;               // 16384
 constexpr int KB = NHW / 256;             // bin blocks of k_xc_cross
-// Offsets per wide k_xc_cross tile.  From 64 offsets on the wide tiles give every
-// SIMD a wave (256 waves a tile, 1024 SIMDs) and what is left over goes to
-// 4-wide tiles; below that all tiles are 4 wide.  257 offsets of 256 windows, a
-// whole call: 355 us with 4-wide tiles, 287 with 8, 279 with 12, 268 with 16;
-// 63 of 128: 85 with 4, 90 with 16; 65 of 128: 92 and 83.
-constexpr int XC_OT = 16, XC_TILE_MIN = 64;
+// Offsets per wide k_xc_cross tile; what is left over goes to 4-wide tiles, and
+// below XC_TILE_MIN offsets all tiles are 4 wide.  12 is what three waves per SIMD
+// hold (168 registers; 16 takes 256).  257 offsets of 256 windows, a whole call: 283
+// us with 8, 254 with 12, 274 with 16; 201 of 100: 115, 108, 122.  Three wide tiles
+// are 768 waves for 1024 SIMDs and win already: 37 of 256 104 us, all 4 wide 114;
+// 49 of 256 116 and 145; 63 of 128 81 and 92.  Two do not: 25 of 256 104 and 104.
+constexpr int XC_OT = 12, XC_TILE_MIN = 3 * XC_OT;
 static_assert(NHW == NCH, "the correlator reuses the 16384-point FFT");
 
 // Sum over the 1024 threads of a workgroup, in every thread (red: 16 doubles).
@@ -96,9 +97,12 @@ k_xc_r2c(const float *__restrict__ x0, int first0, const float *__restrict__ x1,
 // w meets, in a ring that takes one new window per step (unrolled, so its
 // indices are constants): one load of each series and two conversions per OT
 // offsets, where a thread per (bin, offset) loaded and converted both for every
-// offset.  That is 4 OT FP64 FMAs per step, which bound it: 110 us for 257
-// offsets of 256 windows at one wave instruction per CU and cycle, measured 170
-// (before: 1050, the loads and conversions).
+// offset.  The FP64 FMAs bound it, so a complex product is three of them and not
+// four (ax bx, ay by, (ax + ay)(bx - by); the second factor comes once per window):
+// the factors are FP32 values and their sums, which FP64 holds with room to spare, and
+// the rounding of the three sums is 1e-16 of the powers.  82 us for 257 offsets of 256
+// windows at one wave instruction per CU and cycle; a whole call 254 us, with four
+// products and 16 offsets a thread 290, with a thread per (bin, offset) 1165.
 // Bin blocks are the fastest grid dimension, 64 of them, so the tiles of a bin
 // block run on one XCD and read the same windows through its L2 at about the
 // same time.
@@ -106,24 +110,28 @@ template <int OT>
 __device__ __forceinline__ void cross_tile(const float2 *__restrict__ X0, const float2 *__restrict__ X1, int avg,
                                            int n_off, int o0, int k, float2 *__restrict__ S) {
     const int last = n_off + avg - 2;          // last x1 window; a tile past n_off loads it again
-    double sr[OT], si[OT], bx[OT], by[OT];
+    // sums of ax bx, ay by and (ax + ay)(bx - by); a conj(b) = pr + pi + i (pd - pr + pi)
+    double pr[OT], pi[OT], pd[OT], bx[OT], by[OT], bd[OT];
 #pragma unroll
     for (int j = 0; j < OT; ++j) {
         const float2 b = X1[(size_t)min(o0 + j, last) * NHW + k];
-        sr[j] = si[j] = 0.0;
+        pr[j] = pi[j] = pd[j] = 0.0;
         bx[j] = b.x;       // slot OT - 1 is replaced by the first step
         by[j] = b.y;
+        bd[j] = bx[j] - by[j];
     }
     // step i of a block of OT: window o0 + w + j of x1 is in slot (i + j) % OT
     auto step = [&](int i, float2 a, float2 b) {
-        const double ax = a.x, ay = a.y;
-        bx[(i + OT - 1) % OT] = b.x;
-        by[(i + OT - 1) % OT] = b.y;
+        const double ax = a.x, ay = a.y, as = ax + ay;
+        constexpr int N1 = OT - 1;
+        bx[(i + N1) % OT] = b.x;
+        by[(i + N1) % OT] = b.y;
+        bd[(i + N1) % OT] = bx[(i + N1) % OT] - by[(i + N1) % OT];
 #pragma unroll
         for (int j = 0; j < OT; ++j) {
-            const double cx = bx[(i + j) % OT], cy = by[(i + j) % OT];
-            sr[j] = fma(ax, cx, fma(ay, cy, sr[j]));     // a conj(b)
-            si[j] = fma(ay, cx, fma(-ax, cy, si[j]));
+            pr[j] = fma(ax, bx[(i + j) % OT], pr[j]);
+            pi[j] = fma(ay, by[(i + j) % OT], pi[j]);
+            pd[j] = fma(as, bd[(i + j) % OT], pd[j]);
         }
     };
     int w = 0;
@@ -143,7 +151,9 @@ __device__ __forceinline__ void cross_tile(const float2 *__restrict__ X0, const 
             step(i, X0[(size_t)(w + i) * NHW + k], X1[(size_t)min(o0 + w + i + OT - 1, last) * NHW + k]);
 #pragma unroll
     for (int j = 0; j < OT; ++j)
-        if (o0 + j < n_off) S[(size_t)(o0 + j) * NHW + k] = make_float2((float)(sr[j] / avg), (float)(si[j] / avg));
+        if (o0 + j < n_off)
+            S[(size_t)(o0 + j) * NHW + k] =
+                make_float2((float)((pr[j] + pi[j]) / avg), (float)((pd[j] - pr[j] + pi[j]) / avg));
 }
 
 // n_wide tiles of OT offsets, then tiles of 4 for the rest

@@ -1,5 +1,5 @@
 """GPU: the cross-power tiles of sdbe_xcorr_search at their edges (4-wide tiles
-below 64 offsets, 16-wide ones with a 4-wide rest from there on; averages below,
+below 36 offsets, 12-wide ones with a 4-wide rest from there on; averages below,
 at and past a multiple of the tile width) against the FP64 oracle: lag functions
 within 2e-5, peaks and standard deviations within 1e-4 relative (the bars of
 test_gpu_xcorr: FP32 transforms of normalised values)."""
@@ -36,3 +36,8 @@ def test_cross_tiles(n_off, avg):
     assert np.abs(s - so).max() <= 2e-5
     assert np.allclose(peak, po, rtol=1e-4) and np.allclose(std, so.std(axis=1), rtol=1e-4)
     xc.close()
+
+
+@pytest.mark.parametrize("n_off,avg", [(35, 12), (36, 1), (36, 11), (37, 12), (41, 13), (47, 25)])
+def test_cross_tiles_first_wide(n_off, avg):
+    test_cross_tiles(n_off, avg)
