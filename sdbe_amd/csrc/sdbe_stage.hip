@@ -1875,8 +1875,9 @@ int run_trim(sdbe_handle_t *h, const BpDesc *d_bpd, int n_bp, const OutDesc &od,
     constexpr int P = 256 * E;
     const auto kc2r = k_trim_c2r<D>;
     const auto kc2r_pk = h->geom == SDBE_GEOM_8X1024 ? k_trim_c2r_pk<D, true> : k_trim_c2r_pk<D, false>;
-    const auto kseg_f = k_trim_seg<D, E, true>;
-    const auto kseg_c = k_trim_seg<D, E, false>;
+    const auto kseg_f = k_trim_seg<D, E, true, false>;
+    const auto kseg_c = h->cfg.thresh_policy == SDBE_THRESH_PER_BLOCK ? k_trim_seg<D, E, false, false>
+                                                                      : k_trim_seg<D, E, false, true>;
     int *packed = reinterpret_cast<int *>(h->stage);     // a flag per block-pol, in the 64/39 path's code buffer
     for (int bp0 = 0; bp0 < n_bp; bp0 += h->chunk) {
         const int nb = (n_bp - bp0) < h->chunk ? (n_bp - bp0) : h->chunk;

@@ -622,7 +622,7 @@ k_trim_c2r_pk(const BpDesc *__restrict__ bpd, float2 *__restrict__ T, Tables tb,
 // out[bpl] + g P, where out is bpd[bpl].out (float samples) when F32, else
 // stage + bpl * 128 P; FP64 sums of x and x^2 of the segment at
 // part[(bpl * 128 + g) * 2].
-template <int D, int E, bool F32>
+template <int D, int E, bool F32, bool CODES>
 __global__ void __launch_bounds__(trim::seg_threads(D))
 k_trim_seg(const float *__restrict__ T, const BpDesc *__restrict__ bpd, float *__restrict__ stage,
            double *__restrict__ part, trim::Tabs tt, int skip, const float2 *__restrict__ fft_tw,
@@ -652,9 +652,11 @@ k_trim_seg(const float *__restrict__ T, const BpDesc *__restrict__ bpd, float *_
     // the stores, and k_trim_pack has nothing to do for the block.  256 block-pols
     // at 6/11, segments and packing: 806 + 5 us, as floats 800 + 217; at 11/11 3895 +
     // 10 and 3965 + 833.  (Decided here, ahead of the transforms: a branch between
-    // them splits the schedule and takes 130 registers more.)
+    // them splits the schedule and takes 130 registers more.)  Without CODES, for calls
+    // whose blocks all have the PER_BLOCK policy, the branch is not there.
+    static_assert(!(F32 && CODES), "float output has no codes");
     float2 to;
-    const bool codes = !F32 && trim::known_threshold(bpd[bpl], latch, to);
+    const bool codes = CODES && trim::known_threshold(bpd[bpl], latch, to);
     const float2 *z = reinterpret_cast<const float2 *>(T + (size_t)bpl * D * 2 * NCH + (size_t)g * R);
     trim::pass1_global<NR, -1, NT>(buf, z);   // the input goes to registers, not through LDS
     trim::fft_tail<NR, -1, NT>(buf, tt.zr);   // Z in natural order, plain layout
