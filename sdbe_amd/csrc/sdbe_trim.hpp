@@ -653,7 +653,9 @@ k_trim_seg(const float *__restrict__ T, const BpDesc *__restrict__ bpd, float *_
     // at 6/11, segments and packing: 806 + 5 us, as floats 800 + 217; at 11/11 3895 +
     // 10 and 3965 + 833.  (Decided here, ahead of the transforms: a branch between
     // them splits the schedule and takes 130 registers more.)  Without CODES, for calls
-    // whose blocks all have the PER_BLOCK policy, the branch is not there.
+    // whose blocks all have the PER_BLOCK policy, the branch is not there: a group at 10/11
+    // 3111 -> 2962 us, at 6/11 1526 -> 1504 (on two boxes; before there was a code path
+    // 3086 and 2996, 1530 and 1526).
     static_assert(!(F32 && CODES), "float output has no codes");
     float2 to;
     const bool codes = CODES && trim::known_threshold(bpd[bpl], latch, to);
