@@ -15,13 +15,14 @@
 //                   (16384-point complex FFT in LDS + split post-processing)
 //   k_pfb_fold2_r2c the same for calls of more spectra than CUs, two at a time
 //   k_pfb_c2r       packed C2R of each spectrum to the pseudo-timestream
-// The solve, for any prototype without zeros together on the unit circle:
+// The solve, for prototypes that a constant factor loses nothing in
+// (sdbe_pfb_solve.hpp: the rule and what it was measured over):
 //   k_pfb_spectral  once per plan, one thread per branch: the constant
 //                   minimum-phase factor of P P^T and the tables built on it
 //   k_pfb_span, k_pfb_join, k_pfb_solve
 //                   two recursive filters, block-parallel over the rows
-//   k_pfb_corner    calls of up to 256 rows: their tables, then k_pfb_solve alone
-// and for the others the factor-row kernels:
+//   k_pfb_corner    calls of up to 256 rows: their corner, then k_pfb_solve alone
+// and for the others, if one branch is of that kind, the factor-row kernels:
 //   k_pfb_factor    once per plan, one thread per branch: banded Cholesky of
 //                   P P^T (bandwidth 3, Toeplitz per branch), FP64; the factor's
 //                   state is checkpointed every 16 rows
@@ -46,10 +47,12 @@
 #include <vector>
 
 #include "sdbe_device.hpp"
+#include "sdbe_pfb_solve.hpp"
 #include "../../include/sdbe_pfb.h"
 #include "../../include/sdbe_stage.h"
 
 using namespace sdbe;
+using namespace sdbe::pfb;
 
 namespace {
 
@@ -677,321 +680,62 @@ k_pfb_bfin(const float *__restrict__ yh, const double *__restrict__ uck, int nbl
 }
 
 // --------------------------------------------- constant-coefficient solve
-// P P^T is Toeplitz per branch, so it has a constant minimum-phase factor b:
-// b(q) = b0 + b1 q + b2 q^2 + b3 q^3 with the taps' autocorrelation and no zero
-// inside the unit circle (the taps' polynomial with its zeros inside reflected),
-// and with B the lower-triangular Toeplitz matrix of b
-//   P P^T = B B^T + E H H^T E^T,   H[i][m] = b_{i+m+1}  (E: the first three rows).
-// B B^T is two recursive filters with three constant coefficients beta = b_k / b0
-// (no factor rows to recompute or checkpoint), and the corner is a rank-3
-// correction: with z0 the filters' solution, g = W z0[0..2] is taken off the
-// first three right-hand sides, W = H (I + H^T G H)^-1 H^T, G the first 3 x 3
-// block of (B B^T)^-1.  In scaled units v = b0 B^-1 y, zeta = b0^2 z:
-//   v_i = y_i - beta1 v_{i-1} - beta2 v_{i-2} - beta3 v_{i-3},
-//   zeta_i = v_i - beta1 zeta_{i+1} - beta2 zeta_{i+2} - beta3 zeta_{i+3}.
-// Rounding: the tables are computed in double-double and the corner takes one
-// refinement step, so the FP32 rounding of yh is all that is left in the result.
-// Against an 80-bit solve, over the 280 worst branches of a Hamming prototype
-// (double zeros near -0.995): 1.65e-7 to 1.79e-7 at 256 to 4096 rows, where the
-// FP64 factor rows are themselves off by up to 3.0e-7 (4096 rows).  The exception is
-// two zeros together on the unit circle: taps 1, 2, 1 lose 5e-5 in 1000 rows here
-// and 1e-8 by factor rows.
-// k_pfb_spectral counts such branches, and a plan that has any takes those.
+// The factor, its tables, the corner and the rule that admits a plan are in
+// sdbe_pfb_solve.hpp; here they run block-parallel over the rows.
 //
 // Thread (branch, span of 32 rows) keeps its rows' v in registers; a workgroup
-// holds 64 branches x 8 spans and scans the spans' boundary states through LDS.
+// holds 64 branches x 8 spans and scans the spans' boundary states through LDS, and
+// each span's head zeta is taken from its true v (from the v of a zero incoming
+// state it would lose the 32 rows' growth of both filters).
 // Up to 256 rows that is the whole problem.  Above, k_pfb_span takes every
 // 256-row block's outgoing states in both directions (from zero incoming ones) in
 // one read of yh, k_pfb_join composes them per branch into the blocks' true
 // incoming states with the corner, and k_pfb_solve finishes the blocks: two
-// reads of yh and one write of x, all in 256-byte runs.  4096 spectra: span 130 us
-// (4.1 TB/s), join 27, solve 225 (4.8 TB/s, the rate of a large copy); the
-// factor-row kernels, which read yh four times beside 0.8 GB of checkpoints and
-// recompute every factor row four times, take 890.  (Tiles of 8 branches over
+// reads of yh and one write of x, all in 256-byte runs.  4096 spectra: span 128 us
+// (4.2 TB/s), join 29, solve 247 (4.3 TB/s); the factor-row kernels, which read yh
+// four times beside 0.8 GB of checkpoints and recompute every factor row four
+// times, take 890.  A call of 256 rows: corner 13, solve 28.  (Tiles of 8 branches over
 // all 4096 rows read yh once, but in 32-byte runs: 700 us.)
-constexpr int SR = 32, SWV = 8, SBLK = SR * SWV;     // rows per thread, waves and rows per workgroup
-// table rows, [row][LB] doubles
-constexpr int TB_BETA = 0;                // beta1..3
-constexpr int TB_WZ = 3;                  // taps / b0^2
-constexpr int TB_CS = 7;                  // C^32: the state after a span of no input
-constexpr int TB_CB = 16;                 // C^256
-constexpr int TB_RS = 25;                 // a span's head zeta per unit incoming state
-constexpr int TB_HS = 34;                 // its impulse response h27..h31
-constexpr int TB_RB = 39;                 // the same of a block: head zeta
-constexpr int TB_HB = 48;                 // ... h251..h255
-constexpr int TB_GB = 53;                 // ... first 3 x 3 block of (B B^T)^-1
-constexpr int TB_N = 62;
-// ... and of a call
-constexpr int TC_W = 0;                   // corner matrix W (scaled)
-constexpr int TC_RS = 9;                  // TB_RS of the partial last span
-constexpr int TC_G = 18;                  // more than one block: g
-constexpr int TC_N = 21;
 
-// 3 x 3 matrices, m[3 r + c]
-__device__ __forceinline__ void mat_mul(double (&o)[9], const double (&a)[9], const double (&b)[9]) {
-#pragma unroll
-    for (int r = 0; r < 3; ++r)
-#pragma unroll
-        for (int c = 0; c < 3; ++c) o[3 * r + c] = a[3 * r] * b[c] + a[3 * r + 1] * b[3 + c] + a[3 * r + 2] * b[6 + c];
-}
+// Table rows of a call.
+constexpr int TC_S = 0;                   // the corner's Cholesky factor
+constexpr int TC_T = 6;                   // more than one block: t
+constexpr int TC_N = 9;
 
-// Double-double: h + l, |l| at most half an ulp of h.
-struct Dd {
-    double h = 0.0, l = 0.0;
-};
-__device__ __forceinline__ Dd dd_norm(double h, double l) {
-    const double s = h + l;
-    return Dd{s, l - (s - h)};
-}
-__device__ __forceinline__ Dd dd_add(Dd a, Dd b) {
-    const double s = a.h + b.h, t = s - a.h;
-    return dd_norm(s, (a.h - (s - t)) + (b.h - t) + (a.l + b.l));
-}
-__device__ __forceinline__ Dd dd_mul(Dd a, Dd b) {
-    const double p = a.h * b.h;
-    return dd_norm(p, fma(a.h, b.h, -p) + fma(a.h, b.l, a.l * b.h));
-}
-// a - b c
-__device__ __forceinline__ Dd dd_sub_mul(Dd a, Dd b, double c) { return dd_add(a, dd_mul(b, Dd{-c, 0.0})); }
-
-// sum_{k < n} C^k X (C^k)^T (TR) or sum_{k < n} C^k X C^k, by doubling over the
-// bits of n.
-template <bool TR>
-__device__ __forceinline__ void power_sum(int n, const double (&C)[9], const double (&X)[9], double (&S)[9]) {
-    double P[9], t[9], u[9];
-    auto add = [&](const double (&m)[9], const double (&x)[9]) {   // S = x + m S m(^T)
-        mat_mul(t, m, S);
-        if (TR) {
-#pragma unroll
-            for (int r = 0; r < 3; ++r)
-#pragma unroll
-                for (int c = 0; c < 3; ++c)
-                    u[3 * r + c] = t[3 * r] * m[3 * c] + t[3 * r + 1] * m[3 * c + 1] + t[3 * r + 2] * m[3 * c + 2];
-        } else {
-            mat_mul(u, t, m);
-        }
-#pragma unroll
-        for (int i = 0; i < 9; ++i) S[i] = x[i] + u[i];
-    };
-#pragma unroll
-    for (int i = 0; i < 9; ++i) {
-        P[i] = C[i];
-        S[i] = n > 0 ? X[i] : 0.0;
-    }
-    for (int bit = n > 0 ? 30 - __builtin_clz(n) : -1; bit >= 0; --bit) {     // below n's leading bit
-        add(P, S);
-        mat_mul(t, P, P);
-#pragma unroll
-        for (int i = 0; i < 9; ++i) P[i] = t[i];
-        if ((n >> bit) & 1) {
-            add(C, X);
-            mat_mul(t, C, P);
-#pragma unroll
-            for (int i = 0; i < 9; ++i) P[i] = t[i];
-        }
-    }
-}
-
-// Head zeta (rows 0..2, nothing incoming from below) of n rows whose v is the
-// response to the incoming state e_c, in column c: v_k = (C^(k+1))[0][c], and
-// zeta_r = sum_k v_k h_{k-r} with (h_k, h_{k-1}, h_{k-2}) = C^k e_0.
-__device__ __forceinline__ void head_response(int n, double be1, double be2, double be3, double (&rm)[9]) {
-    const double C[9] = {-be1, -be2, -be3, 1.0, 0.0, 0.0, 0.0, 1.0, 0.0};
-    const double X[9] = {-be1, -be2, -be3, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
-    power_sum<false>(n, C, X, rm);
-}
-
-// Per plan, one thread per branch: the minimum-phase factor and the tables.
-// The cubic's real zero by Cardano's formula and Newton steps, deflated from the
-// end that keeps the remaining coefficients accurate, then the quadratic.
-// *clustered counts the branches with two zeros together on the unit circle.
+// Per plan, one thread per branch.  *refused counts the branches that the
+// constant-coefficient solve would lose more in than it may.
 __global__ void __launch_bounds__(SOLVE_WG)
-k_pfb_spectral(const float *__restrict__ win, double *__restrict__ tab, int *__restrict__ clustered) {
+k_pfb_spectral(const float *__restrict__ win, int blocks, double *__restrict__ tab, int *__restrict__ refused) {
     const int n = blockIdx.x * SOLVE_WG + threadIdx.x;
-    const double w[4] = {win[n], win[LB + n], win[2 * LB + n], win[3 * LB + n]};
-    const double sc = fmax(fmax(fabs(w[0]), fabs(w[1])), fmax(fabs(w[2]), fabs(w[3])));
-    // c0 x^3 + c1 x^2 + c2 x + c3, |c0| >= |c3| (either order has the autocorrelation),
-    // zeros wanted in |x| <= 1
-    const bool rev = fabs(w[3]) > fabs(w[0]);
-    double c[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) c[i] = (rev ? w[3 - i] : w[i]) / sc;
-    double b[4];
-    bool close = false;
-    if (fabs(c[0]) <= 1e-15) {      // both ends vanish: two taps
-        const bool f = fabs(c[1]) >= fabs(c[2]);
-        b[0] = f ? c[1] : c[2];
-        b[1] = f ? c[2] : c[1];
-        b[2] = b[3] = 0.0;
-    } else {
-        const double A = c[1] / c[0], B = c[2] / c[0], C = c[3] / c[0];
-        const double Q = (A * A - 3.0 * B) / 9.0, R = (2.0 * A * A * A - 9.0 * A * B + 27.0 * C) / 54.0;
-        double r;
-        if (R * R < Q * Q * Q) {    // three real zeros: the largest
-            const double th = acos(fmax(-1.0, fmin(1.0, R / sqrt(Q * Q * Q))));
-            const double m = -2.0 * sqrt(Q), tau = 6.283185307179586476925286766559;
-            r = m * cos(th / 3.0) - A / 3.0;
-            for (int k = 1; k < 3; ++k) {
-                const double x = m * cos((th + k * tau) / 3.0) - A / 3.0;
-                if (fabs(x) > fabs(r)) r = x;
-            }
-        } else {
-            const double s = -copysign(cbrt(fabs(R) + sqrt(fmax(R * R - Q * Q * Q, 0.0))), R);
-            r = s + (s != 0.0 ? Q / s : 0.0) - A / 3.0;
-        }
-        for (int k = 0; k < 4; ++k) {
-            const double f = ((r + A) * r + B) * r + C, d = (3.0 * r + 2.0 * A) * r + B;
-            if (d == 0.0) break;
-            const double x = r - f / d;
-            if (!(fabs(((x + A) * x + B) * x + C) < fabs(f))) break;
-            r = x;
-        }
-        // x^2 + d1 x + d0: coefficients above the largest of the terms |C|, |B r|,
-        // |A r^2|, |r^3| from the top, those below it from the bottom
-        double d1 = A + r, d0 = B + d1 * r;
-        if (r != 0.0) {
-            const double t0 = fabs(C), t1 = fabs(B * r), t2 = fabs(A * r * r), t3 = fabs(r * r * r);
-            if (fmax(t2, t3) > fmax(t0, t1) || t1 > t0) d0 = -C / r;
-            if (fmax(t2, t3) > fmax(t0, t1)) d1 = (d0 - B) / r;
-        }
-        double pol[4] = {c[0], 0.0, 0.0, 0.0};
-        auto times = [&](double x) {        // times (x' - x), or reflected: (1 - x x')
-            const double u = fabs(x) > 1.0 ? -x : 1.0, v = fabs(x) > 1.0 ? 1.0 : -x;
-#pragma unroll
-            for (int i = 3; i >= 1; --i) pol[i] = pol[i] * u + pol[i - 1] * v;
-            pol[0] *= u;
-        };
-        auto inside = [](double x) { return fabs(x) > 1.0 ? 1.0 / x : x; };
-        times(r);
-        bool any = fabs(r) > 1.0;              // a zero was reflected
-        const double disc = d1 * d1 - 4.0 * d0, ri = inside(r);
-        constexpr double NEAR = 0.998, GAP = 0.02;
-        if (disc >= 0.0) {
-            const double s = -0.5 * (d1 + copysign(sqrt(disc), d1)), x2 = s != 0.0 ? d0 / s : 0.0;
-            times(s);
-            times(x2);
-            any = any || fabs(s) > 1.0 || fabs(x2) > 1.0;
-            const double si = inside(s), xi = inside(x2);
-            close = (fmin(fabs(ri), fabs(si)) > NEAR && fabs(ri - si) < GAP) ||
-                    (fmin(fabs(ri), fabs(xi)) > NEAR && fabs(ri - xi) < GAP) ||
-                    (fmin(fabs(si), fabs(xi)) > NEAR && fabs(si - xi) < GAP);
-        } else {
-            const bool out = d0 > 1.0;
-            any = any || out;
-            const double e0 = out ? d0 : 1.0, e2 = out ? 1.0 : d0;
-            const double p0 = pol[0], p1 = pol[1];
-            pol[0] = p0 * e0;
-            pol[1] = p0 * d1 + p1 * e0;
-            pol[2] = p0 * e2 + p1 * d1;
-            pol[3] = p1 * e2;
-            const double re = -0.5 * d1 / e0, im = 0.5 * sqrt(-disc) / e0, mod = sqrt(fmin(d0, 1.0 / d0));
-            close = mod > NEAR && (2.0 * im < GAP || (fabs(ri) > NEAR && hypot(ri - re, im) < GAP));
-        }
-        // taps that are minimum phase already (in either order) are the factor, exactly
-#pragma unroll
-        for (int i = 0; i < 4; ++i) b[i] = any ? pol[i] : c[i];
-    }
-    if (close) atomicAdd(clustered, 1);
-    const double be1 = b[1] / b[0], be2 = b[2] / b[0], be3 = b[3] / b[0], b0 = b[0] * sc;
-    double *o = tab + n;
-    o[(size_t)(TB_BETA + 0) * LB] = be1;
-    o[(size_t)(TB_BETA + 1) * LB] = be2;
-    o[(size_t)(TB_BETA + 2) * LB] = be3;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) o[(size_t)(TB_WZ + i) * LB] = w[i] / b0 / b0;
-    // The span's and the block's responses, by recursion over their rows in
-    // double-double: near-double zeros close to the unit circle (the Hamming
-    // prototype has some around branches 4050 and 28720) amplify the tables'
-    // rounding into the result, 3e-7 of it with powers by squaring in FP64.
-    Dd v[3][3] = {{{1.0, 0.0}, {}, {}}, {{}, {1.0, 0.0}, {}}, {{}, {}, {1.0, 0.0}}};   // chain c: its last three values
-    Dd h[3] = {}, rm[9] = {}, g[6] = {};
-    for (int k = 0; k < SBLK; ++k) {
-        const Dd in{k == 0 ? 1.0 : 0.0, 0.0};
-        const Dd hk = dd_sub_mul(dd_sub_mul(dd_sub_mul(in, h[0], be1), h[1], be2), h[2], be3);
-        h[2] = h[1];
-        h[1] = h[0];
-        h[0] = hk;
-#pragma unroll
-        for (int c = 0; c < 3; ++c) {
-            const Dd x = dd_sub_mul(dd_sub_mul(dd_sub_mul(Dd{}, v[c][0], be1), v[c][1], be2), v[c][2], be3);
-            v[c][2] = v[c][1];
-            v[c][1] = v[c][0];
-            v[c][0] = x;
-#pragma unroll
-            for (int r = 0; r < 3; ++r) rm[3 * r + c] = dd_add(rm[3 * r + c], dd_mul(x, h[r]));
-        }
-#pragma unroll
-        for (int r = 0, i = 0; r < 3; ++r)
-#pragma unroll
-            for (int c = r; c < 3; ++c, ++i) g[i] = dd_add(g[i], dd_mul(h[r], h[c]));
-        if (k < SR && k >= SR - 5) o[(size_t)(TB_HS + k - (SR - 5)) * LB] = hk.h;
-        if (k >= SBLK - 5) o[(size_t)(TB_HB + k - (SBLK - 5)) * LB] = hk.h;
-        if (k == SR - 1 || k == SBLK - 1) {
-            const int cr = k == SR - 1 ? TB_CS : TB_CB, rr = k == SR - 1 ? TB_RS : TB_RB;
-#pragma unroll
-            for (int r = 0; r < 3; ++r)
-#pragma unroll
-                for (int c = 0; c < 3; ++c) {
-                    o[(size_t)(cr + 3 * r + c) * LB] = v[c][r].h;
-                    o[(size_t)(rr + 3 * r + c) * LB] = rm[3 * r + c].h;
-                }
-        }
-    }
-#pragma unroll
-    for (int r = 0, i = 0; r < 3; ++r)
-#pragma unroll
-        for (int c = r; c < 3; ++c, ++i) o[(size_t)(TB_GB + 3 * r + c) * LB] = o[(size_t)(TB_GB + 3 * c + r) * LB] = g[i].h;
+    const float w[4] = {win[n], win[LB + n], win[2 * LB + n], win[3 * LB + n]};
+    if (!admitted(plan_tables(w, blocks, tab + n, LB))) atomicAdd(refused, 1);
 }
 
-// The corner matrix W of N rows, and G = sum_{i < N} s_i s_i^T with s_i = C^i e_0.
-__device__ __forceinline__ void corner(int N, double be1, double be2, double be3, double (&W)[9], double (&G)[9]) {
-    const double C[9] = {-be1, -be2, -be3, 1.0, 0.0, 0.0, 0.0, 1.0, 0.0};
-    const double X[9] = {1.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
-    double t[9];
-    power_sum<true>(N, C, X, G);
-    // H (scaled by 1 / b0), rows past N zero
-    const double H[9] = {be1, be2, be3, N > 1 ? be2 : 0.0, N > 1 ? be3 : 0.0, 0.0, N > 2 ? be3 : 0.0, 0.0, 0.0};
-    double S[9], K[9];
-    mat_mul(t, G, H);
+__device__ __forceinline__ Beta beta_load(const double *__restrict__ tab, int n) {
+    return Beta{tab[n], tab[LB + n], tab[2 * LB + n]};
+}
+__device__ __forceinline__ void corner_store(double *__restrict__ tc, int n, const Corner &c) {
+    const double s[6] = {c.i0, c.l10, c.l20, c.i1, c.l21, c.i2};
 #pragma unroll
-    for (int r = 0; r < 3; ++r)
+    for (int i = 0; i < 6; ++i) tc[(size_t)(TC_S + i) * LB + n] = s[i];
+}
+__device__ __forceinline__ Corner corner_load(const double *__restrict__ tc, int n) {
+    double s[6];
 #pragma unroll
-        for (int c = 0; c < 3; ++c)
-            S[3 * r + c] = (r == c ? 1.0 : 0.0) + H[r] * t[c] + H[3 + r] * t[3 + c] + H[6 + r] * t[6 + c];
-    // S = L L^T (symmetric, eigenvalues >= 1); K = L^-1 H^T, W = K^T K
-    const double l00 = 1.0 / sqrt(S[0]), l10 = S[3] * l00, l20 = S[6] * l00;
-    const double l11 = 1.0 / sqrt(S[4] - l10 * l10), l21 = (S[7] - l20 * l10) * l11;
-    const double l22 = 1.0 / sqrt(S[8] - l20 * l20 - l21 * l21);
-#pragma unroll
-    for (int c = 0; c < 3; ++c) {      // column c of H^T is row c of H
-        K[c] = H[3 * c] * l00;
-        K[3 + c] = (H[3 * c + 1] - l10 * K[c]) * l11;
-        K[6 + c] = (H[3 * c + 2] - l20 * K[c] - l21 * K[3 + c]) * l22;
-    }
-#pragma unroll
-    for (int r = 0; r < 3; ++r)
-#pragma unroll
-        for (int c = 0; c < 3; ++c) W[3 * r + c] = K[r] * K[c] + K[3 + r] * K[3 + c] + K[6 + r] * K[6 + c];
+    for (int i = 0; i < 6; ++i) s[i] = tc[(size_t)(TC_S + i) * LB + n];
+    return Corner{s[0], s[1], s[2], s[3], s[4], s[5]};
 }
 
-// Per call of at most one block, one thread per branch: its tables.
+// Per call of at most one block, one thread per branch: its corner.
 __global__ void __launch_bounds__(SOLVE_WG)
 k_pfb_corner(const double *__restrict__ tab, int N, double *__restrict__ tc) {
     const int n = blockIdx.x * SOLVE_WG + threadIdx.x;
-    const double be1 = tab[n], be2 = tab[LB + n], be3 = tab[2 * LB + n];
-    double W[9], G[9], rm[9];
-    corner(N, be1, be2, be3, W, G);
-    head_response(N & (SR - 1), be1, be2, be3, rm);
-#pragma unroll
-    for (int i = 0; i < 9; ++i) {
-        tc[(size_t)(TC_W + i) * LB + n] = W[i];
-        tc[(size_t)(TC_RS + i) * LB + n] = rm[i];
-    }
+    const Beta be = beta_load(tab, n);
+    double R[9], G[9];
+    row_responses(N, be, R, G);
+    corner_store(tc, n, corner(be, G));
 }
 
-struct V3 {
-    double a, b, c;
-};
 __device__ __forceinline__ V3 v3_load(const double *__restrict__ p, int n) {
     return V3{p[n], p[LB + n], p[2 * LB + n]};
 }
@@ -1000,16 +744,6 @@ __device__ __forceinline__ void v3_store(double *__restrict__ p, int n, V3 v) {
     p[LB + n] = v.b;
     p[2 * LB + n] = v.c;
 }
-// x + M y, M's element i at m[i * ST]
-template <int ST>
-__device__ __forceinline__ V3 mv_add(V3 x, const double *m, V3 y) {
-    return V3{fma(m[0], y.a, fma(m[ST], y.b, fma(m[2 * ST], y.c, x.a))),
-              fma(m[3 * ST], y.a, fma(m[4 * ST], y.b, fma(m[5 * ST], y.c, x.b))),
-              fma(m[6 * ST], y.a, fma(m[7 * ST], y.b, fma(m[8 * ST], y.c, x.c)))};
-}
-
-// The filter's next value from its last three.
-#define PFB_FILTER(in, s) fma(-be1, (s).a, fma(-be2, (s).b, fma(-be3, (s).c, (in))))
 
 // Outgoing states of block blockIdx.y from zero incoming ones: P = its last three
 // v, Q = its first three zeta.  Q is a sum over the rows, sum_k v_k h_{k-r}, so
@@ -1018,7 +752,7 @@ __global__ void __launch_bounds__(SOLVE_WG)
 k_pfb_span(const float *__restrict__ yh, int N, const double *__restrict__ tab, double *__restrict__ P,
            double *__restrict__ Q) {
     const int n = blockIdx.x * SOLVE_WG + threadIdx.x, blk = blockIdx.y, r0 = blk * SBLK, r1 = min(r0 + SBLK, N);
-    const double be1 = tab[n], be2 = tab[LB + n], be3 = tab[2 * LB + n];
+    const Beta be = beta_load(tab, n);
     V3 st{0.0, 0.0, 0.0}, q = st, h{0.0, 0.0, 0.0};
     double in = 1.0;                       // h's input: an impulse at the block's first row
     constexpr int CH = 32;
@@ -1030,11 +764,11 @@ k_pfb_span(const float *__restrict__ yh, int N, const double *__restrict__ tab, 
 #pragma unroll
         for (int k = 0; k < CH; ++k) {
             if (full || c0 + k < r1) {
-                const double v = PFB_FILTER((double)y[k], st), hk = PFB_FILTER(in, h);
+                const double v = filter(be, (double)y[k], st), hk = filter(be, in, h);
                 in = 0.0;
                 q = V3{fma(v, hk, q.a), fma(v, h.a, q.b), fma(v, h.b, q.c)};
-                st = V3{v, st.a, st.b};
-                h = V3{hk, h.a, h.b};
+                st = shift(v, st);
+                h = shift(hk, h);
             }
         }
     }
@@ -1043,28 +777,21 @@ k_pfb_span(const float *__restrict__ yh, int N, const double *__restrict__ tab, 
 }
 
 // Per branch: the blocks' true incoming states A (from above) and B (from below),
-// the corner's g, and the partial last span's head response.  The walks over the
-// blocks are short dependent chains on few waves (512), so up to JOIN_LDS blocks
-// the states wait in LDS, all loaded at the start (IN_LDS); longer calls keep
-// them in A and Q, which is overwritten.
+// and the corner with its t.  Each step of t composes the blocks anew from the
+// states of k_pfb_span, so that what t takes off the first block is taken off
+// before it is carried on.  The walks over the blocks are short dependent chains on few
+// waves (512), so up to JOIN_LDS blocks the states wait in LDS, all loaded at the
+// start (IN_LDS: P, Q and the heads, 72 KB); longer calls read them again and keep
+// the heads in B.  4096 spectra 29 us, 4097 57 (of 690 for the call).
 constexpr int JOIN_LDS = 16;
 template <bool IN_LDS>
 __global__ void __launch_bounds__(SOLVE_WG)
-k_pfb_join(const double *__restrict__ tab, int N, int nb, const double *__restrict__ P, double *Q, double *A,
-           double *__restrict__ B, double *__restrict__ tc) {
-    __shared__ V3 sh[IN_LDS ? 2 * JOIN_LDS * SOLVE_WG : 1];
+k_pfb_join(const double *__restrict__ tab, int N, int nb, const double *__restrict__ P, const double *__restrict__ Q,
+           double *__restrict__ A, double *B, double *__restrict__ tc) {
+    __shared__ V3 sh[IN_LDS ? 3 * JOIN_LDS * SOLVE_WG : 1];
     const int t = threadIdx.x, n = blockIdx.x * SOLVE_WG + t;
     constexpr size_t B3 = (size_t)3 * LB;
-    // slot 0: P, then A; slot 1: Q
-    auto get = [&](int slot, int k) {
-        return IN_LDS ? sh[(2 * k + slot) * SOLVE_WG + t] : v3_load((slot ? Q : A) + B3 * k, n);
-    };
-    auto put = [&](int slot, int k, V3 v) {
-        if (IN_LDS)
-            sh[(2 * k + slot) * SOLVE_WG + t] = v;
-        else
-            v3_store((slot ? Q : A) + B3 * k, n, v);
-    };
+    auto slot = [&](int i, int k) -> V3 & { return sh[(3 * k + i) * SOLVE_WG + t]; };
     if (IN_LDS) {
         constexpr int U = 8;
         for (int k0 = 0; k0 < nb; k0 += U) {
@@ -1077,196 +804,183 @@ k_pfb_join(const double *__restrict__ tab, int N, int nb, const double *__restri
 #pragma unroll
             for (int i = 0; i < U; ++i)
                 if (k0 + i < nb) {
-                    put(0, k0 + i, p[i]);
-                    put(1, k0 + i, q[i]);
+                    slot(0, k0 + i) = p[i];
+                    slot(1, k0 + i) = q[i];
                 }
         }
     }
-    const double be1 = tab[n], be2 = tab[LB + n], be3 = tab[2 * LB + n];
-    double cb[9], rb[9], rl[9], W[9], G[9];
+    const Beta be = beta_load(tab, n);
+    double cb[9], rb[9], gb[9], rl[9], G[9];
 #pragma unroll
     for (int i = 0; i < 9; ++i) {
         cb[i] = tab[(size_t)(TB_CB + i) * LB + n];
         rb[i] = tab[(size_t)(TB_RB + i) * LB + n];
+        gb[i] = tab[(size_t)(TB_GB + i) * LB + n];
+        rl[i] = rb[i];
     }
-    head_response(N & (SR - 1), be1, be2, be3, rl);
-#pragma unroll
-    for (int i = 0; i < 9; ++i) tc[(size_t)(TC_RS + i) * LB + n] = rl[i];
-    head_response((N - 1) % SBLK + 1, be1, be2, be3, rl);     // the last block's
-    corner(N, be1, be2, be3, W, G);
-    const V3 zero{0.0, 0.0, 0.0};
-    V3 a = zero;
-    for (int k = 0; k < nb; ++k) {
-        const V3 p = IN_LDS ? get(0, k) : v3_load(P + B3 * k, n), q = get(1, k);
-        put(0, k, a);
-        put(1, k, k == nb - 1 ? mv_add<1>(q, rl, a) : mv_add<1>(q, rb, a));
-        a = mv_add<1>(p, cb, a);
-    }
-    V3 z = zero;                                               // zeta at the head of block k
-    for (int k = nb - 1; k >= 0; --k) z = mv_add<1>(get(1, k), cb, z);
-    const double *h = tab + (size_t)TB_HB * LB + n;
-    const double h0 = h[0], h1 = h[LB], h2 = h[2 * LB], h3 = h[3 * LB], h4 = h[4 * LB];
-    // -dg on the first three rows: the states it leaves after the first block, and on
-    auto correct = [&](V3 dg) {
-        V3 d{-(dg.a * h4 + dg.b * h3 + dg.c * h2), -(dg.a * h3 + dg.b * h2 + dg.c * h1),
-             -(dg.a * h2 + dg.b * h1 + dg.c * h0)};
-        for (int k = 1; k < nb; ++k) {
-            const V3 p = get(0, k), q = get(1, k);
-            put(0, k, V3{p.a + d.a, p.b + d.b, p.c + d.c});
-            put(1, k, k == nb - 1 ? mv_add<1>(q, rl, d) : mv_add<1>(q, rb, d));
-            d = mv_add<1>(zero, cb, d);
-        }
-    };
-    V3 g = mv_add<1>(zero, W, z);
-    correct(g);
-    // One step of refinement: W comes from a Gram matrix, whose condition is that
-    // of the corner squared.  With the head zeta of the corrected solution, g must
-    // be H H^T zeta; the residual r is corrected by (I + H H^T G)^-1 r = r - W G r.
-    z = zero;
-    for (int k = nb - 1; k > 0; --k) z = mv_add<1>(get(1, k), cb, z);
     {
-        const double *gb = tab + (size_t)TB_GB * LB + n;
-        V3 q = get(1, 0);
-        q = V3{q.a - (gb[0] * g.a + gb[LB] * g.b + gb[2 * LB] * g.c),
-               q.b - (gb[3 * LB] * g.a + gb[4 * LB] * g.b + gb[5 * LB] * g.c),
-               q.c - (gb[6 * LB] * g.a + gb[7 * LB] * g.b + gb[8 * LB] * g.c)};
-        z = mv_add<1>(q, cb, z);
-        const double H[9] = {be1, be2, be3, be2, be3, 0.0, be3, 0.0, 0.0};          // symmetric
-        const V3 r = mv_add<1>(V3{-g.a, -g.b, -g.c}, H, mv_add<1>(zero, H, z));
-        const V3 wgr = mv_add<1>(zero, W, mv_add<1>(zero, G, r));
-        const V3 dg{r.a - wgr.a, r.b - wgr.b, r.c - wgr.c};
-        correct(dg);
-        g = V3{g.a + dg.a, g.b + dg.b, g.c + dg.c};
+        const int rows = (N - 1) % SBLK + 1;               // the last block's
+        double pw[9];
+        block_gram(rows == SBLK ? nb : nb - 1, cb, gb, pw, G);
+        if (rows != SBLK) {                                 // workgroup-uniform
+            double gl[9], s[9], u[9];
+            row_responses(rows, be, rl, gl);
+            mat_mul(s, pw, gl);
+            mat_mul_t(u, s, pw);
+#pragma unroll
+            for (int i = 0; i < 9; ++i) G[i] += u[i];
+        }
     }
-    v3_store(tc + (size_t)TC_G * LB, n, g);
-    if (IN_LDS)
-        for (int k = 0; k < nb; ++k) v3_store(A + B3 * k, n, get(0, k));
-    V3 b = zero;
-    for (int k = nb - 1; k >= 0; --k) {
-        v3_store(B + B3 * k, n, b);
-        b = mv_add<1>(get(1, k), cb, b);
+    const Corner cn = corner(be, G);
+    corner_store(tc, n, cn);
+    const double *hp = tab + (size_t)TB_HB * LB + n;
+    const double h0 = hp[0], h1 = hp[LB], h2 = hp[2 * LB], h3 = hp[3 * LB], h4 = hp[4 * LB];
+    const V3 zero{0.0, 0.0, 0.0};
+    V3 tt = zero;
+#pragma unroll 1
+    for (int it = 0; it <= CORNER_STEPS; ++it) {
+        const bool last = it == CORNER_STEPS;
+        const V3 g = hankel(be, tt);
+        V3 a = zero;
+        for (int k = 0; k < nb; ++k) {
+            V3 p = IN_LDS ? slot(0, k) : v3_load(P + B3 * k, n), q = IN_LDS ? slot(1, k) : v3_load(Q + B3 * k, n);
+            if (k == 0) {      // the block's response to -g on its first three rows
+                p = v3_sub(p, V3{fma(g.a, h4, fma(g.b, h3, g.c * h2)), fma(g.a, h3, fma(g.b, h2, g.c * h1)),
+                                 fma(g.a, h2, fma(g.b, h1, g.c * h0))});
+                q = mv_add<1>(q, gb, V3{-g.a, -g.b, -g.c});
+            }
+            q = mv_add<1>(q, k == nb - 1 ? rl : rb, a);
+            if (IN_LDS)
+                slot(2, k) = q;
+            else
+                v3_store(B + B3 * k, n, q);
+            if (last) v3_store(A + B3 * k, n, a);
+            a = mv_add<1>(p, cb, a);
+        }
+        V3 z = zero;                                        // zeta at the head of block k
+        for (int k = nb - 1; k >= 0; --k) {
+            const V3 q = IN_LDS ? slot(2, k) : v3_load(B + B3 * k, n);
+            if (last) v3_store(B + B3 * k, n, z);
+            z = mv_add<1>(q, cb, z);
+        }
+        if (!last) tt = v3_add(tt, corner_step(cn, be, z, tt));
     }
+    v3_store(tc + (size_t)TC_T * LB, n, tt);
 }
 
 // One block of 256 rows x 64 branches (a row of a wave: 256 contiguous bytes).
-// ONE: the block is the whole problem, and the corner is solved here; else its
-// incoming states and g come from k_pfb_join.  Rows past N read as zero and are
+// ONE: the block is the whole problem, and the corner is sought here; else its
+// incoming states and t come from k_pfb_join.  Rows past N read as zero and are
 // not written (range-checked buffers).
 template <bool ONE>
 __global__ void __launch_bounds__(64 * SWV, 4)
 k_pfb_solve(const float *__restrict__ yh, int N, const double *__restrict__ tab, const double *__restrict__ tc,
             const double *__restrict__ A, const double *__restrict__ B, float *__restrict__ x) {
-    // rows of the workgroup's table in LDS
-    constexpr int L_CS = 0, L_RS = 9, L_HS = 18, L_TC = 23, L_N = L_TC + TC_N;
-    static_assert(TB_HS == TB_RS + 9, "a span's responses are contiguous");
-    __shared__ double T[L_N * 64];
-    __shared__ V3 tot[SWV][64], sg[64], sd[64];
-    const int t = threadIdx.x, br = t & 63, wave = t >> 6, n0 = (int)blockIdx.x * 64, n = n0 + br;
-    const int blk = ONE ? 0 : (int)blockIdx.y, r0 = SBLK * blk + SR * wave;
+    __shared__ double cs[9 * 64];                // C^32
+    __shared__ V3 tot[SWV][64], sd[64];
+    // wave in a scalar register: v changes under branches on it, which must not be divergent
+    const int t = threadIdx.x, br = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
+    const int n0 = (int)blockIdx.x * 64, n = n0 + br, blk = ONE ? 0 : (int)blockIdx.y, r0 = SBLK * blk + SR * wave;
     const int nv = N - r0;                       // this span's rows: nv, at most 32 (none if <= 0)
     const __amdgpu_buffer_rsrc_t ry =
         __builtin_amdgcn_make_buffer_rsrc((void *)(yh + (size_t)SBLK * blk * LB), 0,
                                           min(N - SBLK * blk, SBLK) * LB * (int)sizeof(float), 0x00020000);
     double v[SR];
-    const double be1 = tab[n], be2 = tab[LB + n], be3 = tab[2 * LB + n];
-    V3 gin{0.0, 0.0, 0.0}, c0{0.0, 0.0, 0.0}, b0 = c0;
+    const Beta be = beta_load(tab, n);
+    const V3 zero{0.0, 0.0, 0.0};
+    V3 c0 = zero, tt = zero;
     if (!ONE) {
-        if (blk == 0 && wave == 0) gin = v3_load(tc + (size_t)TC_G * LB, n);
+        if (blk == 0 && wave == 0) tt = v3_load(tc + (size_t)TC_T * LB, n);
         c0 = v3_load(A + (size_t)3 * blk * LB, n);
-        b0 = v3_load(B + (size_t)3 * blk * LB, n);
     }
     {
         float y[SR];
         const int vo = 4 * (SR * wave * LB + n);
 #pragma unroll
         for (int k = 0; k < SR; ++k) y[k] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(ry, vo + 4 * LB * k, 0, 0));
-        for (int e = t; e < L_N * 64; e += 64 * SWV) {
-            const int r = e >> 6, c = n0 + (e & 63);
-            T[e] = r < L_RS   ? tab[(size_t)(TB_CS + r) * LB + c]
-                   : r < L_TC ? tab[(size_t)(TB_RS + r - L_RS) * LB + c]
-                              : tc[(size_t)(r - L_TC) * LB + c];
-        }
+        for (int e = t; e < 9 * 64; e += 64 * SWV) cs[e] = tab[(size_t)(TB_CS + (e >> 6)) * LB + n0 + (e & 63)];
 #pragma unroll
         for (int k = 0; k < SR; ++k) v[k] = (double)y[k];
     }
-    if (!ONE) {
-        v[0] -= gin.a;
-        v[1] -= gin.b;
-        v[2] -= gin.c;
+    if (!ONE) {                                  // tt is zero but in the block's first rows
+        const V3 g = hankel(be, tt);
+        v[0] -= g.a;
+        v[1] -= g.b;
+        v[2] -= g.c;
     }
-    const V3 zero{0.0, 0.0, 0.0};
-    const double *cs = T + L_CS * 64 + br;
-    // the span from zero states, both ways
-    V3 p = zero, q = zero;
-#pragma unroll
-    for (int k = 0; k < SR; ++k) {
-        v[k] = PFB_FILTER(v[k], p);
-        p = V3{v[k], p.a, p.b};
-    }
-    const bool part = nv < SR;                   // the span ends early
-    if (part) {
-#pragma unroll
-        for (int k = 0; k < SR; ++k)
-            if (k >= nv) v[k] = 0.0;
-    }
-#pragma unroll
-    for (int k = SR - 1; k >= 0; --k) q = V3{PFB_FILTER(v[k], q), q.a, q.b};
-    // incoming state: a_j = C^(32 j) c0 + sum_{i < j} C^(32 (j - 1 - i)) p_i
-    tot[wave][br] = p;
-    __syncthreads();
-    V3 a = c0;
-    for (int i = 0; i < wave; ++i) a = mv_add<64>(tot[i][br], cs, a);
-    __syncthreads();
-    // from below: C^(32 (7 - j)) b0 + sum_{i > j} C^(32 (i - 1 - j)) q_i
-    auto suffix = [&](V3 in) {
-        tot[wave][br] = in;
-        __syncthreads();
-        V3 c = b0;
-        for (int i = SWV - 1; i > wave; --i) c = mv_add<64>(tot[i][br], cs, c);
-        return c;
-    };
-    // head response of this span (the partial last one has its own; none past it)
-    const double *rm = T + (part ? L_TC + TC_RS : L_RS) * 64 + br;
-    if (nv > 0) q = mv_add<64>(q, rm, a);
-    V3 b = suffix(q);
-    if (ONE) {
-        if (wave == 0) {
-            const double *h = T + L_HS * 64 + br;
-            const V3 zh = mv_add<64>(q, cs, b);               // zeta[0..2] without the corner
-            const V3 g = mv_add<64>(zero, T + (L_TC + TC_W) * 64 + br, zh);
-            sg[br] = g;
-            // state after the first span from -g on its first three rows
-            sd[br] = V3{-(g.a * h[4 * 64] + g.b * h[3 * 64] + g.c * h[2 * 64]),
-                        -(g.a * h[3 * 64] + g.b * h[2 * 64] + g.c * h[64]),
-                        -(g.a * h[2 * 64] + g.b * h[64] + g.c * h[0])};
-        }
-        __syncthreads();
-        if (wave > 0) {        // C^(32 (j - 1)) of it
-            V3 d = sd[br];
-            for (int i = 1; i < wave; ++i) d = mv_add<64>(zero, cs, d);
-            a = V3{a.a + d.a, a.b + d.b, a.c + d.c};
-            if (nv > 0) q = mv_add<64>(q, rm, d);
-        } else {
-            gin = sg[br];
-        }
-        b = suffix(q);
-    }
-    if (nv <= 0) return;
-    // the rows from their true states
-    {
-        V3 d = a;
+    // x + C^32 y; the matrix is read where it is used (its 18 registers are v's)
+    auto carry = [&](V3 x, V3 y) { return mv_add<64>(x, cs + lds_opaque(br), y); };
+    // Spans past the last row stay out of the arithmetic and off the scans (their
+    // states are zero): a call of few rows is one wave per workgroup.
+    const bool mine = nv > 0;
+    const int spans = min((N - SBLK * blk + SR - 1) / SR, SWV);
+    V3 d = c0, b = zero;                         // b: the state from below
+    if (mine) {                                  // the span from a zero state
+        V3 p = zero;
 #pragma unroll
         for (int k = 0; k < SR; ++k) {
-            const double dk = PFB_FILTER(!ONE ? 0.0 : k == 0 ? -gin.a : k == 1 ? -gin.b : k == 2 ? -gin.c : 0.0, d);
-            v[k] += dk;
-            d = V3{dk, d.a, d.b};
+            v[k] = filter(be, v[k], p);
+            p = shift(v[k], p);
+        }
+        tot[wave][br] = p;
+    }
+    __syncthreads();
+    // incoming state: C^(32 j) c0 + sum_{i < j} C^(32 (j - 1 - i)) p_i
+    if (mine)
+        for (int i = 0; i < wave; ++i) d = carry(tot[i][br], d);
+    __syncthreads();
+    V3 g = zero;
+    const int steps = ONE ? 1 : blk == 0 ? CORNER_STEPS_BLOCK : 0;
+#pragma unroll 1
+    for (int it = 0;; ++it) {
+        int m = n;                               // each step's own: the addresses below are not kept through the loop
+        asm("" : "+v"(m) : "s"(it));
+        V3 q = zero;                             // the span's head zeta with nothing incoming from below
+        if (mine) {
+            // v changes by the filter's response to -g on the span's first three
+            // rows and to the incoming state d
+#pragma unroll
+            for (int k = 0; k < SR; ++k) {
+                const double dk = filter(be, k == 0 ? -g.a : k == 1 ? -g.b : k == 2 ? -g.c : 0.0, d);
+                v[k] += dk;
+                d = shift(dk, d);
+            }
+            if (nv < SR) {                       // the span ends early
+#pragma unroll
+                for (int k = 0; k < SR; ++k)
+                    if (k >= nv) v[k] = 0.0;
+            }
+#pragma unroll
+            for (int k = SR - 1; k >= 0; --k) q = shift(filter(be, v[k], q), q);
+            tot[wave][br] = q;
+        }
+        __syncthreads();
+        if (mine) {                              // C^(32 (7 - j)) times the block's + sum_{i > j} C^(32 (i - 1 - j)) q_i
+            b = ONE ? zero : v3_load(B + (size_t)3 * blk * LB, m);
+            for (int i = spans - 1; i > wave; --i) b = carry(tot[i][br], b);
+        }
+        if (it == steps) break;
+        d = zero;
+        if (wave == 0) {
+            const V3 dt = corner_step(corner_load(tc, m), be, carry(q, b), tt);
+            tt = v3_add(tt, dt);
+            g = hankel(be, dt);
+            if (spans > 1) {
+                V3 e = V3{-g.a, 0.0, 0.0};
+                e = shift(filter(be, -g.b, e), e);
+                e = shift(filter(be, -g.c, e), e);
+#pragma unroll 4
+                for (int k = 3; k < SR; ++k) e = shift(filter(be, 0.0, e), e);
+                sd[br] = e;
+            }
+        }
+        __syncthreads();
+        if (mine && wave > 0) {                  // C^(32 (j - 1)) of the first span's
+            d = sd[br];
+            for (int i = 1; i < wave; ++i) d = carry(zero, d);
         }
     }
-    if (part) {
-#pragma unroll
-        for (int k = 0; k < SR; ++k)
-            if (k >= nv) v[k] = 0.0;
-    }
+    if (!mine) return;
     const double w0 = tab[(size_t)TB_WZ * LB + n], w1 = tab[(size_t)(TB_WZ + 1) * LB + n],
                  w2 = tab[(size_t)(TB_WZ + 2) * LB + n], w3 = tab[(size_t)(TB_WZ + 3) * LB + n];
     // x[i + 3] = w0 z[i+3] + w1 z[i+2] + w2 z[i+1] + w3 z[i]; the first span also x[0..2].
@@ -1277,10 +991,10 @@ k_pfb_solve(const float *__restrict__ yh, int N, const double *__restrict__ tab,
     const int vs = lds_opaque(4 * (SR * wave * LB + n));   // not the loads' offsets kept live until here
 #pragma unroll
     for (int k = SR - 1; k >= 0; --k) {
-        const double z = PFB_FILTER(v[k], b);
+        const double z = filter(be, v[k], b);
         __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint((float)(w0 * b.c + w1 * b.b + w2 * b.a + w3 * z)), rx,
                                               vs + 4 * LB * k, 0, 0);
-        b = V3{z, b.a, b.b};
+        b = shift(z, b);
     }
     if (r0 == 0) {
         x[(size_t)2 * LB + n] = (float)(w0 * b.c + w1 * b.b + w2 * b.a);
@@ -1288,7 +1002,6 @@ k_pfb_solve(const float *__restrict__ yh, int N, const double *__restrict__ tab,
         x[n] = (float)(w0 * b.a);
     }
 }
-#undef PFB_FILTER
 
 }  // namespace
 
@@ -1312,7 +1025,7 @@ struct sdbe_pfb {
     double *bst = nullptr;        // [4][nb][3][32768] ... its blocks' states, out and in, both ways
     int nb = 0;                   // blocks of max_spec rows
     int n_cu = 256;               // compute units of the device
-    int constant = 0;             // no branch has zeros together on the unit circle
+    int constant = 0;             // every branch is admitted to the constant-coefficient solve
 };
 
 namespace {
@@ -1363,7 +1076,8 @@ int sdbe_pfb_create(int device, int32_t n_taps, const float *h_window, int32_t m
     if (!p) return SDBE_ERR_NOMEM;
     p->device = device;
     p->max_spec = max_spectra;
-    int rc = SDBE_OK, clustered = 0, *d_clustered = nullptr, ncu = 0;
+    int rc = SDBE_OK, refused = 0, *d_refused = nullptr, ncu = 0;
+    const int nb = (max_spectra + SBLK - 1) / SBLK;
     if (hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, device) == hipSuccess && ncu > 0) p->n_cu = ncu;
     std::vector<float2> img(FFT_TW_N);
     std::vector<double2> tw(1024);
@@ -1386,23 +1100,24 @@ int sdbe_pfb_create(int device, int32_t n_taps, const float *h_window, int32_t m
     PALLOC(p->yh, (size_t)max_spectra * LB * sizeof(float));
     PALLOC(p->tab, (size_t)TB_N * LB * sizeof(double));
     PALLOC(p->tc, (size_t)TC_N * LB * sizeof(double));
-    d_clustered = reinterpret_cast<int *>(p->tc);    // until the first call writes its tables
+    d_refused = reinterpret_cast<int *>(p->tc);    // until the first call writes its tables
     if (hipMemcpy(p->fft_img, img.data(), FFT_TW_N * sizeof(float2), hipMemcpyHostToDevice) != hipSuccess ||
         hipMemcpy(p->tw1k, tw.data(), 1024 * sizeof(double2), hipMemcpyHostToDevice) != hipSuccess ||
         hipMemcpy(p->win, h_window, (size_t)NT * LB * sizeof(float), hipMemcpyHostToDevice) != hipSuccess ||
-        hipMemcpy(d_clustered, &clustered, sizeof(int), hipMemcpyHostToDevice) != hipSuccess) {
+        hipMemcpy(d_refused, &refused, sizeof(int), hipMemcpyHostToDevice) != hipSuccess) {
         rc = SDBE_ERR_HIP;
         goto fail;
     }
-    hipLaunchKernelGGL(k_pfb_spectral, dim3(LB / SOLVE_WG), dim3(SOLVE_WG), 0, 0, (const float *)p->win, p->tab,
-                       d_clustered);
-    if (hipMemcpy(&clustered, d_clustered, sizeof(int), hipMemcpyDeviceToHost) != hipSuccess) {
+    hipLaunchKernelGGL(k_pfb_spectral, dim3(LB / SOLVE_WG), dim3(SOLVE_WG), 0, 0, (const float *)p->win, nb, p->tab,
+                       d_refused);
+    if (hipGetLastError() != hipSuccess ||
+        hipMemcpy(&refused, d_refused, sizeof(int), hipMemcpyDeviceToHost) != hipSuccess) {
         rc = SDBE_ERR_HIP;
         goto fail;
     }
-    p->constant = clustered == 0;
+    p->constant = refused == 0;
     if (p->constant) {
-        p->nb = (max_spectra + SBLK - 1) / SBLK;
+        p->nb = nb;
         PALLOC(p->bst, (size_t)4 * 3 * p->nb * LB * sizeof(double));
     } else {                                         // the factor-row kernels
         // one transfer per span; checkpoints up to the chunk after the last full span
@@ -1488,9 +1203,9 @@ int sdbe_pfb_inverse(sdbe_pfb_t *p, const void *d_spec, int32_t n_spectra, float
                    *B = A + (size_t)3 * p->nb * LB;
             hipLaunchKernelGGL(k_pfb_span, dim3(LB / SOLVE_WG, nb), wg, 0, s, yh, N, tab, P, Q);
             if (nb <= JOIN_LDS)
-                hipLaunchKernelGGL(k_pfb_join<true>, br, wg, 0, s, tab, N, nb, (const double *)P, Q, A, B, p->tc);
+                hipLaunchKernelGGL(k_pfb_join<true>, br, wg, 0, s, tab, N, nb, (const double *)P, (const double *)Q, A, B, p->tc);
             else
-                hipLaunchKernelGGL(k_pfb_join<false>, br, wg, 0, s, tab, N, nb, (const double *)P, Q, A, B, p->tc);
+                hipLaunchKernelGGL(k_pfb_join<false>, br, wg, 0, s, tab, N, nb, (const double *)P, (const double *)Q, A, B, p->tc);
             hipLaunchKernelGGL(k_pfb_solve<false>, dim3(LB / 64, nb), dim3(64 * SWV), 0, s, yh, N, tab,
                                (const double *)p->tc, (const double *)A, (const double *)B, d_x);
         }
