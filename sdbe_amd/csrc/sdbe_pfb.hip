@@ -930,7 +930,7 @@ k_pfb_solve(const float *__restrict__ yh, int N, const double *__restrict__ tab,
         for (int i = 0; i < wave; ++i) d = carry(tot[i][br], d);
     __syncthreads();
     V3 g = zero;
-    const int steps = ONE ? 1 : blk == 0 ? CORNER_STEPS_BLOCK : 0;
+    const int steps = ONE ? CORNER_STEPS : blk == 0 ? CORNER_STEPS_BLOCK : 0;
 #pragma unroll 1
     for (int it = 0;; ++it) {
         int m = n;                               // each step's own: the addresses below are not kept through the loop

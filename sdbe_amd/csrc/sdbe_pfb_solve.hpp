@@ -361,9 +361,9 @@ __host__ __device__ __forceinline__ V3 corner_step(const Corner &c, const Beta &
     const double z2 = y2 * c.i2, z1 = (y1 - c.l21 * z2) * c.i1;
     return V3{(y0 - c.l10 * z1 - c.l20 * z2) * c.i0, z1, z2};
 }
-// Steps of t in the join: from nothing and one of refinement; the block that holds
-// the corner takes one more from its own rows, since t rounded as it comes from
-// the join is (B B^T)^-1's first columns off.
+// Steps of t: from nothing and one of refinement wherever it is sought; the
+// block that holds the corner takes one more from its own rows, since t rounded
+// as it comes from the join is (B B^T)^-1's first columns off.
 constexpr int CORNER_STEPS = 2, CORNER_STEPS_BLOCK = 1;
 
 }  // namespace pfb

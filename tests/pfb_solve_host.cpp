@@ -101,7 +101,7 @@ void block(const Branch &br, const std::vector<float> &y, int blk, bool one, con
         for (int i = 0; i < w; ++i) a = mv_add<1>(tot[i], cs, a);
         change(w, ZERO, a);
     }
-    const int steps = one ? 1 : blk == 0 ? CORNER_STEPS_BLOCK : 0;
+    const int steps = one ? CORNER_STEPS : blk == 0 ? CORNER_STEPS_BLOCK : 0;
     for (int it = 0;; ++it) {
         for (int w = 0; w < SWV; ++w) {
             q[w] = ZERO;

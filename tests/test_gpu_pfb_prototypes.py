@@ -82,7 +82,7 @@ def _condition(taps, n):
 
 @pytest.mark.parametrize("kind,exact,rows", [
     ("hann_sinc", True, (1, 2, 3, 33, 255, 256, 257, 511, 4097)),
-    ("hamming", True, (257, 289, 511, 512, 1000, 4096, 4097)),
+    ("hamming", True, (1, 2, 3, 20, 31, 32, 33, 64, 128, 225, 255, 256, 257, 289, 511, 512, 1000, 4096, 4097)),
     ("kaiser 5", True, (128, 300)),
     ("gauss 0.954", False, (64, 128, 300, 512)),
     ("gauss 0.955", False, (64, 256, 512)),
