@@ -618,7 +618,7 @@ k_group_bitmap(const int *__restrict__ map, uint8_t *__restrict__ bitmap, int *_
 // go forward over a contiguous range of block-pols per XCD (xcd_contig), stages B
 // and C2 backward over the same ranges (xcd_map: nb and the grid are multiples of 8;
 // workgroups are dealt round-robin over the 8 XCDs).  All in one order: 33
-// block-pols 524 us (now 509), 64: 718 (708), 256: 2551 (2541).
+// block-pols as floats 507 us (now 500); at 256 no more than the runs differ.
 __device__ __forceinline__ int back_bp(int lin, int per, int nb, int xcd_map, int &item) {
     lin = __builtin_amdgcn_readfirstlane(lin);
     const int slot = xcd_map ? lin >> 3 : lin, n = xcd_map ? nb >> 3 : nb, b = slot / per;
@@ -1039,7 +1039,7 @@ k_stats(const double *__restrict__ part, int bp0, double2 *__restrict__ ms, doub
 // of the last polarisation-0 block-pol up to it (sigma 0), or the slot's own if
 // there is none.  f and the slot's last polarisation-0 block-pol are minima and
 // maxima over the chunk, so no thread walks it (one thread's walk over LDS took
-// 28 us for 256 block-pols, this THRTIME); the search back before f runs only
+// 28 us for 256 block-pols, this 4.6); the search back before f runs only
 // for empty leading blocks.
 constexpr int THRESH_MAX_CHUNK = SDBE_MAX_CHUNK;
 template <int MAXB>

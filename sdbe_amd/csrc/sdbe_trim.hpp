@@ -650,8 +650,8 @@ k_trim_seg(const float *__restrict__ T, const BpDesc *__restrict__ bpd, float *_
     const int bpl = (int)gridDim.x / trim::NSEG - 1 - bw;
     // With a known threshold the samples leave as codes and not as floats: 1/16 of
     // the stores, and k_trim_pack has nothing to do for the block.  256 block-pols
-    // at 6/11, segments and packing: 806 + 5 us, as floats 800 + 217; at 11/11 3895 +
-    // 10 and 3965 + 833.  (Decided here, ahead of the transforms: a branch between
+    // at 6/11, segments and packing: 819 + 20 us, with PER_BLOCK thresholds, as floats,
+    // 769 + 210; at 11/11 3963 + 65 and 3952 + 772.  (Decided here, ahead of the transforms: a branch between
     // them splits the schedule and takes 130 registers more.)  Without CODES, for calls
     // whose blocks all have the PER_BLOCK policy, the branch is not there: a group at 10/11
     // 3111 -> 2962 us, at 6/11 1526 -> 1504 (on two boxes; before there was a code path
@@ -828,7 +828,7 @@ k_trim_stats(const double *__restrict__ part, int P, int bp0, double2 *__restric
 // TB/s): a wave reads 4 KB in four coalesced loads of 16 bytes a lane, each lane's
 // four codes are a byte of a word of its four lanes, and of four lanes lane i
 // stores the word of load i.  One such piece a wave; with 2 to 8 a launch that finds
-// the codes stored is shorter (256 block-pols at 11/11: 45 and 10 us), but one that
+// the codes stored is shorter (256 block-pols at 11/11: 45 and 10 us, with one 65), but one that
 // does not takes 15 to 50 us more.
 __global__ void __launch_bounds__(256)
 k_trim_pack(const float *__restrict__ stage, const float2 *__restrict__ thr, const BpDesc *__restrict__ bpd, int P,
